@@ -11,6 +11,7 @@
 #include <string>
 #include <vector>
 
+#include "moe_decode.h"
 #include "moe_internal.h"
 
 using namespace moe;
@@ -1624,6 +1625,31 @@ static int decode_check(moe_handle *h, int n) {
     return MOE_OK;
 }
 
+// The router's part of a decode call by 16 waves per token instead of 4: with
+// 4 a lane walks 16 or more router rows in series from D * Er_pad = 64 K on
+// (2048 x 64: the call of one token 100 us, 49 us with 16 waves and a launch
+// of its own instead of once per block).  A rule on the layer alone, so that
+// a token's logits do not depend on the batch.
+static int decode_wide_route(const moe_handle *h) { return (long long)h->D * h->Er_pad > 64 * 1024; }
+
+// Whether a decode call of n tokens runs grouped by expert (four launches)
+// instead of token by token (two launches, the routing repeated by every
+// block).  Measured by the multiply-adds of the call's expert products, n kt
+// 3 D H, both ways in us: fp32 / bf16, one token: 13 M 15 / 17, 25 M 23 / 23
+// and 16 / 19, 50 M 52 / 41 and 36 / 28; several: 17 M 14 / 16 and 11 / 16,
+// 25 M 27 / 18 and 25 / 18, 34 M 22 / 17 and 16 / 16; fp8: 8 M 13 / 16, 13 M
+// 19 / 16, 17 M 20 / 16.
+static bool decode_batched(const moe_handle *h, int n) {
+    const int c = std::min(n, kDecodeChunk);
+    // workspace: y of every entry; bf16 / fp8: x in the split workspace and h
+    // in hbuf, 6 bytes per element
+    if ((long long)c * h->kt * h->Dout > (long long)h->rows_max * h->ld_y) return false;
+    if (h->wt != WT_F32 && (6LL * c * h->D_pad > 4 * h->split_cap || 3LL * c * h->kt > h->act_rows)) return false;
+    if (decode_wide_route(h)) return true;
+    const long long mac = (long long)n * h->kt * 3 * h->D * h->H;
+    return mac >= (h->wt == WT_FP8 ? 12000000LL : (n == 1 ? 40000000LL : 24000000LL));
+}
+
 static int decode_locked(moe_handle *h, const float *x_dev, int n, float *out_dev, hipStream_t s,
                          hipEvent_t done = nullptr) {
     DecodeArgs a{};
@@ -1635,6 +1661,23 @@ static int decode_locked(moe_handle *h, const float *x_dev, int n, float *out_de
     a.Dpad = h->D_pad; a.H = h->H; a.Hpad = h->H_pad; a.Dout = h->Dout;
     a.s1 = h->s1; a.s3 = h->s3; a.s2 = h->s2; a.Dout_npad = h->Dout_npad;
     a.h = (float *)h->hbuf; a.out = out_dev;
+    if (decode_batched(h, n)) {
+        for (int t0 = 0; t0 < n; t0 += kDecodeChunk) {
+            DecodeArgs c = a;
+            c.n = std::min(kDecodeChunk, n - t0);
+            c.x = a.x + (long long)t0 * a.D; c.out = a.out + (long long)t0 * a.Dout;
+            c.logits = a.logits + (long long)t0 * a.E; c.probs = a.probs + (long long)t0 * a.E;
+            c.idx = a.idx + (long long)t0 * a.kt; c.gates = a.gates + (long long)t0 * a.kt;
+            DecodeBatch b{};
+            b.w1t = h->w1t; b.w3t = h->w3t; b.w2t = h->w2t;
+            if (h->wt != WT_F32) { b.xs = (uint16_t *)h->split_ws; b.hs = (uint16_t *)h->hbuf; }
+            b.y = h->y;
+            HIP_TRY(h, launch_decode_route(c, decode_wide_route(h), b.xs, s));
+            HIP_TRY(h, launch_decode_batch(c, b, s, t0 + c.n == n ? done : nullptr));
+        }
+        h->last_T = -1;
+        return MOE_OK;
+    }
     HIP_TRY(h, launch_decode_ffn(a, h->ncu, s, done));
     h->last_T = -1;  // the routing buffers no longer describe a layer forward
     return MOE_OK;

@@ -3,7 +3,8 @@
 // tokens), its k selected gated experts as matrix-vector products, combined
 // in slot order, and the layer's shared experts (process_shared_experts!,
 // :184-216) averaged and blended 0.5 / 0.5 with them.  Weight-bandwidth bound: every selected expert's three
-// matrices are read once per token; two kernels per call.
+// matrices are read once per token; two kernels per call.  Batches and large
+// layers run grouped by expert (moe_decode_batch.h).
 //
 //   decode_up_kernel   : the token's routing (logits = W' xb + b, softmax,
 //                        top-k, gates; inference.jl:62-66), recomputed by every
@@ -22,6 +23,8 @@
 // (clamped addresses, out-of-row chunks selected to zero).
 #include <hip/hip_ext.h>
 
+#include "moe_decode.h"
+#include "moe_decode_batch.h"
 #include "moe_internal.h"
 
 namespace moe {
@@ -42,50 +45,17 @@ __device__ __forceinline__ float4 load_w4(const void *w, long long o) {
     }
 }
 
-__device__ __forceinline__ float readlane_f(float v, int i) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
-}
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-
-// Sum over each 16-lane row in a fixed order, every lane of the row ending
-// with the same bits: pairs (quad_perm 1,0,3,2), quads (quad_perm 2,3,0,1),
-// 8-lane halves (row_half_mirror), rows (row_mirror); additions commute
-// exactly, so partner lanes hold identical values after every step.
-__device__ __forceinline__ float row16_sum(float v) {
-    v = v + dpp_f<0xb1>(v);
-    v = v + dpp_f<0x4e>(v);
-    v = v + dpp_f<0x141>(v);
-    v = v + dpp_f<0x140>(v);
-    return v;
-}
-
-// Wave sum (all 64 lanes active), uniform result: row sums, then the four rows
-// in row order.
-__device__ __forceinline__ float wave_sum(float v) {
-    v = row16_sum(v);
-    return ((readlane_f(v, 0) + readlane_f(v, 16)) + readlane_f(v, 32)) + readlane_f(v, 48);
-}
-
-__device__ __forceinline__ float4 zero_unless(bool v, float4 a) {
-    return v ? a : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-}
-
-__device__ __forceinline__ float dot4_acc(float acc, float4 a, float4 b) {
-#pragma clang fp contract(off)
-    acc = acc + a.x * b.x;
-    acc = acc + a.y * b.y;
-    acc = acc + a.z * b.z;
-    acc = acc + a.w * b.w;
-    return acc;
-}
-
-// ---- routing of one token by a 256-thread block --------------------------------
+// ---- routing of one token by a block of NW waves --------------------------------
+template <int NW>
 struct DecodeRouteLds {
-    __attribute__((aligned(16))) float part[4][MOE_MAX_EXPERTS];  // per-wave logit partials
+    __attribute__((aligned(16))) float part[NW][MOE_MAX_EXPERTS];  // per-wave logit partials
+    __device__ __forceinline__ float logit(int e) const {          // their sum in wave order
+#pragma clang fp contract(off)
+        float v = part[0][e];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v = v + part[w][e];
+        return v;
+    }
 };
 
 // The routed slots' experts of one token (0-based), 16 bits each: slot j in
@@ -111,9 +81,9 @@ struct DecodeSel {
 // lanes, i.e. the experts in ascending order; every register array is read
 // with compile-time indices only (a part picked at run time would be a
 // private-memory array).
-template <int NH>
+template <int NH, int NW>
 __device__ __forceinline__ DecodeSel decode_gates(const DecodeArgs &a, int t, bool write,
-                                                           const DecodeRouteLds &L, float &gate) {
+                                                           const DecodeRouteLds<NW> &L, float &gate) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63, E = a.E;
     float lg[NH], ev[NH], pv[NH];
@@ -122,7 +92,7 @@ __device__ __forceinline__ DecodeSel decode_gates(const DecodeArgs &a, int t, bo
     for (int h = 0; h < NH; ++h) {
         const int e = lane + 64 * h;
         const int ec = min(e, a.Er_pad - 1);
-        float v = ((L.part[0][ec] + L.part[1][ec]) + L.part[2][ec]) + L.part[3][ec];
+        float v = L.logit(ec);
         if (a.br) v = v + a.br[min(e, E - 1)];
         lg[h] = v;
     }
@@ -261,13 +231,14 @@ __device__ __forceinline__ float wave_fmax(float v, bool rows4) {  // v never Na
 // adding exact zeros; the k slots are k rounds of "largest isless key, lowest
 // expert among equal keys", the partialsortperm order that decode_gates
 // derives from ranks.
+template <int NW>
 __device__ __forceinline__ DecodeSel decode_gates64(const DecodeArgs &a, int t, bool write,
-                                                             const DecodeRouteLds &L, float &gate) {
+                                                             const DecodeRouteLds<NW> &L, float &gate) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63, E = a.E;
     const bool valid = lane < E, rows4 = E > 16;
     const int ec = min(lane, a.Er_pad - 1);
-    float lg = ((L.part[0][ec] + L.part[1][ec]) + L.part[2][ec]) + L.part[3][ec];
+    float lg = L.logit(ec);
     if (a.br) lg = lg + a.br[min(lane, E - 1)];
     const float m = wave_fmax(valid && !__builtin_isnan(lg) ? lg : -INFINITY, rows4);
     float ev = (m == INFINITY) ? ((lg == INFINITY) ? 1.0f : 0.0f) : (float)exp((double)(lg - m));
@@ -316,9 +287,9 @@ __device__ __forceinline__ DecodeSel decode_gates64(const DecodeArgs &a, int t, 
 }
 
 // Logits: lane (q, c) = q C + c of wave w sums x[d] W[d][4q..4q+3] over the
-// chunk g = w C + c of D in d order (one float4 per router row, 4 rows in
+// chunk g = w C + c of D in d order (one float4 per router row, RF rows in
 // flight); the C chunks of a wave are added by a fixed tree (DPP steps within
-// 16-lane rows, then lane xor 16 and 32), the 4 wave sums in wave order, then
+// 16-lane rows, then lane xor 16 and 32), the NW wave sums in wave order, then
 // the bias.  Every wave then evaluates compute_gates on its own copy (identical
 // results, no second barrier) with the recipe of the layer's routing kernel:
 // m = max (NaN ignored), e_i = (float)exp((double)(l_i - m)) (a +Inf maximum
@@ -327,10 +298,12 @@ __device__ __forceinline__ DecodeSel decode_gates64(const DecodeArgs &a, int t, 
 // keys (partialsortperm(p, 1:k, rev=true)): the rank of expert i is the number
 // of experts before it in that order; the gates are p of the slots over their
 // sum in slot order.  Lane l holds experts l, l + 64, l + 128, ... < E.
+// WRITE_ONLY: the waves that do not write stop after the logits.
 // Returns the 0-based experts of the routed slots (uniform), and in `gate`
 // of lane j < k that slot's gate; `write` (wave 0 of
 // one block per token) stores logits, probs, indices, gates.
-__device__ __forceinline__ DecodeSel decode_route_block(const DecodeArgs &a, int t, bool write, DecodeRouteLds &L,
+template <int NW, bool WRITE_ONLY = false>
+__device__ __forceinline__ DecodeSel decode_route_block(const DecodeArgs &a, int t, bool write, DecodeRouteLds<NW> &L,
                                                  float &gate) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -339,7 +312,7 @@ __device__ __forceinline__ DecodeSel decode_route_block(const DecodeArgs &a, int
     while (QP < Q) QP <<= 1;                            // Q <= MOE_MAX_EXPERTS / 4
     const int C = QP >= 64 ? 1 : 64 / QP;               // chunks per wave
     const int NQ = QP > 64 ? QP / 64 : 1;               // float4 columns per lane (lane, lane + 64, ...)
-    const int CH = (a.D + 4 * C - 1) / (4 * C);
+    const int CH = (a.D + NW * C - 1) / (NW * C);
     const float *x = a.x + (long long)t * a.D;
     const float4 *wr4 = (const float4 *)a.wr;
     for (int qi = 0; qi < NQ; ++qi) {
@@ -348,17 +321,18 @@ __device__ __forceinline__ DecodeSel decode_route_block(const DecodeArgs &a, int
         {
             const int d0 = (w * C + c) * CH, d1 = min(a.D, d0 + CH);
             const int qq = min(q, Q - 1);
-            for (int d = d0; d < d1; d += 4) {
-                float xv[4];
-                float4 wv[4];
+            constexpr int RF = NW == 4 ? 4 : 8;  // router rows in flight
+            for (int d = d0; d < d1; d += RF) {
+                float xv[RF];
+                float4 wv[RF];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
+                for (int u = 0; u < RF; ++u) {
                     const int dd = min(d + u, d1 - 1);
                     xv[u] = x[dd];
                     wv[u] = wr4[(long long)dd * Q + qq];
                 }
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
+                for (int u = 0; u < RF; ++u)
                     if (d + u < d1) {
                         acc.x = acc.x + xv[u] * wv[u].x;
                         acc.y = acc.y + xv[u] * wv[u].y;
@@ -391,6 +365,7 @@ __device__ __forceinline__ DecodeSel decode_route_block(const DecodeArgs &a, int
         if (c == 0 && q < Q) *(float4 *)&L.part[w][4 * q] = acc;
     }
     __syncthreads();
+    if (WRITE_ONLY && !write) return DecodeSel{};
 
     if (E > 256) return decode_gates<8>(a, t, write, L, gate);
     if (E > 128) return decode_gates<4>(a, t, write, L, gate);
@@ -465,11 +440,37 @@ __device__ __forceinline__ void decode_up_units(const DecodeArgs &a, int t, int 
 // block (token t, y) routes t, then runs its waves' units
 template <int WT>
 __global__ __launch_bounds__(256) void decode_up_kernel(DecodeArgs a) {
-    __shared__ DecodeRouteLds L;
+    __shared__ DecodeRouteLds<4> L;
     const int w = threadIdx.x >> 6;
     float gate;
     const DecodeSel sel = decode_route_block(a, blockIdx.x, blockIdx.y == 0 && w == 0, L, gate);
     decode_up_units<WT>(a, blockIdx.x, blockIdx.y * 4 + w, gridDim.y * 4, sel);
+}
+
+// ---- batches (moe_decode_batch.h): block t routes token t; with xs, its x as
+// three bf16 parts (pad columns 0)
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void decode_route_kernel(DecodeArgs a, uint16_t *xs) {
+    __shared__ DecodeRouteLds<NW> L;
+    const int t = blockIdx.x;
+    float gate;
+    if (xs) {
+        const float *x = a.x + (long long)t * a.D;
+        uint16_t *dst = xs + (long long)t * 3 * a.Dpad;
+        for (int d = threadIdx.x; d < a.Dpad; d += 64 * NW) {
+            uint16_t p[3];
+            split_bf16x3(d < a.D ? x[d] : 0.0f, p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) dst[(long long)q * a.Dpad + d] = p[q];
+        }
+    }
+    decode_route_block<NW, true>(a, t, threadIdx.x < 64, L, gate);
+}
+
+hipError_t launch_decode_route(const DecodeArgs &a, int wide, uint16_t *xs, hipStream_t s) {
+    if (wide) hipLaunchKernelGGL(decode_route_kernel<16>, dim3(a.n), dim3(1024), 0, s, a, xs);
+    else hipLaunchKernelGGL(decode_route_kernel<4>, dim3(a.n), dim3(256), 0, s, a, xs);
+    return hipGetLastError();
 }
 
 // ---- down: one wave per output row i of token t; slots two at a time, U

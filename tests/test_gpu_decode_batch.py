@@ -1,0 +1,75 @@
+"""GPU parity of decode calls that run grouped by expert (several tokens, or a
+layer whose router is large): against the oracle on the GPU's own logits,
+routing and gates bit-exact, and against single calls.
+
+The output tolerance is 1e-5 for every weight type: the oracle sees the
+dequantised weights, activations stay fp32 (bf16 and fp8 weights meet them as
+three exact bf16 parts), and fp32 sums of K <= 2048 products are within about
+sqrt(K) 2^-24 = 3e-6 of each other."""
+import numpy as np
+import pytest
+
+from test_gpu_layer import Case, rel_err
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+@pytest.mark.parametrize("wdtype", ["f32", "bf16", "fp8"])
+@pytest.mark.parametrize("D,H,Dout,E,k,lsh,n", [
+    (512, 1376, 512, 8, 2, 0, 16),   # groups of at most 16
+    (260, 300, 90, 2, 1, 0, 130),    # about 32 per group and chunk; sizes off every tile; three chunks, the last of 2
+    (1000, 700, 40, 5, 2, 1, 65),    # a shared expert that takes whole chunks of 64, then one token
+    (200, 330, 200, 3, 3, 0, 41),    # every expert takes all 41 tokens (three column tiles)
+    (128, 96, 160, 40, 12, 3, 64),   # 15 slots per token: the index list at its largest but one
+    (2048, 64, 64, 40, 2, 0, 1),     # the 16-wave router, one token
+    (2048, 128, 72, 300, 8, 0, 5),   # ... with eight experts per lane, most experts idle
+])
+def test_decode_grouped(moe, oracle, wdtype, D, H, Dout, E, k, lsh, n):
+    c = Case(moe, oracle, T=n, D=D, H=H, Dout=Dout, E=E + lsh, k=k, wdtype=wdtype, seed=300 + n + E, lsh=lsh,
+             max_tokens=2 * n + 2)
+    try:
+        x = np.ascontiguousarray(c.x)
+        out, logits, idx, gates = c.dev.decode(x)
+        again = c.dev.decode(x)[0]
+        assert np.array_equal(out.view(np.uint32), again.view(np.uint32))
+        ref_logits = x.astype(np.float64) @ c.wr.T.astype(np.float64)
+        assert np.max(np.abs(logits - ref_logits)) <= 1e-5 * max(1.0, float(np.max(np.abs(ref_logits))))
+        ref, ridx, rgates, _ = oracle.decode_ffn(x, c.wr, c.ex, k=k, logits=logits, num_shared=lsh)
+        assert np.array_equal(idx[:, lsh:] - lsh, ridx)
+        assert np.array_equal(gates[:, lsh:].view(np.uint32), rgates.view(np.uint32))
+        assert rel_err(out, ref) <= TOL, rel_err(out, ref)
+        # the layer's forward still finds its workspace as it expects it
+        if Dout == D:
+            f1 = c.run(training=False)[0]
+            c.dev.decode(x)
+            f2 = c.run(training=False)[0]
+            assert np.array_equal(f1.view(np.uint32), f2.view(np.uint32))
+    finally:
+        c.dev.close()
+
+
+@pytest.mark.parametrize("wdtype,n", [("f32", 40), ("bf16", 70), ("fp8", 70)])
+def test_decode_grouped_independent_of_the_batch(moe, oracle, wdtype, n):
+    # a token's result is the same bits in any batch that runs grouped, and
+    # in fp32 in a single call too; a token with an infinity or a NaN in x
+    # leaves the others' bits alone
+    c = Case(moe, oracle, T=n, D=512, H=700, E=6, k=2, wdtype=wdtype, seed=77, max_tokens=2 * n)
+    try:
+        print(f"grouped decode of {n}, w={wdtype}", flush=True)
+        x = np.ascontiguousarray(c.x)
+        out = c.dev.decode(x)[0]
+        lo = 1 if wdtype == "f32" else 24
+        for t, m in ((0, lo), (n - lo, lo), (3, 33)):
+            o = c.dev.decode(np.ascontiguousarray(x[t:t + m]))[0]
+            assert np.array_equal(o.view(np.uint32), out[t:t + m].view(np.uint32)), (t, m)
+        bad = x.copy()
+        bad[2, 5], bad[7, 0], bad[9, 1] = np.inf, np.nan, 3.4e38
+        o = c.dev.decode(bad)[0]
+        keep = np.ones(n, bool)
+        keep[[2, 7, 9]] = False
+        assert np.array_equal(o[keep].view(np.uint32), out[keep].view(np.uint32))
+        assert np.isnan(o[7]).all()
+    finally:
+        c.dev.close()
