@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "moe_decode.h"
+#include "moe_gemm.h"
 #include "moe_internal.h"
 
 using namespace moe;
@@ -1013,9 +1014,11 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
     h->ld_y = h->bf16_gemm ? (int)round_up(h->Dout, 64) + 64 : h->Dout;
     A((void **)&h->y, sizeof(float) * (size_t)h->rows_max * h->ld_y);
     // tail split: at most gemm_slots partial blocks of BM x 256 floats
-    // (rem * S <= slots) for either GEMM; the fp32 kernel's K split of small
-    // tile grids: about two workgroups per CU of NB x 128 x 128 floats
-    h->split_cap = h->bf16_gemm ? (long long)gemm_slots(h) * h->bm * 256 : 2LL * h->ncu * kGemmBM * kGemmBN;
+    // (rem * S <= slots) for either GEMM; the fp32 kernels' K ranges: about two
+    // workgroups per CU of 128 x 128 floats, of 128 x 256 where the handle's
+    // batches reach the f32x3 kernel
+    h->split_cap = h->bf16_gemm ? (long long)gemm_slots(h) * h->bm * 256
+                                : 2LL * h->ncu * kGemmBM * kGemmBN * (f32x3_rows(h->max_tiles - 1, h->E) ? 2 : 1);
     A((void **)&h->split_ws, sizeof(float) * (size_t)h->split_cap);
     if (r != MOE_OK) return cleanup(r);
     // Pads of the packed weights and of the activation rows must read as 0.

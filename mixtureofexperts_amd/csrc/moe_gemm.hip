@@ -1,6 +1,7 @@
-// moe_gemm.hip -- the fp32 (reference-precision) grouped GEMM over
+// moe_gemm.hip -- the fp32 (reference-precision) grouped GEMMs over
 // variable-size expert segments on CDNA4 MFMA, with the expert FFN's
-// elementwise work fused into the epilogues.  Handles with bf16 or fp8
+// elementwise work fused into the epilogues: grouped_gemm_kernel (fp32 MFMA,
+// short segments) and the one of moe_gemm_f32x3.h (longer ones).  Handles with bf16 or fp8
 // weights run the LDS-DMA kernel of moe_gemm_bf16.hip instead.
 //
 //   MODE_GATED_UP : h = act(A W1^T) .* (A W3^T)      GatedExpert
@@ -27,7 +28,9 @@
 // split_ws block (tile, ks) = NB x BM x BN floats, [b][row][col];
 // fold_f32_kernel sums the S ranges in order and runs the epilogue.
 #include <algorithm>
+#include <type_traits>
 
+#include "moe_gemm.h"
 #include "moe_internal.h"
 
 namespace moe {
@@ -40,10 +43,13 @@ __device__ inline float act_apply(int act, float x) {
     switch (act) {
     case MOE_ACT_SILU:  // x * sigmoid(x)
         return x / (1.0f + expf(-x));
-    case MOE_ACT_GELU: {  // NNlib gelu, tanh form
-        const float c = 0.7978845608028654f;  // sqrt(2/pi)
-        const float u = c * (x + 0.044715f * x * x * x);
-        return 0.5f * x * (1.0f + tanhf(u));
+    case MOE_ACT_GELU: {
+        // NNlib gelu, tanh form: 0.5 x (1 + tanh(u)) = x * sigmoid(2 u), u =
+        // sqrt(2/pi) (x + 0.044715 x^3).  The sigmoid form has no cancellation
+        // where tanh(u) nears -1 and costs one exp and one division, about a
+        // third of tanhf (the f32x3 kernel's epilogue has 64 of them per lane)
+        const float u2 = 1.5957691216057308f * (x + 0.044715f * x * x * x);
+        return x / (1.0f + expf(-u2));
     }
     case MOE_ACT_RELU:
         return x > 0.0f ? x : 0.0f;
@@ -223,14 +229,16 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GemmArgs g) {
     }
 }
 
+#include "moe_gemm_f32x3.h"
+
 // Fold of the K-split tiles: block (tile, y) covers elements 256 y .. of the
 // tile; a thread sums its element's S partial sums in range order (a fixed
 // order, so results are deterministic; all S loads in flight first) and
 // applies the kernel's epilogue to it.
-template <int MODE>
+template <int MODE, int BN>
 __global__ __launch_bounds__(256) void fold_f32_kernel(GemmArgs g) {
     constexpr int NB = (MODE == MODE_GATED_UP) ? 2 : 1;
-    constexpr int BM = kGemmBM, BN = kGemmBN;
+    constexpr int BM = kGemmBM;
     const int mt = blockIdx.x % g.m_tiles_grid, nt = blockIdx.x / g.m_tiles_grid;
     if (nt >= g.n_tiles || mt >= g.num_tiles[0]) return;
     const int2 te = g.tiles[mt];
@@ -275,7 +283,22 @@ static hipError_t launch_one(const GemmArgs &g, hipStream_t s) {
     hipLaunchKernelGGL((grouped_gemm_kernel<MODE>), dim3((unsigned)total), dim3(256), 0, s, g);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && g.ksplit > 1) {
-        hipLaunchKernelGGL((fold_f32_kernel<MODE>), dim3((unsigned)(g.m_tiles_grid * g.n_tiles), kGemmBM * kGemmBN / 256),
+        hipLaunchKernelGGL((fold_f32_kernel<MODE, kGemmBN>),
+                           dim3((unsigned)(g.m_tiles_grid * g.n_tiles), kGemmBM * kGemmBN / 256), dim3(256), 0, s, g);
+        e = hipGetLastError();
+    }
+    return e;
+}
+
+template <int MODE>
+static hipError_t launch_f32x3(const GemmArgs &g, hipStream_t s) {
+    constexpr int BN = MODE == MODE_GATED_UP ? 128 : 256;
+    long long total = (long long)g.m_tiles_grid * g.n_tiles * g.ksplit;
+    total = (total + 7) / 8 * 8;
+    hipLaunchKernelGGL((grouped_gemm_f32x3_kernel<MODE>), dim3((unsigned)total), dim3(512), 0, s, g);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && g.ksplit > 1) {
+        hipLaunchKernelGGL((fold_f32_kernel<MODE, BN>), dim3((unsigned)(g.m_tiles_grid * g.n_tiles), kGemmBM * BN / 256),
                            dim3(256), 0, s, g);
         e = hipGetLastError();
     }
@@ -290,13 +313,51 @@ static int f32_ksplit(const GemmArgs &g, int nb) {
     if (!g.split_ws || g.ncu < 1 || tiles <= 0) return 1;
     long long S = std::min<long long>(kF32SplitMax, (2LL * g.ncu) / tiles);
     S = std::min<long long>(S, g.K / 32);
-    S = std::min<long long>(S, g.split_cap / (tiles * nb * kGemmBM * kGemmBN));
+    S = std::min<long long>(S, std::min<long long>(g.split_cap, 2LL * g.ncu * kGemmBM * kGemmBN) /
+                                   (tiles * nb * kGemmBM * kGemmBN));
     return (int)std::max<long long>(1, S);
+}
+
+// Expert segments of 32 rows or more on average run on the bf16 matrix unit:
+// below that the weights' 4 bytes per element bound both kernels, and short
+// segments have more K ranges in grouped_gemm_kernel.  Whole layer,
+// grouped_gemm_kernel / f32x3, us: 1024 / 4096 gated, 16 rows 127 / 125, 32 rows 206 /
+// 128; 768 / 3072 standard, 16 rows 64 / 68, 32 rows 94 / 63; 64 experts of 512 /
+// 1024, 16 rows 132 / 137, 32 rows 219 / 142.
+bool f32x3_rows(int m_tiles_grid, int E) { return 4LL * (m_tiles_grid - E) >= E; }
+
+// K ranges of the f32x3 kernel over one workgroup per CU: the S whose rounds
+// of 1 / S tiles end first (the fold as 8 % of a tile), each range of eight
+// stages or more (1001 / 2731 gated, 144 down tiles of 88 stages: S = 3, one
+// tile's time -> 2/3).
+static int f32x3_ksplit(const GemmArgs &g) {
+    const long long tiles = (long long)g.m_tiles_grid * g.n_tiles;
+    if (!g.split_ws || g.ncu < 1 || tiles <= 0) return 1;
+    int best = 1;
+    double cost = (double)((tiles + g.ncu - 1) / g.ncu);
+    for (int S = 2; S <= kF32SplitMax; ++S) {
+        if (tiles * S * kGemmBM * 256 > g.split_cap || S * 8 > g.K / 32) break;
+        const double c = (double)((tiles * S + g.ncu - 1) / g.ncu) / S + 0.08;
+        if (c < 0.9 * cost) {
+            cost = c;
+            best = S;
+        }
+    }
+    return best;
 }
 
 hipError_t launch_grouped_gemm_f32(int mode, const GemmArgs &g0, hipStream_t s) {
     if (g0.m_tiles_grid <= 0 || g0.n_tiles <= 0) return hipSuccess;
     GemmArgs g = g0;
+    if (f32x3_rows(g.m_tiles_grid, g.E)) {
+        // n_tiles counts 128 output columns; standard and down tiles take 256
+        if (mode != MODE_GATED_UP) g.n_tiles = (g.n_tiles + 1) / 2;
+        g.ksplit = f32x3_ksplit(g);
+        if (mode == MODE_GATED_UP) return launch_f32x3<MODE_GATED_UP>(g, s);
+        if (mode == MODE_STD_UP) return launch_f32x3<MODE_STD_UP>(g, s);
+        if (mode == MODE_DOWN) return launch_f32x3<MODE_DOWN>(g, s);
+        return hipErrorInvalidValue;
+    }
     g.ksplit = f32_ksplit(g, mode == MODE_GATED_UP ? 2 : 1);
     if (mode == MODE_GATED_UP) return launch_one<MODE_GATED_UP>(g, s);
     if (mode == MODE_STD_UP) return launch_one<MODE_STD_UP>(g, s);

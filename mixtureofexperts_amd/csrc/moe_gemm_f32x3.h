@@ -1,0 +1,308 @@
+// moe_gemm_f32x3.h -- the fp32 grouped GEMM on the bf16 matrix unit, for expert
+// segments of many rows.  Part of moe_gemm.hip.
+//
+// An fp32 value is the sum of three bf16 ones (8 significant bits each, rounded
+// to nearest: |x1| <= 2^-9 |x|, |x2| <= 2^-17 |x|), and an fp32 product to
+// fp32 accuracy the sum of the six products of parts i + j <= 2: the three
+// left out are below 2^-25 of it, random in sign, under the rounding of the
+// fp32 sum.  Six v_mfma_f32_32x32x16_bf16 replace eight v_mfma_f32_32x32x2_f32
+// and take 192 cycles instead of 512; the running sums stay fp32 and take
+// 6 roundings per 16 K instead of 8.
+//
+// What bounds it: the matrix unit's power at large sizes, per-tile latencies
+// (24 stages between prologue and epilogue) at small K.  Against
+// grouped_gemm_kernel (whole layer forward, 8 experts, top-2, 4096 tokens):
+// 4096 / 14336 gated 25.4 -> 14.6 ms (198 TFLOP/s of fp32 products), 768 / 3072
+// standard 746 -> 463 us, 1024 / 4096 gated 1861 -> 1081 us; error against 64
+// bits 2.8e-6 -> 2.4e-6, 1.13e-6 -> 0.99e-6, 1.44e-6 -> 1.24e-6.  Two 128 x 128
+// workgroups per CU instead of one kept the MFMAs busier (77 instead of 68 %
+// of cycles) at a lower clock (1.51 instead of 1.66 GHz) and took 4 % longer:
+// what counts is the work besides the MFMAs.  Splitting the last round's tiles
+// into K ranges gained nothing for the same reason (467 and 463 us).
+// Tile 128 rows x 256 weight rows (gated:
+// 128 of W1 and the same 128 of W3), 8 waves as 2 (rows) x 4 (columns), two
+// per SIMD, each 64 x 64.  A stage is 32 K: every thread loads 8 K values of
+// three rows (one of A, two of the weights) two stages ahead, splits them one
+// stage ahead and writes them to the other of two LDS buffers (72 KB each),
+// so the split's vector instructions, the LDS writes and the reads of the
+// next sub-step's fragments run between the MFMAs and there is one barrier
+// per stage (96 MFMAs per SIMD).  Splitting in the kernel repeats it for every tile that reads an
+// operand, but keeps weights, xp and h at 4 bytes in memory and in L2.
+//
+// LDS rows are 64 B (32 bf16 of one part), 16-byte chunk c of row r at c ^
+// ((r >> 2) & 3), as in the bf16 kernel.
+//
+// Infinities, NaN and values that round up to an infinity: their parts give
+// NaN or infinite sums, and every output that is not finite is recomputed
+// from the fp32 operands, one K value after the other.
+//
+// K split (g.ksplit = S > 1): as in grouped_gemm_kernel, blocks of BM x 256
+// floats.
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+
+// Eight fp32 -> three chunks of eight bf16.
+__device__ __forceinline__ void split8(const f32x4_t &a, const f32x4_t &b, u32x4_t (&p)[3]) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float x = i < 2 ? a[2 * i] : b[2 * i - 4], y = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const bf16x2_t h = {(__bf16)x, (__bf16)y};
+            uint32_t u;
+            __builtin_memcpy(&u, &h, 4);
+            p[q][i] = u;
+            if (q < 2) {
+                x = x - __uint_as_float(u << 16);
+                y = y - __uint_as_float(u & 0xffff0000u);
+            }
+        }
+    }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void grouped_gemm_f32x3_kernel(GemmArgs g) {
+    constexpr int NB = (MODE == MODE_GATED_UP) ? 2 : 1;
+    constexpr int BM = kGemmBM, BR = 256;         // tile rows, weight rows
+    constexpr int BN = BR / NB;                   // output columns
+    constexpr int ROWS = BM + BR;                 // LDS rows of a part
+    constexpr int PART = ROWS * 64, STAGE = 3 * PART;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * STAGE];
+
+    // tile order as in grouped_gemm_kernel
+    const int L = blockIdx.x;
+    const int per = gridDim.x >> 3;
+    const int S = g.ksplit;
+    const int id0 = (L & 7) * per + (L >> 3);
+    const int ks = id0 % S, id = id0 / S;
+    const int mt = id % g.m_tiles_grid;
+    const int nt = id / g.m_tiles_grid;
+    if (nt >= g.n_tiles) return;
+    if (mt >= g.num_tiles[0]) return;
+    const int2 te = g.tiles[mt];
+    const int e = te.x, m0 = te.y;
+    const int rows = min(BM, g.counts[e] - m0);
+    const long long arow0 = (long long)g.offsets[e] + m0;
+    const int n0 = nt * BN;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = w & 1, wn = w >> 1;
+    const int half = lane >> 5, r32 = lane & 31;
+
+    // this thread's three rows: row tid / 4 of A, of the first and of the
+    // second 128 weight rows; K values 8 (tid % 4) .. + 8 of each stage
+    const int tr = tid >> 2, tc = tid & 3;
+    const float *A = (const float *)g.A;
+    const float *B0 = (const float *)g.B0 + (long long)e * g.b_stride + (long long)n0 * g.ldb;
+    const float *B1 = NB == 2 ? (const float *)g.B1 + (long long)e * g.b_stride + (long long)n0 * g.ldb
+                              : B0 + 128 * g.ldb;
+    const float *src[3] = {A + (arow0 + min(tr, rows - 1)) * g.lda + 8 * tc, B0 + (long long)tr * g.ldb + 8 * tc,
+                           B1 + (long long)tr * g.ldb + 8 * tc};
+    // (rows tr, 128 + tr and 256 + tr of a part share their swizzle)
+    const int wofs = tr * 64 + ((tc ^ ((tr >> 2) & 3)) << 4);
+    f32x4_t ra[3][2];
+    auto load = [&](int i, int kt) {
+        ra[i][0] = *(const f32x4_t *)(src[i] + (long long)kt * 32);
+        ra[i][1] = *(const f32x4_t *)(src[i] + (long long)kt * 32 + 4);
+    };
+    auto split_store = [&](int buf, int i) {
+        u32x4_t p[3];
+        split8(ra[i][0], ra[i][1], p);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *(u32x4_t *)(lds + buf * STAGE + q * PART + i * 128 * 64 + wofs) = p[q];
+    };
+
+    // fragments: A blocks of 32 rows wm + 2 i (so a tile of few rows is shared
+    // by both wave rows), weight blocks j of the wave's columns (gated: the W1
+    // and W3 rows of 32 h columns)
+    const int sw = (r32 >> 2) & 3;
+    const int afr = (wm * 32 + r32) * 64;
+    int bfr[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bfr[j] = (BM + (NB == 2 ? j * 128 + wn * 32 : wn * 64 + j * 32) + r32) * 64;
+    f32x16_t acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
+
+    const int KTT = g.K / 32;
+    const int kb = (ks * KTT) / S, ke = ((ks + 1) * KTT) / S;
+    const int kl = ke - 1;  // the loads past the range repeat its last stage, into a buffer that nothing reads
+
+    // Stage s is in buffer (s - kb) % 2; its fragments of sub-step 0 are read
+    // in the second half of stage s - 1.  Per stage:
+    //   MFMAs of (s, 0) | reads of (s, 1)     | the weight rows of stage s + 1: split, written, loaded for s + 2
+    //   barrier: stage s + 1 is written, and nothing more is read from buffer s
+    //   MFMAs of (s, 1) | reads of (s + 1, 0) | the A row of stage s + 2: split, written, loaded for s + 3
+    auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+#pragma unroll
+    for (int i = 0; i < 3; ++i) load(i, kb);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) split_store(0, i);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) load(i, min(kb + 1, kl));
+    split_store(1, 0);
+    load(0, min(kb + 2, kl));
+    barrier();
+
+    auto run = [&](auto NV_) {
+        constexpr int NV = decltype(NV_)::value;  // row blocks of this wave that hold rows of the tile
+        bf16x8_t fa[2][2][3], fb[2][2][3];
+        auto read = [&](int buf, int kk) {
+            if constexpr (NV > 0) {
+                const uint8_t *rb = lds + buf * STAGE + (((kk * 2 + half) ^ sw) << 4);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+#pragma unroll
+                    for (int i = 0; i < NV; ++i) fa[kk][i][q] = *(const bf16x8_t *)(rb + q * PART + afr + i * 64 * 64);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) fb[kk][j][q] = *(const bf16x8_t *)(rb + q * PART + bfr[j]);
+                }
+            }
+        };
+        auto mfmas = [&](int kk) {
+#pragma unroll
+            for (int t = 0; t < 6; ++t) {
+                constexpr int PA[6] = {0, 0, 1, 1, 0, 2}, PB[6] = {0, 1, 0, 1, 2, 0};
+#pragma unroll
+                for (int i = 0; i < NV; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][i][PA[t]], fb[kk][j][PB[t]], acc[i][j],
+                                                                            0, 0, 0);
+            }
+        };
+        // after each MFMA: VA vector instructions of the split, then an LDS read or write
+        auto interleave = [&](auto VA_, auto NW_) {
+            constexpr int NM = 12 * NV, NR = 3 * (NV + 2), NW = decltype(NW_)::value;
+#pragma unroll
+            for (int t = 0; t < NM; ++t) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, decltype(VA_)::value, 0);       // vector instructions
+                if (t < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);              // one LDS read
+                if (t >= NM - NW) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);        // one LDS write
+            }
+        };
+        read(0, 0);
+        for (int kt = kb; kt < ke; ++kt) {
+            const int cur = (kt - kb) & 1;
+            read(cur, 1);
+            split_store(cur ^ 1, 1);
+            split_store(cur ^ 1, 2);
+            load(1, min(kt + 2, kl));
+            load(2, min(kt + 2, kl));
+            mfmas(0);
+            if constexpr (NV > 0) interleave(std::integral_constant<int, 10 / NV>{}, std::integral_constant<int, 6>{});
+            barrier();
+            read(cur ^ 1, 0);
+            split_store(cur, 0);
+            load(0, min(kt + 3, kl));
+            mfmas(1);
+            if constexpr (NV > 0) interleave(std::integral_constant<int, 6 / NV>{}, std::integral_constant<int, 3>{});
+        }
+    };
+    const int nv = (rows > wm * 32 ? 1 : 0) + (rows > wm * 32 + 64 ? 1 : 0);  // wave-uniform
+    if (nv == 2) run(std::integral_constant<int, 2>{});
+    else if (nv == 1) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 0>{});
+
+    // ---- epilogue: lane holds column r32 of each 32x32 block, rows
+    // 8*(q/4) + 4*half + q%4.
+    const long long sofs = (long long)e * g.s_stride;
+    // row of the tile of element q of row block i; output column of column block j
+    auto row_of = [&](int i, int q) { return (wm + 2 * i) * 32 + 8 * (q >> 2) + 4 * half + (q & 3); };
+    auto col_of = [&](int j) { return (NB == 2 ? wn * 32 : wn * 64 + j * 32) + r32; };
+    float *ws = S > 1 ? g.split_ws + ((long long)(mt * g.n_tiles + nt) * S + ks) * (BM * BR) : nullptr;
+    unsigned long long bad = 0;  // outputs with a sum that is not finite: bit (j 2 + i) 16 + q
+    // the activation is picked once per tile, and a block's 16 outputs are
+    // computed side by side before their stores (picked per output, the GELU
+    // epilogue of a 24-stage tile took as long as its MFMAs)
+    auto block = [&](int i, int j, auto &&out) {
+        const int nl = col_of(j);
+        if (n0 + nl >= g.N) return;
+        float v[16];
+        const float bias = (MODE != MODE_GATED_UP && g.bias) ? g.bias[sofs + n0 + nl] : 0.0f;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const float v0 = acc[i][j][q], v1 = acc[i][1][q];
+            const bool fin = __builtin_isfinite(v0) && (NB == 1 || __builtin_isfinite(v1));
+            if (!fin && row_of(i, q) < rows) bad |= 1ull << ((j * 2 + i) * 16 + q);
+            v[q] = out(arow0 + row_of(i, q), n0 + nl, bias, v0, v1);
+        }
+        float *c = (float *)g.C + arow0 * g.ldc + n0 + nl;
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            if (row_of(i, q) < rows) c[(long long)row_of(i, q) * g.ldc] = v[q];
+    };
+    auto tile = [&](auto &&out) {
+#pragma unroll
+        for (int j = 0; j < 2 / NB; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) block(i, j, out);
+    };
+    auto finish = [&](auto ACT_, long long row, int n, float bias, float v0, float v1) -> float {
+        constexpr int ACT = decltype(ACT_)::value;
+        if constexpr (MODE == MODE_GATED_UP) return act_apply(ACT, v0) * v1;
+        else if constexpr (MODE == MODE_STD_UP) return dropout_h(g, row, n, act_apply(ACT, v0 + bias));
+        else return v0 + bias;
+    };
+    auto tile_act = [&](auto ACT_) {
+        if (MODE == MODE_STD_UP && g.drop_p > 0.0f) {
+            tile([&](long long row, int n, float bias, float v0, float v1) { return finish(ACT_, row, n, bias, v0, v1); });
+        } else {
+            tile([&](long long, int, float bias, float v0, float v1) -> float {
+                if constexpr (MODE == MODE_STD_UP) return act_apply(decltype(ACT_)::value, v0 + bias);
+                else return finish(ACT_, 0, 0, bias, v0, v1);
+            });
+        }
+    };
+    if (S > 1) {  // a K range: its raw sums, [b][row][column] of split_ws block (tile, ks)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    const int ml = row_of(i, q);
+                    if (ml >= rows) continue;
+                    const int jo = NB == 2 ? 0 : j;
+                    if (!__builtin_isfinite(acc[i][j][q])) bad |= 1ull << ((jo * 2 + i) * 16 + q);
+                    ws[((NB == 2 ? j : 0) * BM + ml) * BN + col_of(jo)] = acc[i][j][q];
+                }
+    } else if constexpr (MODE == MODE_DOWN) {
+        tile_act(std::integral_constant<int, MOE_ACT_IDENTITY>{});
+    } else {
+        switch (g.act) {
+        case MOE_ACT_SILU: tile_act(std::integral_constant<int, MOE_ACT_SILU>{}); break;
+        case MOE_ACT_GELU: tile_act(std::integral_constant<int, MOE_ACT_GELU>{}); break;
+        case MOE_ACT_RELU: tile_act(std::integral_constant<int, MOE_ACT_RELU>{}); break;
+        default: tile_act(std::integral_constant<int, MOE_ACT_IDENTITY>{});
+        }
+    }
+    while (bad) {  // once more from the fp32 rows, one K value after the other; NaN ends a sum
+        const int u = __builtin_ctzll(bad);
+        bad &= bad - 1;
+        const int ml = row_of((u >> 4) & 1, u & 15), nl = col_of(u >> 5), n = n0 + nl;
+        const float *ar = A + (arow0 + ml) * g.lda, *w0 = B0 + (long long)nl * g.ldb, *w1 = B1 + (long long)nl * g.ldb;
+        float v0 = 0.0f, v1 = 0.0f;
+        for (int k = kb * 32; k < ke * 32 && v0 == v0; ++k) v0 = fmaf(ar[k], w0[k], v0);
+        if (NB == 2)
+            for (int k = kb * 32; k < ke * 32 && v1 == v1; ++k) v1 = fmaf(ar[k], w1[k], v1);
+        if (S > 1) {
+            ws[ml * BN + nl] = v0;
+            if (NB == 2) ws[(BM + ml) * BN + nl] = v1;
+            continue;
+        }
+        float v = v0 + ((MODE != MODE_GATED_UP && g.bias) ? g.bias[sofs + n] : 0.0f);
+        if (MODE != MODE_DOWN) v = act_apply(g.act, v);
+        if (MODE == MODE_GATED_UP) v = v * v1;
+        if (MODE == MODE_STD_UP) v = dropout_h(g, arow0 + ml, n, v);
+        ((float *)g.C)[(arow0 + ml) * g.ldc + n] = v;
+    }
+}

@@ -1,0 +1,93 @@
+"""The fp32 layer on expert segments long enough for the bf16 matrix unit
+(three exact bf16 parts per value, six products): against the oracle and, more
+tightly, against 64-bit sums, with infinities and NaN as fp32 gives them.
+
+Bound of the error against 64 bits: each of the two GEMMs sums K products with
+fp32 rounding, a relative error of about sqrt(K) 2^-25 per output (rounding
+errors of random sign on partial sums that grow like sqrt(k)); the layer
+combines both: 8 sqrt(K) 2^-25 <= 1.3e-5 at K = 2816, 4.6e-6 at K = 330."""
+import numpy as np
+import pytest
+
+from test_gpu_layer import Case, check_case
+
+pytestmark = pytest.mark.gpu
+
+
+def exact_forward(c, idx, gates):
+    x = c.x.astype(np.float64)
+    out = np.zeros((c.T, c.Dout))
+    act = {"silu": lambda a: a / (1 + np.exp(-a)), "relu": lambda a: np.maximum(a, 0), "identity": lambda a: a,
+           "gelu": lambda a: 0.5 * a * (1 + np.tanh(np.sqrt(2 / np.pi) * (a + 0.044715 * a ** 3)))}[c.act]
+    for e, w in enumerate(c.ex):
+        t, s = np.nonzero(idx == e + 1)
+        a = x[t] @ w["w1"].T.astype(np.float64)
+        if c.expert_type == "gated":
+            y = (act(a) * (x[t] @ w["w3"].T.astype(np.float64))) @ w["w2"].T.astype(np.float64)
+        else:
+            y = act(a + w["b1"]) @ w["w2"].T.astype(np.float64) + w["b2"]
+        np.add.at(out, t, gates[t, s][:, None].astype(np.float64) * y)
+    return out
+
+
+@pytest.mark.parametrize("T,D,H,Dout,E,k,etype,act", [
+    (512, 100, 330, 90, 8, 2, "gated", "silu"),       # partial tiles, pads in every dimension
+    (64, 64, 128, 260, 2, 1, "gated", "gelu"),        # about 32 rows per expert: one row block, two K stages
+    (1000, 330, 260, 512, 3, 2, "standard", "gelu"),  # both row blocks, std tiles of 256 columns, biases
+    (300, 2816, 64, 64, 2, 2, "standard", "relu"),    # a K split of a small tile grid (88 stages)
+    (700, 64, 2816, 40, 2, 1, "gated", "identity"),   # ... of the down GEMM
+])
+def test_f32x3_layer(moe, oracle, T, D, H, Dout, E, k, etype, act):
+    c = Case(moe, oracle, T=T, D=D, H=H, Dout=Dout, E=E, k=k, gate="switch" if k == 1 else "topk", expert_type=etype,
+             act=act, wdtype="f32", seed=500 + T)
+    try:
+        out, _ = check_case(c, 1e-5)
+        again, _, res = c.run(training=True)
+        assert np.array_equal(out.view(np.uint32), again.view(np.uint32))
+        ref = exact_forward(c, res["indices"], res["gates"])
+        err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+        assert err <= 8 * np.sqrt(max(D, H)) * 2.0 ** -25, err
+    finally:
+        c.dev.close()
+
+
+@pytest.mark.parametrize("H", [96, 2816])
+def test_f32x3_infinities_and_nan(moe, oracle, H):
+    # values whose parts overflow or are not finite: the outputs they enter
+    # are the ones a sequence of fp32 operations gives, the others keep their
+    # bits.  Identity experts whose first output columns copy x (w1 = 1 on one
+    # input, w2 = 1 on one unit), the rest random.  H = 2816: K ranges.
+    T, D = 200, 64
+    c = Case(moe, oracle, T=T, D=D, H=H, E=2, k=1, gate="switch", expert_type="standard", act="identity", wdtype="f32",
+             seed=61, max_tokens=T)
+    try:
+        print(f"f32x3 infinities H={H}", flush=True)
+        w1 = np.zeros((H, D), np.float32)
+        w1[np.arange(D), np.arange(D)] = 1.0
+        w2 = np.zeros((D, H), np.float32)
+        w2[np.arange(D), np.arange(D)] = 1.0
+        for e in range(2):
+            c.dev.set_expert(e, w1, w2, None, np.zeros(H, np.float32), np.zeros(D, np.float32))
+        # the caller's routing, every token to expert 1 with gate 1: the gates
+        # do not depend on x then
+        def forward(x):
+            return c.dev.forward_routed(x, 0, False, np.ones((T, 1), np.int32), np.ones((T, 1), np.float32))[0]
+
+        x = np.ascontiguousarray(c.x)
+        out = forward(x)
+        assert np.array_equal(out, x)
+        big = x.copy()
+        big[3, :] = 3.4e38     # finite in fp32, above bf16's largest value
+        big[4, :] = -3.4028235e38
+        o = forward(big)
+        assert np.array_equal(o, big)
+        bad = x.copy()
+        bad[5, 7], bad[6, 9], bad[130, 0] = np.inf, np.nan, -np.inf
+        o = forward(bad)
+        # an infinity or NaN times the zero weights of a row is NaN, as in fp32
+        assert np.isnan(o[6]).all() and o[5, 7] != x[5, 7] and not np.isfinite(o[5, 7])
+        keep = np.ones(T, bool)
+        keep[[5, 6, 130]] = False
+        assert np.array_equal(o[keep], x[keep])
+    finally:
+        c.dev.close()
