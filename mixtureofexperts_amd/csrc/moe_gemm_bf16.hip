@@ -1,6 +1,6 @@
 // moe_gemm_bf16.hip -- the bf16 grouped expert GEMM (the layer's MFMA-bound
 // hot spot) for CDNA4: direct global->LDS loads into a ring of LDS stages,
-// 256-column block tiles on v_mfma_f32_32x32x16_bf16, with the expert FFN's
+// 256-column block tiles on v_mfma_f32_16x16x32_bf16, with the expert FFN's
 // elementwise work in the epilogue.
 //
 //   MODE_GATED_UP : h = act(A W1^T) .* (A W3^T)       GatedExpert (src/experts/gated.jl:29-34)
@@ -26,20 +26,20 @@
 // assigned in contiguous per-XCD ranges: the blocks that share a weight tile
 // and walk K in step run behind the same L2.
 //
-// Block: 4 waves, one per SIMD, as 2 (M) x 2 (N); each wave owns a (BM/2) x 128
-// sub-tile and interleaves its MFMAs with the fragment reads of the next
-// sub-step and the loads NS-1 stages ahead.  A wave runs MFMAs only on its
+// Block: BM / 32 waves, as BM / 64 (M) x 2 (N); each wave owns 64 x 128 outputs
+// and interleaves its MFMAs with the fragment reads of the next half stage
+// and the loads NS-1 stages ahead.  A wave runs MFMAs only on its
 // 32-row blocks that hold rows of the tile: the last tile of an expert skips
 // the padding past the expert's last row.
 //
 // For MODE_GATED_UP the 256 B-tile rows are 128 rows of W1 followed by the
-// same 128 rows of W3, and each wave's four 32-column blocks are (gate, up)
+// same 128 rows of W3, and each wave's eight 16-column blocks are (gate, up)
 // pairs for 64 h columns, so the silu-mul pairs sit in the same lane's
 // registers.
 //
 // LDS: per stage an A tile (BM rows) and a B tile (256 rows) of 32 bf16 =
 // 64 B per row; the 16-byte chunks of row r are stored at chunk ^ ((r >> 2) & 3)
-// so the fragment reads (32 rows, one chunk) spread over all 64 banks.  Each
+// so the fragment reads (16 rows, four chunks) spread over all 64 banks.  Each
 // global_load_lds_dwordx4 writes 1 KB = 16 rows linearly (lane l -> offset
 // 16 l), so the swizzle is part of the tile images.
 #include <algorithm>
@@ -50,7 +50,7 @@
 namespace moe {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 #define MOE_LDS_AS __attribute__((address_space(3)))
 
 // Activation in the epilogue of the bf16 path (outputs are rounded to bf16 or
@@ -289,12 +289,12 @@ __device__ __forceinline__ void load_plan(const GemmArgs &g, const TileJob &jb, 
     }
 }
 
-// B-tile row of fragment block j of a wave whose column group is wn (WN
-// B-tile rows per group).  Gated: blocks 2m and 2m + 1 are the W1 and W3 rows
-// of h columns wn * WN / 2 + 32 m.
-template <int NB, int WN>
-__device__ __forceinline__ int b_frag_row(int j, int wn) {
-    return (NB == 2) ? ((j & 1) * 128 + wn * (WN / 2) + (j >> 1) * 32) : (wn * WN + j * 32);
+// B-tile row of fragment block j (16 rows) of a wave, past its first one (WN
+// B-tile rows per wave column group).  Gated: blocks 2m and 2m + 1 are the W1
+// and W3 rows of h columns 16 m.
+template <int NB>
+__device__ constexpr int b_frag_row(int j) {
+    return (NB == 2) ? ((j & 1) * 128 + (j >> 1) * 16) : (j * 16);
 }
 
 // Component c (a compile-time constant after unrolling) of a float4.
@@ -305,12 +305,16 @@ __device__ __forceinline__ float f4_at(const float4 &v, int c) {
 template <int N>
 using ic = std::integral_constant<int, N>;
 
+// Threads of a workgroup: waves of 64 x 128 outputs, 4 of them for 128-row
+// tiles, 8 for 256-row tiles.
+constexpr int gemm_threads(int BM) { return 2 * BM; }
+
 // ---- epilogue ---------------------------------------------------------------------
 // The MFMA computes the transposed block (weights are its A operand): lane l
-// holds token row l % 32 of the 32-row block and output columns 8 (q / 4) +
-// 4 (l / 32) + q % 4, i.e. four consecutive columns per q / 4.  row0: the
-// wave's first tile row.  WF8: the accumulators are scaled by the weight
-// rows' scales (s0: W1 or W2, s1: W3) before bias and activation.
+// holds token row l % 16 of the 16-row block and the four consecutive output
+// columns from 4 (l / 16) of the 16-column block.  Row blocks 2 b, 2 b + 1 of
+// wave row wm are the tile's 32 rows wm + MW b.  WF8: the accumulators are scaled by the weight rows' scales (s0: W1 or
+// W2, s1: W3) before bias and activation.
 //
 // bf16 outputs (h of both up modes; y of the down GEMM when c_bf16) go to
 // put(ml, lc, v0, v1, v2, v3): tile row ml, tile column lc (a multiple of 4),
@@ -319,11 +323,11 @@ using ic = std::integral_constant<int, N>;
 // N or ldc is not a multiple of 8, stores them directly (DirectPut: 8 bytes
 // per lane, 32 rows per store instruction).  fp32 y and the partials of
 // split tiles are stored directly.
-template <int MODE, int ACT, int IM, int JN, int WN, int WF8, typename Put>
-__device__ __forceinline__ void store_tile(const GemmArgs &g, const TileJob &jb, const f32x16_t (&acc)[IM][JN],
-                                           int row0, int wn, int lane, Put &&put) {
-    const int half = lane >> 5;
-    const int r32 = lane & 31;
+template <int MODE, int BM, int ACT, int MW, int IM, int JN, int WN, int WF8, typename Put>
+__device__ __forceinline__ void store_tile(const GemmArgs &g, const TileJob &jb, const f32x4_t (&acc)[IM][JN],
+                                           int wm, int wn, int lane, Put &&put) {
+    const int q4 = lane >> 4;
+    const int r16 = lane & 15;
     const long long sofs = (long long)jb.e * g.s_stride;
     // The per-column vectors of the lane's column groups (weight scales, the
     // bias) are loaded in batches ahead of the accumulator reads that use
@@ -332,113 +336,105 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const TileJob &jb,
     if constexpr (MODE == MODE_GATED_UP) {
         // h pad columns [N, Npad) come out as act(0) * 0 = 0 from the zero weight
         // pad rows, so the whole tile is stored (ldc = Npad).
-        constexpr int NG = (JN / 2) * 4;  // column groups of 4 h columns of the lane
+        constexpr int NG = JN / 2;  // column groups of 4 h columns of the lane
         float4 sg[NG], su[NG];
         if constexpr (WF8) {
 #pragma unroll
-            for (int q = 0; q < NG; ++q) {
-                const int lc = wn * (WN / 2) + (q >> 2) * 32 + 8 * (q & 3) + 4 * half;
-                sg[q] = *(const float4 *)(g.s0 + sofs + jb.n0 + lc);
-                su[q] = *(const float4 *)(g.s1 + sofs + jb.n0 + lc);
+            for (int m = 0; m < NG; ++m) {
+                const int lc = wn * (WN / 2) + m * 16 + 4 * q4;
+                sg[m] = *(const float4 *)(g.s0 + sofs + jb.n0 + lc);
+                su[m] = *(const float4 *)(g.s1 + sofs + jb.n0 + lc);
             }
         }
 #pragma unroll
-        for (int m = 0; m < JN / 2; ++m)
+        for (int m = 0; m < NG; ++m) {
+            const int lc = wn * (WN / 2) + m * 16 + 4 * q4;
 #pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const int q = m * 4 + g4;
-                const int lc = wn * (WN / 2) + m * 32 + 8 * g4 + 4 * half;
+            for (int i = 0; i < IM; ++i) {
+                const int ml = (wm + MW * (i >> 1)) * 32 + (i & 1) * 16 + r16;
+                float v[4];
 #pragma unroll
-                for (int i = 0; i < IM; ++i) {
-                    const int ml = row0 + i * 32 + r32;
-                    float v[4];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        float gt = acc[i][2 * m][4 * g4 + c], up = acc[i][2 * m + 1][4 * g4 + c];
-                        if constexpr (WF8) {
-                            gt = gt * f4_at(sg[q], c);
-                            up = up * f4_at(su[q], c);
-                        }
-                        v[c] = act_fast<ACT>(gt) * up;
+                for (int c = 0; c < 4; ++c) {
+                    float gt = acc[i][2 * m][c], up = acc[i][2 * m + 1][c];
+                    if constexpr (WF8) {
+                        gt = gt * f4_at(sg[m], c);
+                        up = up * f4_at(su[m], c);
                     }
-                    put(ml, lc, v[0], v[1], v[2], v[3]);
+                    v[c] = act_fast<ACT>(gt) * up;
                 }
+                put(ml, lc, v[0], v[1], v[2], v[3]);
             }
+        }
     } else {
         // MODE_STD_UP stores bf16 h (pads are act(b1 pad = 0) of zero rows: 0 for
         // silu, gelu, relu, identity); MODE_DOWN stores y with ldc = N, in bf16
-        // (c_bf16) or fp32.  The lane's column blocks in two parts (four with
-        // fp8 scales on 256-row tiles, whose accumulators leave fewer
-        // registers), each with one batch of vector loads.
+        // (c_bf16) or fp32.  The lane's column blocks in two parts, each with one
+        // batch of vector loads.
         const bool vec4 = (MODE == MODE_STD_UP) || ((g.ldc & 3) == 0);
         const bool yb = (MODE == MODE_STD_UP) || (g.c_bf16 && jb.nks == 1);
         const bool has_bias = g.bias && jb.ks == 0;  // split K: the bias belongs to one partial sum only
-        constexpr int JH = ((WF8 || MODE == MODE_STD_UP) && IM == 4) ? 1 : (JN + 1) / 2;  // column blocks per part
+        constexpr int JH = JN / 2;  // column blocks per part
         auto part = [&](auto H_, auto DROP_) {
             constexpr int H = decltype(H_)::value;
             constexpr bool DROP = decltype(DROP_)::value;
             constexpr int J0 = H * JH, J1 = (J0 + JH < JN) ? J0 + JH : JN;
-            float4 bv[JH * 4], sc[JH * 4];
+            float4 bv[JH], sc[JH];
 #pragma unroll
-            for (int q = 0; q < (J1 - J0) * 4; ++q) {
-                const int n = jb.n0 + wn * WN + (J0 + (q >> 2)) * 32 + 8 * (q & 3) + 4 * half;
+            for (int q = 0; q < J1 - J0; ++q) {
+                const int n = jb.n0 + wn * WN + (J0 + q) * 16 + 4 * q4;
                 bv[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 if (has_bias) bv[q] = *(const float4 *)(g.bias + sofs + n);
                 if constexpr (WF8) sc[q] = *(const float4 *)(g.s0 + sofs + n);
             }
 #pragma unroll
-            for (int j = J0; j < J1; ++j)
+            for (int j = J0; j < J1; ++j) {
+                const int q = j - J0;
+                const int lc = wn * WN + j * 16 + 4 * q4;
+                const int n = jb.n0 + lc;
 #pragma unroll
-                for (int g4 = 0; g4 < 4; ++g4) {
-                    const int q = (j - J0) * 4 + g4;
-                    const int lc = wn * WN + j * 32 + 8 * g4 + 4 * half;
-                    const int n = jb.n0 + lc;
+                for (int i = 0; i < IM; ++i) {
+                    const int ml = (wm + MW * (i >> 1)) * 32 + (i & 1) * 16 + r16;
+                    float a[4];
 #pragma unroll
-                    for (int i = 0; i < IM; ++i) {
-                        const int ml = row0 + i * 32 + r32;
-                        float a[4];
+                    for (int c = 0; c < 4; ++c) {
+                        a[c] = acc[i][j][c];
+                        if constexpr (WF8) a[c] = a[c] * f4_at(sc[q], c);
+                        a[c] = a[c] + f4_at(bv[q], c);
+                    }
+                    if constexpr (MODE == MODE_STD_UP) {
+                        float h4[4];
 #pragma unroll
                         for (int c = 0; c < 4; ++c) {
-                            a[c] = acc[i][j][4 * g4 + c];
-                            if constexpr (WF8) a[c] = a[c] * f4_at(sc[q], c);
-                            a[c] = a[c] + f4_at(bv[q], c);
+                            h4[c] = act_fast<ACT>(a[c]);
+                            if constexpr (DROP) h4[c] = dropout_h(g, jb.arow0 + ml, n + c, h4[c]);
                         }
-                        if constexpr (MODE == MODE_STD_UP) {
-                            float h4[4];
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) {
-                                h4[c] = act_fast<ACT>(a[c]);
-                                if constexpr (DROP) h4[c] = dropout_h(g, jb.arow0 + ml, n + c, h4[c]);
-                            }
-                            put(ml, lc, h4[0], h4[1], h4[2], h4[3]);
-                        } else if (yb) {
-                            put(ml, lc, a[0], a[1], a[2], a[3]);
+                        put(ml, lc, h4[0], h4[1], h4[2], h4[3]);
+                    } else if (yb) {
+                        put(ml, lc, a[0], a[1], a[2], a[3]);
+                    } else {
+                        if (ml >= jb.rows) continue;
+                        // fp32 y: K range 0 (or an unsplit tile) writes y; range
+                        // r >= 1 its partial block in split_ws (BM x 256, row
+                        // stride 256).  bf16 y: every range writes its block.
+                        const long long blk = g.c_bf16 ? (long long)jb.split_j * jb.nks + jb.ks
+                                                       : (long long)jb.split_j * (jb.nks - 1) + jb.ks - 1;
+                        float *crow = (jb.ks == 0 && !g.c_bf16)
+                                          ? (float *)g.C + (jb.arow0 + ml) * g.ldc
+                                          : g.split_ws + blk * BM * 256 + (long long)ml * 256 - jb.n0;
+                        if (vec4 && n + 3 < g.N) {
+                            *(float4 *)(crow + n) = make_float4(a[0], a[1], a[2], a[3]);
                         } else {
-                            if (ml >= jb.rows) continue;
-                            // fp32 y: K range 0 (or an unsplit tile) writes y; range
-                            // r >= 1 its partial block in split_ws (BM x 256, row
-                            // stride 256).  bf16 y: every range writes its block.
-                            const long long blk = g.c_bf16 ? (long long)jb.split_j * jb.nks + jb.ks
-                                                           : (long long)jb.split_j * (jb.nks - 1) + jb.ks - 1;
-                            float *crow = (jb.ks == 0 && !g.c_bf16)
-                                              ? (float *)g.C + (jb.arow0 + ml) * g.ldc
-                                              : g.split_ws + blk * (IM * 64) * 256 + (long long)ml * 256 - jb.n0;
-                            if (vec4 && n + 3 < g.N) {
-                                *(float4 *)(crow + n) = make_float4(a[0], a[1], a[2], a[3]);
-                            } else {
 #pragma unroll
-                                for (int c = 0; c < 4; ++c)
-                                    if (n + c < g.N) crow[n + c] = a[c];
-                            }
+                            for (int c = 0; c < 4; ++c)
+                                if (n + c < g.N) crow[n + c] = a[c];
                         }
                     }
                 }
+            }
         };
         auto tile = [&](auto DROP_) {
             part(ic<0>{}, DROP_);
-            if constexpr (JN > JH) part(ic<1>{}, DROP_);
-            if constexpr (JN > 2 * JH) part(ic<2>{}, DROP_);
-            if constexpr (JN > 3 * JH) part(ic<3>{}, DROP_);
+            part(ic<1>{}, DROP_);
         };
         if constexpr (MODE == MODE_STD_UP) {
             if (g.drop_p > 0.0f) tile(std::true_type{});
@@ -487,33 +483,33 @@ struct StagePut {
 // Stores the staged tile.  Up GEMMs: h goes out as the down GEMM's A tile
 // image, in which the tile's CW / 64 K stages of 64-B rows are one contiguous
 // region (all BM rows, including rows past the valid ones): thread t writes
-// 16-byte units t, t + 256, ..., unit u being chunk position u & 3 of row
+// 16-byte units t, t + NT, ... (NT threads), unit u being chunk position u & 3 of row
 // (u >> 2) mod BM of stage block u / (4 BM).  Down GEMM: y rows; thread t
-// copies chunk t mod CH of rows t / CH + k (256 / CH), valid rows only and
+// copies chunk t mod CH of rows t / CH + k (NT / CH), valid rows only and
 // the chunks below N (N a multiple of 8).  U LDS reads are in flight before
 // their global stores.
 template <int MODE, int BM, int CH, typename RowAddr>
 __device__ __forceinline__ void store_staged(const GemmArgs &g, const TileJob &jb, RowAddr row_addr) {
-    constexpr int U = 8;
+    constexpr int U = 8, NT = gemm_threads(BM);
     if constexpr (MODE != MODE_DOWN) {
         constexpr int NU = BM * CH;  // 16-byte units of the tile
         const long long KTT = g.ldc / 32;  // h: K of the down GEMM = ldc
         uint8_t *base = (uint8_t *)g.C + ((long long)jb.mt * KTT + jb.n0 / 32) * BM * 64;
 #pragma unroll
-        for (int u0 = 0; u0 < NU; u0 += 256 * U) {
+        for (int u0 = 0; u0 < NU; u0 += NT * U) {
             u32x4_t v[U];
 #pragma unroll
             for (int q = 0; q < U; ++q) {
-                const int u = u0 + q * 256 + (int)threadIdx.x;
+                const int u = u0 + q * NT + (int)threadIdx.x;
                 const int r = (u >> 2) % BM;
                 const int ch = (u / (4 * BM)) * 4 + ((u & 3) ^ ((r >> 2) & 3));  // column chunk in the tile
                 v[q] = *(const MOE_LDS_AS u32x4_t *)(row_addr(r) + ((ch ^ (r & (CH - 1))) << 4));
             }
 #pragma unroll
-            for (int q = 0; q < U; ++q) *(u32x4_t *)(base + (long long)(u0 + q * 256 + threadIdx.x) * 16) = v[q];
+            for (int q = 0; q < U; ++q) *(u32x4_t *)(base + (long long)(u0 + q * NT + threadIdx.x) * 16) = v[q];
         }
     } else {
-        constexpr int RPP = 256 / CH;  // rows per pass of the workgroup
+        constexpr int RPP = NT / CH;  // rows per pass of the workgroup
         const int ch = threadIdx.x % CH;
         const int rr = threadIdx.x / CH;
         const bool colok = jb.n0 + ch * 8 < g.N;
@@ -539,17 +535,17 @@ __device__ __forceinline__ void store_staged(const GemmArgs &g, const TileJob &j
 // h image blocks (units as in store_staged, per n-tile).
 template <int MODE, int BM, int CH, typename RowAddr>
 __device__ __forceinline__ void store_staged_pair(const GemmArgs &g, const TileJob &jb, RowAddr row_addr) {
-    constexpr int U = 8;
+    constexpr int U = 8, NT = gemm_threads(BM);
     constexpr int BMA = BM / 2;
     constexpr int NUH = BMA * CH;                               // 16-byte units per n-tile
     constexpr int NTW = (MODE == MODE_GATED_UP) ? 128 : 256;    // h columns per n-tile
     const long long KTT = g.ldc / 32;
 #pragma unroll
-    for (int u0 = 0; u0 < 2 * NUH; u0 += 256 * U) {
+    for (int u0 = 0; u0 < 2 * NUH; u0 += NT * U) {
         u32x4_t v[U];
 #pragma unroll
         for (int q = 0; q < U; ++q) {
-            const int u = u0 + q * 256 + (int)threadIdx.x;
+            const int u = u0 + q * NT + (int)threadIdx.x;
             const int hf = u / NUH, up = u - hf * NUH;
             const int r = (up >> 2) % BMA;
             const int ch = (up / (4 * BMA)) * 4 + ((up & 3) ^ ((r >> 2) & 3));
@@ -557,7 +553,7 @@ __device__ __forceinline__ void store_staged_pair(const GemmArgs &g, const TileJ
         }
 #pragma unroll
         for (int q = 0; q < U; ++q) {
-            const int u = u0 + q * 256 + (int)threadIdx.x;
+            const int u = u0 + q * NT + (int)threadIdx.x;
             const int hf = u / NUH, up = u - hf * NUH;
             uint8_t *base = (uint8_t *)g.C + ((long long)jb.mt * KTT + (jb.n0 + hf * NTW) / 32) * BM * 64;
             *(u32x4_t *)(base + (long long)(up / (4 * BMA)) * BM * 64 + (up % (4 * BMA)) * 16) = v[q];
@@ -612,11 +608,20 @@ struct RowOffsetPut {
     }
 
 // ============================================================================
-// 4-wave interleaved kernel, BM = 128 or 256.
+// The kernel, BM = 128 or 256.
 // ============================================================================
-// OCC: workgroups per CU.  128-row tiles (small experts, weight-bandwidth
-// bound, or short K) run two per CU on a shorter ring, so one workgroup's
-// prologue and epilogue overlap the other's main loop.
+// v_mfma_f32_16x16x32_bf16: at the card's power limit a loop of it alone runs
+// 2040 TFLOP/s, one of v_mfma_f32_32x32x16_bf16 1770 (random operands, 128 x
+// 128 per wave), and the GEMMs here are at that limit.  Up / down GEMM, us, with
+// the 32x32x16 instruction (128 x 128 waves on 256-row tiles) and now: 66 fp8
+// experts of 2048 / 1408, 8192 tokens: 654 / 350 and 604 / 323; 8 bf16 experts
+// of 4096 / 14336, 4096 tokens: 1577 / 841 and 1506 / 790 (1.28 PFLOP/s, up).
+// A wave's 64 x 128 outputs are 128 accumulator registers; a 128 x 128 wave
+// (256 of them in 64 blocks) spilled hundreds.
+// Two waves per SIMD: one workgroup of eight on 256-row tiles; on 128-row
+// tiles (small experts, weight-bandwidth bound, or short K) two workgroups of
+// four on a shorter ring, so one's prologue and epilogue overlap the other's
+// main loop (OCC: workgroups per CU).
 //
 // The LDS ring: one array of RING bytes; slot J of a stage size STAGE at J
 // STAGE.  The staged epilogue reuses it as rows of CW bytes.
@@ -629,19 +634,29 @@ struct RingShape {
 
 // One work item.  SPLIT: a K range of a split up-GEMM tile, which stores its
 // partial sums (its own instantiation: the branch after the main loop would
-// keep registers live through it).  PAIR: a paired item (decode_item): 4
-// waves as 2 (n-tile
-// of the pair) x 2 (N), each over the item's BM / 2 rows; otherwise 2 (M) x 2
-// (N) over the BM rows of one n-tile.
-template <int IM, int JN>
-__device__ __forceinline__ void store_partial(const GemmArgs &g, const TileJob &jb, const f32x16_t (&acc)[IM][JN]);
+// keep registers live through it).  Waves: MW (M) x 2 (N) over the BM rows of
+// one n-tile, wave row wm taking the 32-row blocks wm and wm + MW (so that a
+// partial tile's blocks are spread over the SIMDs); PAIR: a paired item
+// (decode_item), 2 (M) x 2 (n-tile of the pair) x 2 (N) over the item's BM / 2
+// rows.
+template <int BM, int IM, int JN>
+__device__ __forceinline__ void store_partial(const GemmArgs &g, const TileJob &jb, const f32x4_t (&acc)[IM][JN]);
 template <int MODE, int BM, int ACT, int WF8, int OCC, bool PAIR, int IM, int JN>
-__device__ __forceinline__ void tile_epilogue(const GemmArgs &g, const TileJob &jb, const f32x16_t (&acc)[IM][JN],
+__device__ __forceinline__ void tile_epilogue(const GemmArgs &g, const TileJob &jb, const f32x4_t (&acc)[IM][JN],
                                               uint8_t *ring_);
+
+// Wave w's place: row group wm of MW, n-tile pt of a pair, column half wn.
+struct WavePlace { int wm, pt, wn; };
+template <int BM, bool PAIR>
+__device__ __forceinline__ WavePlace wave_place(int w) {
+    if constexpr (PAIR) return WavePlace{w & 1, (w >> 1) & 1, w >> 2};
+    else return WavePlace{w % (BM / 64), 0, w / (BM / 64)};
+}
 
 template <int MODE, int BM, int ACT, int WF8, int OCC, bool PAIR, bool SPLIT = false>
 __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, uint8_t *ring_) {
-    constexpr int NWAVE = 4;
+    constexpr int NWAVE = gemm_threads(BM) / 64;
+    static_assert(!PAIR || BM == 256, "pairs: 256-row tiles");
     constexpr int NB = (MODE == MODE_GATED_UP) ? 2 : 1;
     constexpr int ROWB = 64;             // bytes per LDS A row = 32 bf16 of K (one stage)
     constexpr int BROWB = WF8 ? 32 : 64; // bytes per LDS B row
@@ -654,10 +669,11 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
     // LDS ring slots (<= 144 KB per CU)
     constexpr int NS = PAIR ? RING / STAGE : RingShape<BM, WF8, OCC>::NS;
     static_assert(NS >= 3 && NS <= 6, "ring depth");
-    constexpr int WM = BM / 2;           // wave tile rows (2 waves along M; PAIR: the item's BM / 2 rows)
+    constexpr int MW = BMA / 64;         // waves along M, 64 rows each
     constexpr int WN = 128;              // wave tile columns (2 waves along N)
-    constexpr int IM = WM / 32;          // 32-row blocks per wave
-    constexpr int JN = WN / 32;          // 32-column blocks per wave
+    constexpr int IM = 4;                // 16-row blocks per wave
+    constexpr int JN = WN / 16;          // 16-column blocks per wave
+    constexpr int JH = JN / 2;           // of which in each half of a stage
     constexpr int LA = BMA / (16 * NWAVE);  // A loads (16 rows each) per wave per stage
     constexpr int LB = BRW / ((WF8 ? 32 : 16) * NWAVE);  // B loads per wave per stage
     constexpr int NL = LA + LB;          // 16-byte loads per lane per stage
@@ -671,7 +687,8 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
     const int KT = jb.KT;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = w & 1, wn = w >> 1;
+    const WavePlace wp = wave_place<BM, PAIR>(w);
+    const int wm = wp.wm, wn = wp.wn;
 
     const uint8_t *gsrc[NL];
     uint32_t ldst[NL];
@@ -683,45 +700,39 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
                   __builtin_amdgcn_readfirstlane(l));
     };
 
-    // ---- fragment addressing (fragment row bases are multiples of 32, so
-    // swz(row) = (r32 >> 2) & 3) ------------------------------------------------
-    // Lane (r32, half) supplies 8 K values per k16 sub-step kk: K 16 kk + 8 half
-    // (bf16 weights, A chunk 2 kk + half) or K 16 half + 8 kk (fp8 weights: A
-    // chunk 2 half + kk, and the lane's 16 weight bytes of the stage, K 16 half
-    // .. +16, are one B chunk read once per stage).  The MFMA sums over K, so any
-    // assignment of K values to (sub-step, lane half) shared by A and B works.
-    const int half = lane >> 5;
-    const int r32 = lane & 31;
-    const int a_frag = ((PAIR ? 0 : wm * WM) + r32) * ROWB;
-    int b_frag[JN];
-#pragma unroll
-    for (int j = 0; j < JN; ++j)
-        b_frag[j] = A_BYTES + ((PAIR ? wm * 256 : 0) + b_frag_row<NB, WN>(j, wn) + r32) * BROWB +
-                    (WF8 ? ((half ^ ((r32 >> 3) & 1)) << 4) : 0);
-    int choff[2];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-        choff[kk] = ((WF8 ? (half * 2 + kk) : (kk * 2 + half)) ^ ((r32 >> 2) & 3)) << 4;
+    // ---- fragment addressing (fragment row bases are multiples of 16, so the
+    // swizzle depends on the lane alone) -----------------------------------------
+    // Lane (r16, q4) supplies row r16 of a 16-row block, K 8 q4 .. +8 of the
+    // stage (A and bf16 weights: chunk q4 of the row; fp8 weights: half of
+    // chunk q4 / 2).
+    const int q4 = lane >> 4;
+    const int r16 = lane & 15;
+    const int a_frag = (wm * 32 + r16) * ROWB + ((q4 ^ ((r16 >> 2) & 3)) << 4);
+    const int b_frag = A_BYTES + (wp.pt * 256 + wn * (NB == 2 ? WN / 2 : WN) + r16) * BROWB +
+                       (WF8 ? ((((q4 >> 1) ^ ((r16 >> 3) & 1)) << 4) + ((q4 & 1) << 3))
+                            : ((q4 ^ ((r16 >> 2) & 3)) << 4));
 
-    f32x16_t acc[IM][JN];
+    f32x4_t acc[IM][JN];
 #pragma unroll
     for (int i = 0; i < IM; ++i)
 #pragma unroll
         for (int j = 0; j < JN; ++j)
 #pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
+            for (int q = 0; q < 4; ++q) acc[i][j][q] = 0.0f;
 
-    bf16x8_t fa[2][IM], fb[2][JN];
-    u32x4_t braw[JN];  // WF8: this stage's weight bytes (K 16 half .. +16) per column block
+    bf16x8_t fa[IM], fb[2][JH];
+    u32x2_t braw[2][JH];  // WF8: the weight bytes, widened when they are used
 
     // ---- main loop --------------------------------------------------------------
-    // Stage s (32 K columns, two k16 sub-steps) lives in ring slot s % NS and is
-    // loaded NS - 1 stages ahead.  Per stage:
-    //   sub-step 0: MFMAs of (s, 0) | LDS reads of (s, 1)   | loads of stage s+NS-1, first half
+    // Stage s (32 K columns) lives in ring slot s % NS and is loaded NS - 1
+    // stages ahead.  Its MFMAs run in two halves of the wave's columns, rows in
+    // order; a row block's fragment is replaced by the next stage's once the
+    // second half is past it.  Per stage:
+    //   half 0: MFMAs of columns [0, JH)  | LDS reads of (s, columns [JH, JN))       | loads of stage s+NS-1, first half
     //   wait until this wave's loads of stage s+1 landed; barrier (every wave's have)
-    //   sub-step 1: MFMAs of (s, 1) | LDS reads of (s+1, 0) | loads of stage s+NS-1, second half
-    // Stage s+NS-1 goes to the slot of stage s-1, whose last reads (its sub-step
-    // 1 fragments) ended before the barrier of stage s-1.  Past the last stage
+    //   half 1: MFMAs of columns [JH, JN) | LDS reads of (s+1, rows, columns [0, JH)) | loads of stage s+NS-1, second half
+    // Stage s+NS-1 goes to the slot of stage s-1, whose last reads (its half 0)
+    // ended before the barrier of stage s-1.  Past the last stage
     // the loads repeat stage KT-1 (in bounds, into a slot nothing reads again),
     // which keeps the vmcnt arithmetic exact: when the barrier of stage s is
     // reached, the loads issued after those of stage s+1 are NS-3 whole stages
@@ -737,119 +748,116 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
     // 0 and their rows are not stored.
     auto run = [&](auto NV_) {
         constexpr int NV = decltype(NV_)::value;
-        constexpr int NMF = NV * JN;
-        // WF8: sub-step 0 reads the stage's weight bytes; each sub-step widens
-        // its 8 bytes (words 2 kk, 2 kk + 1 of braw) to bf16.
-        auto read_frags = [&](auto J_, int kk, bf16x8_t *af, bf16x8_t *bfr) {
+        constexpr int NF = 2 * NV;  // row blocks of 16
+        auto read_a = [&](auto J_, int i) { 
+            fa[i] = *(const MOE_LDS_AS bf16x8_t *)(slot(J_) + a_frag + ((i >> 1) * MW * 32 + (i & 1) * 16) * ROWB);
+        };
+        auto read_b = [&](auto J_, int hf) {
             if constexpr (NV > 0) {
-                const MOE_LDS_AS uint8_t *sb = slot(J_);
+                const MOE_LDS_AS uint8_t *sb = slot(J_) + b_frag;
 #pragma unroll
-                for (int r = 0; r < NV; ++r)
-                    af[r] = *(const MOE_LDS_AS bf16x8_t *)(sb + a_frag + r * 32 * ROWB + choff[kk]);
-#pragma unroll
-                for (int j = 0; j < JN; ++j) {
-                    if constexpr (WF8) {
-                        if (kk == 0) braw[j] = *(const MOE_LDS_AS u32x4_t *)(sb + b_frag[j]);
-                        bfr[j] = widen_fp8x8(braw[j][2 * kk], braw[j][2 * kk + 1]);
-                    } else {
-                        bfr[j] = *(const MOE_LDS_AS bf16x8_t *)(sb + b_frag[j] + choff[kk]);
-                    }
+                for (int j = 0; j < JH; ++j) {
+                    const int o = b_frag_row<NB>(hf * JH + j) * BROWB;
+                    if constexpr (WF8) braw[hf][j] = *(const MOE_LDS_AS u32x2_t *)(sb + o);
+                    else fb[hf][j] = *(const MOE_LDS_AS bf16x8_t *)(sb + o);
                 }
             }
         };
-        auto mfmas = [&](const bf16x8_t *af, const bf16x8_t *bfr) {
+        auto widen = [&](int hf) {
+            if constexpr (WF8 && NV > 0)
 #pragma unroll
-            for (int i = 0; i < NV; ++i)
-#pragma unroll
-                for (int j = 0; j < JN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[j], af[i], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < JH; ++j) fb[hf][j] = widen_fp8x8(braw[hf][j][0], braw[hf][j][1]);
         };
-        // One MFMA, then one fragment read of the next sub-step (NRD of them),
-        // while both last; then the remaining MFMAs (or reads).
-        auto interleave = [&](auto NRD_) {
-            constexpr int NRD = decltype(NRD_)::value;
-            constexpr int NPAIR = NMF < NRD ? NMF : NRD;
-            if constexpr (NMF > 0) {
+        auto row_mfmas = [&](int i, int hf) {
 #pragma unroll
-                for (int t = 0; t < NPAIR; ++t) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one DS read
-                }
-                if constexpr (NMF > NPAIR) __builtin_amdgcn_sched_group_barrier(0x008, NMF - NPAIR, 0);
-                if constexpr (NRD > NPAIR) __builtin_amdgcn_sched_group_barrier(0x100, NRD - NPAIR, 0);
-            }
+            for (int j = 0; j < JH; ++j)
+                acc[i][hf * JH + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[hf][j], fa[i], acc[i][hf * JH + j], 0, 0, 0);
         };
-        read_frags(ic<0>{}, 0, fa[0], fb[0]);
+#pragma unroll
+        for (int i = 0; i < NF; ++i) read_a(ic<0>{}, i);
+        read_b(ic<0>{}, 0);
         auto stage = [&](auto J_, int st) {
             constexpr int J = decltype(J_)::value;
             using Jn = ic<(J + 1) % NS>;       // slot of stage s+1
             using Jl = ic<(J + NS - 1) % NS>;  // slot of stage s-1 = s+NS-1
             const int kl = min(st + NS - 1, KT - 1);
-            read_frags(J_, 1, fa[1], fb[1]);
+            read_b(J_, 1);
 #pragma unroll
             for (int t = 0; t < NL0; ++t) dma(Jl{}, kl, t);
-            mfmas(fa[0], fb[0]);
-            interleave(ic<(NV > 0) ? (WF8 ? NV : NV + JN) : 0>{});
+            widen(0);
+#pragma unroll
+            for (int i = 0; i < NF; ++i) row_mfmas(i, 0);
+            // a row's MFMAs, then one fragment read, while there are reads
+#pragma unroll
+            for (int t = 0; t < NF; ++t) {
+                __builtin_amdgcn_sched_group_barrier(0x008, JH, 0);
+                if (t < JH) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
             wait_vmcnt<AFTER>();
             barrier_lds();
-            read_frags(Jn{}, 0, fa[0], fb[0]);
+            read_b(Jn{}, 0);
 #pragma unroll
             for (int t = NL0; t < NL; ++t) dma(Jl{}, kl, t);
-            mfmas(fa[1], fb[1]);
-            interleave(ic<(NV > 0) ? NV + JN : 0>{});
+            widen(1);
+#pragma unroll
+            for (int i = 0; i < NF; ++i) {
+                row_mfmas(i, 1);
+                read_a(Jn{}, i);
+            }
+#pragma unroll
+            for (int t = 0; t < NF; ++t) {
+                if (t < JH) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, JH, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
         };
         MOE_STAGE_LOOP(NS, KT)
     };
-    const int nv = min(IM, (max(0, jb.rows - (PAIR ? 0 : wm * WM)) + 31) >> 5);  // wave-uniform
-    if (nv == IM) run(ic<IM>{});
-    else if (nv == 0) run(ic<0>{});
+    const int nv = (jb.rows > wm * 32 ? 1 : 0) + (jb.rows > (wm + MW) * 32 ? 1 : 0);  // wave-uniform
+    if (nv == 2) run(ic<2>{});
     else if (nv == 1) run(ic<1>{});
-    else if constexpr (IM > 2) {
-        if (nv == 2) run(ic<2>{});
-        else run(ic<3>{});
-    }
+    else run(ic<0>{});
     wait_vmcnt<0>();  // no load may still be writing LDS when the workgroup ends
     if constexpr (SPLIT) {
         // a K range of a split up-GEMM tile: its partial sums, for fold_up_kernel
-        store_partial<IM, JN>(g, jb, acc);
+        store_partial<BM, IM, JN>(g, jb, acc);
         return;
     }
     tile_epilogue<MODE, BM, ACT, WF8, OCC, PAIR>(g, jb, acc, ring_);
 }
 
 // Partial sums of one K range of a split up-GEMM tile, in fragment order:
-// block (split_j S + ks) of split_ws holds BM x 256 floats, thread t's
-// accumulator values (i, j, q) at float (((i JN + j) 4 + q / 4) 256 + t) 4 +
-// q % 4, so each wave writes and reads whole 1 KB runs.
-template <int IM, int JN>
-__device__ __forceinline__ void store_partial(const GemmArgs &g, const TileJob &jb, const f32x16_t (&acc)[IM][JN]) {
-    float *ws = g.split_ws + ((long long)jb.split_j * jb.nks + jb.ks) * (IM * JN * 16 * 256) + threadIdx.x * 4;
+// block (split_j S + ks) of split_ws holds BM x 256 floats, thread t's (of NT)
+// accumulator block (i, j) at float ((i JN + j) NT + t) 4, so each wave writes
+// and reads whole 1 KB runs.
+template <int BM, int IM, int JN>
+__device__ __forceinline__ void store_partial(const GemmArgs &g, const TileJob &jb, const f32x4_t (&acc)[IM][JN]) {
+    float *ws = g.split_ws + ((long long)jb.split_j * jb.nks + jb.ks) * BM * 256 + threadIdx.x * 4;
 #pragma unroll
     for (int i = 0; i < IM; ++i)
 #pragma unroll
         for (int j = 0; j < JN; ++j)
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4)
-                *(float4 *)(ws + ((i * JN + j) * 4 + q4) * 1024) =
-                    make_float4(acc[i][j][4 * q4], acc[i][j][4 * q4 + 1], acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
+            *(float4 *)(ws + (i * JN + j) * 4 * gemm_threads(BM)) =
+                make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
 }
 
 // The epilogue of a tile whose accumulators are complete.  bf16 outputs are
 // staged in the (idle) LDS ring, rows of CW bytes: h as its tile image; y
 // rows when y is bf16, the tile not split and N, ldc multiples of 8 (whole
-// 16-byte chunks).  A paired item stages the rows of its n-tile nt + wm at
-// rows wm BM / 2 ..
+// 16-byte chunks).  A paired item stages the rows of its n-tile nt + pt at
+// rows pt BM / 2 ..
 template <int MODE, int BM, int ACT, int WF8, int OCC, bool PAIR, int IM, int JN>
-__device__ __forceinline__ void tile_epilogue(const GemmArgs &g, const TileJob &jb, const f32x16_t (&acc)[IM][JN],
+__device__ __forceinline__ void tile_epilogue(const GemmArgs &g, const TileJob &jb, const f32x4_t (&acc)[IM][JN],
                                               uint8_t *ring_) {
     constexpr int NB = (MODE == MODE_GATED_UP) ? 2 : 1;
     constexpr int BMA = PAIR ? BM / 2 : BM;
-    constexpr int WM = BM / 2;
+    constexpr int MW = BMA / 64;
     constexpr int WN = 128;
     constexpr int RING = RingShape<BM, WF8, OCC>::BYTES;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = w & 1, wn = w >> 1;
+    const WavePlace wp = wave_place<BM, PAIR>(w);
+    const int wm = wp.wm, wn = wp.wn;
     constexpr int CW = (MODE == MODE_GATED_UP ? 128 : 256) * 2;  // output bytes per tile row
     constexpr int CH = CW / 16;
     static_assert(BM * CW <= RING, "LDS staging of the output tile");
@@ -859,25 +867,25 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &g, const TileJob &
         __syncthreads();  // every wave's ring reads and loads are done
         if constexpr (PAIR) {
             TileJob jw = jb;
-            jw.n0 = jb.n0 + wm * (NB == 2 ? 128 : 256);
+            jw.n0 = jb.n0 + wp.pt * (NB == 2 ? 128 : 256);
             using SP = StagePut<CH, decltype(row_addr)>;
-            store_tile<MODE, ACT, IM, JN, WN, WF8>(g, jw, acc, 0, wn, lane,
-                                                   RowOffsetPut<SP>{SP{row_addr}, wm * BMA});
+            store_tile<MODE, BM, ACT, MW, IM, JN, WN, WF8>(g, jw, acc, wm, wn, lane,
+                                                           RowOffsetPut<SP>{SP{row_addr}, wp.pt * BMA});
             __syncthreads();
             store_staged_pair<MODE, BM, CH>(g, jb, row_addr);
         } else {
-            store_tile<MODE, ACT, IM, JN, WN, WF8>(g, jb, acc, wm * WM, wn, lane,
-                                                   StagePut<CH, decltype(row_addr)>{row_addr});
+            store_tile<MODE, BM, ACT, MW, IM, JN, WN, WF8>(g, jb, acc, wm, wn, lane,
+                                                           StagePut<CH, decltype(row_addr)>{row_addr});
             __syncthreads();
             store_staged<MODE, BM, CH>(g, jb, row_addr);
         }
     } else if constexpr (MODE == MODE_DOWN) {
-        store_tile<MODE, ACT, IM, JN, WN, WF8>(g, jb, acc, wm * WM, wn, lane, DirectPut{g, jb});
+        store_tile<MODE, BM, ACT, MW, IM, JN, WN, WF8>(g, jb, acc, wm, wn, lane, DirectPut{g, jb});
     }
 }
 
 template <int MODE, int BM, int ACT, int WF8, int OCC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void grouped_gemm_bf16_kernel(
+__global__ __launch_bounds__(gemm_threads(BM)) __attribute__((amdgpu_waves_per_eu(2, 2))) void grouped_gemm_bf16_kernel(
     GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) uint8_t ring[RingShape<BM, WF8, OCC>::BYTES];
     TileJob jb;
@@ -906,9 +914,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 // ============================================================================
 // Fold of the up GEMM's split tiles (tail_split).  Work unit (j, i, mo) of a
 // split tile j: for every thread t of the tile's workgroup, its accumulator
-// blocks [i][2 mo], [i][2 mo + 1] (a 32-row block and 64 B-tile columns of its
-// wave: one W1 | W3 column pair of the gated mode, two column blocks
-// otherwise).  Thread t of a fold workgroup sums those blocks' K-range
+// blocks [2 i .. 2 i + 1][4 mo .. 4 mo + 3] (32 rows and 64 B-tile columns of
+// its wave: the W1 and W3 rows of 32 h columns in the gated mode).  Thread t of a fold workgroup sums those blocks' K-range
 // partials in range order (a fixed order, so results are deterministic) and
 // runs the tile's epilogue on them (fp8 scales, bias, activation, dropout),
 // storing its bf16 h values straight into the h tile image (ImagePut).
@@ -931,27 +938,30 @@ struct ImagePut {
 template <int MODE, int BM, int ACT, int WF8>
 __global__ __launch_bounds__(256) void fold_up_kernel(GemmArgs g) {
     constexpr int NB = (MODE == MODE_GATED_UP) ? 2 : 1;
-    constexpr int IM = BM / 64, JN = 4;  // the accumulator blocks of tile_body's waves
+    constexpr int JN = 8, NT = gemm_threads(BM);  // 16-column blocks and threads of tile_body
     constexpr int WN = 128;
-    constexpr long long BLK = IM * JN * 16 * 256;  // floats per partial block
+    constexpr long long BLK = (long long)BM * 256;  // floats per partial block
     const int W = work_items(g);
     const TailSplit ts = tail_split(W, g.ncu, g.ksplit, g.K / 32);
     if (ts.S < 2) return;
-    const int nunit = (W - ts.nfull) * IM * 2;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, wm = w & 1, wn = w >> 1;
+    constexpr int UT = 4 * (NT / 256);  // units per tile: 32-row block, 64 columns, 256 threads
+    const int nunit = (W - ts.nfull) * UT;
     const long long KTT = g.ldc / 32;  // h: K of the down GEMM = ldc
     for (int u = blockIdx.x; u < nunit; u += gridDim.x) {
-        const int j = u / (IM * 2), i = (u >> 1) % IM, mo = u & 1;
+        const int j = u / UT, i = u & 1, mo = (u >> 1) & 1;
+        const int t = ((u / 4) % (NT / 256)) * 256 + threadIdx.x, lane = t & 63;
+        const int w = __builtin_amdgcn_readfirstlane(t >> 6);
         // every partial of the unit in flight before the work-item decode
         // (a chain of dependent loads) runs
-        const float *ws = g.split_ws + (long long)j * ts.S * BLK + ((i * JN + 2 * mo) * 4) * 1024 + t * 4;
+        const float *ws = g.split_ws + (long long)j * ts.S * BLK + (2 * i * JN + 4 * mo) * 4 * NT + t * 4;
+        auto blk = [](int q) { return ((q >> 2) * JN + (q & 3)) * 4 * NT; };  // block q = 4 row + column
         constexpr int RB = 4;  // ranges whose loads are in flight together
         float4 p[RB][8], a[8];
 #pragma unroll
         for (int r = 0; r < RB; ++r)
 #pragma unroll
             for (int q = 0; q < 8; ++q)
-                if (r < ts.S) p[r][q] = *(const float4 *)(ws + r * BLK + q * 1024);
+                if (r < ts.S) p[r][q] = *(const float4 *)(ws + r * BLK + blk(q));
         TileJob jb;
         decode_item<BM, NB>(g, ts.nfull + j, jb);
         jb.ks = 0;
@@ -968,7 +978,7 @@ __global__ __launch_bounds__(256) void fold_up_kernel(GemmArgs g) {
                 for (int r = 0; r < RB; ++r)
 #pragma unroll
                     for (int q = 0; q < 8; ++q)
-                        if (r0 + r < ts.S) p[r][q] = *(const float4 *)(ws + (r0 + r) * BLK + q * 1024);
+                        if (r0 + r < ts.S) p[r][q] = *(const float4 *)(ws + (r0 + r) * BLK + blk(q));
             }
 #pragma unroll
             for (int r = (r0 == 0 ? 1 : 0); r < RB; ++r)
@@ -979,28 +989,25 @@ __global__ __launch_bounds__(256) void fold_up_kernel(GemmArgs g) {
                         a[q].z = a[q].z + p[r][q].z; a[q].w = a[q].w + p[r][q].w;
                     }
         }
-        f32x16_t acc[1][2];
+        f32x4_t acc[2][4];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            acc[0][q >> 2][4 * (q & 3)] = a[q].x;
-            acc[0][q >> 2][4 * (q & 3) + 1] = a[q].y;
-            acc[0][q >> 2][4 * (q & 3) + 2] = a[q].z;
-            acc[0][q >> 2][4 * (q & 3) + 3] = a[q].w;
-        }
+        for (int q = 0; q < 8; ++q) acc[q >> 2][q & 3] = f32x4_t{a[q].x, a[q].y, a[q].z, a[q].w};
         // the columns of these blocks: gated, h columns wn WN / 2 + 32 mo ..;
-        // otherwise B-tile columns wn WN + 64 mo ..; a paired item's wave wm
-        // holds n-tile nt + wm over the item's rows
+        // otherwise B-tile columns wn WN + 64 mo ..; a paired item's waves hold
+        // n-tile nt + pt over the item's rows
         TileJob jw = jb;
-        int row0;
+        int blk32;  // the unit's 32 rows
         if (jb.pair) {
-            jw.n0 += wm * (NB == 2 ? 128 : 256);
-            row0 = i * 32;
+            const WavePlace wp = wave_place<BM, true>(w);
+            jw.n0 += wp.pt * (NB == 2 ? 128 : 256) + ((NB == 2) ? wp.wn * (WN / 2) + 32 * mo : wp.wn * WN + 64 * mo);
+            blk32 = wp.wm + 2 * i;
         } else {
-            row0 = wm * (BM / 2) + i * 32;
+            const WavePlace wp = wave_place<BM, false>(w);
+            jw.n0 += (NB == 2) ? wp.wn * (WN / 2) + 32 * mo : wp.wn * WN + 64 * mo;
+            blk32 = wp.wm + (BM / 64) * i;
         }
-        jw.n0 += (NB == 2) ? wn * (WN / 2) + 32 * mo : wn * WN + 64 * mo;
         ImagePut<BM> put{(uint8_t *)g.C + ((long long)jw.mt * KTT + jw.n0 / 32) * BM * 64};
-        store_tile<MODE, ACT, 1, 2, WN, WF8>(g, jw, acc, row0, 0, lane, put);
+        store_tile<MODE, BM, ACT, 0, 2, 4, WN, WF8>(g, jw, acc, blk32, 0, lane, put);
     }
 }
 
@@ -1152,7 +1159,7 @@ static hipError_t launch_bf16(const GemmArgs &g, hipStream_t s) {
     // 128-row tiles run two workgroups per CU (the down GEMM's tail split then
     // plans its last round over g.ncu = 2 slots per CU)
     constexpr int OCC = (BM == 128) ? 2 : 1;
-    hipLaunchKernelGGL((grouped_gemm_bf16_kernel<MODE, BM, ACT, WF8, OCC>), dim3((unsigned)total), dim3(256), 0, s, g);
+    hipLaunchKernelGGL((grouped_gemm_bf16_kernel<MODE, BM, ACT, WF8, OCC>), dim3((unsigned)total), dim3(gemm_threads(BM)), 0, s, g);
     hipError_t e = hipGetLastError();
     // the up GEMM's split tiles (256-row tiles only) are folded in work units
     // over g.ncu workgroups

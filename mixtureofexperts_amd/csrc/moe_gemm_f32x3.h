@@ -5,29 +5,31 @@
 // to nearest: |x1| <= 2^-9 |x|, |x2| <= 2^-17 |x|), and an fp32 product to
 // fp32 accuracy the sum of the six products of parts i + j <= 2: the three
 // left out are below 2^-25 of it, random in sign, under the rounding of the
-// fp32 sum.  Six v_mfma_f32_32x32x16_bf16 replace eight v_mfma_f32_32x32x2_f32
-// and take 192 cycles instead of 512; the running sums stay fp32 and take
-// 6 roundings per 16 K instead of 8.
+// fp32 sum.  Per 32 x 32 outputs and 16 K, six bf16 products take 192 cycles
+// of the matrix unit, eight v_mfma_f32_32x32x2_f32 512; the running sums stay
+// fp32 and take 6 roundings per 32 K instead of 16.
 //
 // What bounds it: the matrix unit's power at large sizes, per-tile latencies
 // (24 stages between prologue and epilogue) at small K.  Against
 // grouped_gemm_kernel (whole layer forward, 8 experts, top-2, 4096 tokens):
-// 4096 / 14336 gated 25.4 -> 14.6 ms (198 TFLOP/s of fp32 products), 768 / 3072
-// standard 746 -> 463 us, 1024 / 4096 gated 1861 -> 1081 us; error against 64
-// bits 2.8e-6 -> 2.4e-6, 1.13e-6 -> 0.99e-6, 1.44e-6 -> 1.24e-6.  Two 128 x 128
-// workgroups per CU instead of one kept the MFMAs busier (77 instead of 68 %
-// of cycles) at a lower clock (1.51 instead of 1.66 GHz) and took 4 % longer:
-// what counts is the work besides the MFMAs.  Splitting the last round's tiles
-// into K ranges gained nothing for the same reason (467 and 463 us).
-// Tile 128 rows x 256 weight rows (gated:
-// 128 of W1 and the same 128 of W3), 8 waves as 2 (rows) x 4 (columns), two
-// per SIMD, each 64 x 64.  A stage is 32 K: every thread loads 8 K values of
-// three rows (one of A, two of the weights) two stages ahead, splits them one
-// stage ahead and writes them to the other of two LDS buffers (72 KB each),
-// so the split's vector instructions, the LDS writes and the reads of the
-// next sub-step's fragments run between the MFMAs and there is one barrier
-// per stage (96 MFMAs per SIMD).  Splitting in the kernel repeats it for every tile that reads an
-// operand, but keeps weights, xp and h at 4 bytes in memory and in L2.
+// 4096 / 14336 gated 25.4 -> 14.2 ms, 768 / 3072 standard 746 -> 440 us, 1024 / 4096
+// gated 1861 -> 1040 us; error against 64 bits 2.8e-6 -> 2.4e-6, 1.13e-6 ->
+// 0.99e-6, 1.44e-6 -> 1.24e-6.  Two 128 x 128 workgroups per CU instead of one
+// kept the MFMAs busier (77 instead of 68 % of cycles) at a lower clock (1.51
+// instead of 1.66 GHz) and took 4 % longer: what counts is the work besides the
+// MFMAs, and the MFMA's own (16x16x32 5 % faster than 32x32x16).  Splitting the
+// last round's tiles into K ranges gained nothing for the same reason (467 and
+// 463 us).
+//
+// Tile 128 rows x 256 weight rows (gated: 128 of W1 and the same 128 of W3), 8
+// waves as 2 (rows) x 4 (columns), two per SIMD, each 64 x 64.  A stage is 32
+// K: every thread loads 8 K values of three rows (one of A, two of the
+// weights) two stages ahead, splits them one stage ahead and writes them to
+// the other of two LDS buffers (72 KB each), so the split's vector
+// instructions, the LDS writes and the reads of the next half's fragments run
+// between the MFMAs and there is one barrier per stage (192 MFMAs per SIMD).
+// Splitting in the kernel repeats it for every tile that reads an operand, but
+// keeps weights, xp and h at 4 bytes in memory and in L2.
 //
 // LDS rows are 64 B (32 bf16 of one part), 16-byte chunk c of row r at c ^
 // ((r >> 2) & 3), as in the bf16 kernel.
@@ -90,7 +92,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = w & 1, wn = w >> 1;
-    const int half = lane >> 5, r32 = lane & 31;
+    const int q4 = lane >> 4, r16 = lane & 15;
 
     // this thread's three rows: row tid / 4 of A, of the first and of the
     // second 128 weight rows; K values 8 (tid % 4) .. + 8 of each stage
@@ -115,31 +117,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int q = 0; q < 3; ++q) *(u32x4_t *)(lds + buf * STAGE + q * PART + i * 128 * 64 + wofs) = p[q];
     };
 
-    // fragments: A blocks of 32 rows wm + 2 i (so a tile of few rows is shared
-    // by both wave rows), weight blocks j of the wave's columns (gated: the W1
-    // and W3 rows of 32 h columns)
-    const int sw = (r32 >> 2) & 3;
-    const int afr = (wm * 32 + r32) * 64;
-    int bfr[2];
+    // fragments (16 rows x 32 K): A row blocks 2 i, 2 i + 1 of the 32 rows wm +
+    // 2 i (so a tile of few rows is shared by both wave rows), weight blocks j
+    // of the wave's columns (gated: W1 and W3 rows of 16 h columns in turn)
+    const int sw = (q4 ^ ((r16 >> 2) & 3)) << 4;
+    const int afr = (wm * 32 + r16) * 64 + sw;
+    const int bfr = (BM + wn * (NB == 2 ? 32 : 64) + r16) * 64 + sw;
+    f32x4_t acc[4][4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bfr[j] = (BM + (NB == 2 ? j * 128 + wn * 32 : wn * 64 + j * 32) + r32) * 64;
-    f32x16_t acc[2][2];
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     const int KTT = g.K / 32;
     const int kb = (ks * KTT) / S, ke = ((ks + 1) * KTT) / S;
     const int kl = ke - 1;  // the loads past the range repeat its last stage, into a buffer that nothing reads
 
-    // Stage s is in buffer (s - kb) % 2; its fragments of sub-step 0 are read
-    // in the second half of stage s - 1.  Per stage:
-    //   MFMAs of (s, 0) | reads of (s, 1)     | the weight rows of stage s + 1: split, written, loaded for s + 2
+    // Stage s is in buffer (s - kb) % 2.  Its MFMAs run in two halves of the
+    // wave's columns, rows in order; a row block's fragments are replaced by
+    // the next stage's once the second half is past it.  Per stage:
+    //   columns 0, 1 | reads of (s, columns 2, 3)        | the weight rows of stage s + 1: split, written, loaded for s + 2
     //   barrier: stage s + 1 is written, and nothing more is read from buffer s
-    //   MFMAs of (s, 1) | reads of (s + 1, 0) | the A row of stage s + 2: split, written, loaded for s + 3
+    //   columns 2, 3 | reads of (s + 1, rows, columns 0, 1) | the A row of stage s + 2: split, written, loaded for s + 3
     auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 #pragma unroll
     for (int i = 0; i < 3; ++i) load(i, kb);
@@ -153,58 +152,71 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
     auto run = [&](auto NV_) {
         constexpr int NV = decltype(NV_)::value;  // row blocks of this wave that hold rows of the tile
-        bf16x8_t fa[2][2][3], fb[2][2][3];
-        auto read = [&](int buf, int kk) {
-            if constexpr (NV > 0) {
-                const uint8_t *rb = lds + buf * STAGE + (((kk * 2 + half) ^ sw) << 4);
+        constexpr int NF = 2 * NV;
+        bf16x8_t fa[4][3], fb[2][2][3];
+        auto read_a = [&](int buf, int i) {
 #pragma unroll
-                for (int q = 0; q < 3; ++q) {
-#pragma unroll
-                    for (int i = 0; i < NV; ++i) fa[kk][i][q] = *(const bf16x8_t *)(rb + q * PART + afr + i * 64 * 64);
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) fb[kk][j][q] = *(const bf16x8_t *)(rb + q * PART + bfr[j]);
-                }
-            }
+            for (int q = 0; q < 3; ++q)
+                fa[i][q] = *(const bf16x8_t *)(lds + buf * STAGE + q * PART + afr + ((i >> 1) * 64 + (i & 1) * 16) * 64);
         };
-        auto mfmas = [&](int kk) {
+        auto read_b = [&](int buf, int hf) {
+            if constexpr (NV > 0)
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        fb[hf][j][q] = *(const bf16x8_t *)(lds + buf * STAGE + q * PART + bfr +
+                                                           (NB == 2 ? j * 128 + hf * 16 : (2 * hf + j) * 16) * 64);
+        };
+        auto row_mfmas = [&](int i, int hf) {
 #pragma unroll
             for (int t = 0; t < 6; ++t) {
                 constexpr int PA[6] = {0, 0, 1, 1, 0, 2}, PB[6] = {0, 1, 0, 1, 2, 0};
 #pragma unroll
-                for (int i = 0; i < NV; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][i][PA[t]], fb[kk][j][PB[t]], acc[i][j],
-                                                                            0, 0, 0);
+                for (int j = 0; j < 2; ++j)
+                    acc[i][2 * hf + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[hf][j][PB[t]], fa[i][PA[t]],
+                                                                                 acc[i][2 * hf + j], 0, 0, 0);
             }
         };
-        // after each MFMA: VA vector instructions of the split, then an LDS read or write
-        auto interleave = [&](auto VA_, auto NW_) {
-            constexpr int NM = 12 * NV, NR = 3 * (NV + 2), NW = decltype(NW_)::value;
+        // after each pair of MFMAs: VA vector instructions of the split, an LDS
+        // read, at the end the LDS writes
+        auto interleave = [&](auto VA_, auto NR_, auto NW_) {
+            constexpr int NM = 6 * NF, NR = decltype(NR_)::value, NW = decltype(NW_)::value;
 #pragma unroll
             for (int t = 0; t < NM; ++t) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, decltype(VA_)::value, 0);       // vector instructions
-                if (t < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);              // one LDS read
-                if (t >= NM - NW) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);        // one LDS write
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);                     // MFMAs
+                __builtin_amdgcn_sched_group_barrier(0x002, decltype(VA_)::value, 0);  // vector instructions
+                if (t < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);         // LDS read
+                if (t >= NM - NW) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // LDS write
             }
         };
-        read(0, 0);
+#pragma unroll
+        for (int i = 0; i < NF; ++i) read_a(0, i);
+        read_b(0, 0);
         for (int kt = kb; kt < ke; ++kt) {
             const int cur = (kt - kb) & 1;
-            read(cur, 1);
+            read_b(cur, 1);
             split_store(cur ^ 1, 1);
             split_store(cur ^ 1, 2);
             load(1, min(kt + 2, kl));
             load(2, min(kt + 2, kl));
-            mfmas(0);
-            if constexpr (NV > 0) interleave(std::integral_constant<int, 10 / NV>{}, std::integral_constant<int, 6>{});
+#pragma unroll
+            for (int i = 0; i < NF; ++i) row_mfmas(i, 0);
+            if constexpr (NV > 0)
+                interleave(std::integral_constant<int, 10 / NV>{}, std::integral_constant<int, 6>{},
+                           std::integral_constant<int, 6>{});
             barrier();
-            read(cur ^ 1, 0);
+            read_b(cur ^ 1, 0);
             split_store(cur, 0);
             load(0, min(kt + 3, kl));
-            mfmas(1);
-            if constexpr (NV > 0) interleave(std::integral_constant<int, 6 / NV>{}, std::integral_constant<int, 3>{});
+#pragma unroll
+            for (int i = 0; i < NF; ++i) {
+                row_mfmas(i, 1);
+                read_a(cur ^ 1, i);
+            }
+            if constexpr (NV > 0)
+                interleave(std::integral_constant<int, 6 / NV>{}, std::integral_constant<int, 6 * NF>{},
+                           std::integral_constant<int, 3>{});
         }
     };
     const int nv = (rows > wm * 32 ? 1 : 0) + (rows > wm * 32 + 64 ? 1 : 0);  // wave-uniform
@@ -212,69 +224,77 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     else if (nv == 1) run(std::integral_constant<int, 1>{});
     else run(std::integral_constant<int, 0>{});
 
-    // ---- epilogue: lane holds column r32 of each 32x32 block, rows
-    // 8*(q/4) + 4*half + q%4.
+    // ---- epilogue: lane holds row r16 of each row block and the columns 4 q4
+    // .. + 3 of each weight block.
     const long long sofs = (long long)e * g.s_stride;
-    // row of the tile of element q of row block i; output column of column block j
-    auto row_of = [&](int i, int q) { return (wm + 2 * i) * 32 + 8 * (q >> 2) + 4 * half + (q & 3); };
-    auto col_of = [&](int j) { return (NB == 2 ? wn * 32 : wn * 64 + j * 32) + r32; };
+    auto row_of = [&](int i) { return (wm + 2 * (i >> 1)) * 32 + (i & 1) * 16 + r16; };
+    // first column of the lane in column block j (gated: of h, from blocks 2 j and 2 j + 1)
+    auto col_of = [&](int j) { return wn * (NB == 2 ? 32 : 64) + j * 16 + 4 * q4; };
+    constexpr int NJ = 4 / NB;
     float *ws = S > 1 ? g.split_ws + ((long long)(mt * g.n_tiles + nt) * S + ks) * (BM * BR) : nullptr;
-    unsigned long long bad = 0;  // outputs with a sum that is not finite: bit (j 2 + i) 16 + q
-    // the activation is picked once per tile, and a block's 16 outputs are
-    // computed side by side before their stores (picked per output, the GELU
-    // epilogue of a 24-stage tile took as long as its MFMAs)
-    auto block = [&](int i, int j, auto &&out) {
-        const int nl = col_of(j);
-        if (n0 + nl >= g.N) return;
-        float v[16];
-        const float bias = (MODE != MODE_GATED_UP && g.bias) ? g.bias[sofs + n0 + nl] : 0.0f;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const float v0 = acc[i][j][q], v1 = acc[i][1][q];
-            const bool fin = __builtin_isfinite(v0) && (NB == 1 || __builtin_isfinite(v1));
-            if (!fin && row_of(i, q) < rows) bad |= 1ull << ((j * 2 + i) * 16 + q);
-            v[q] = out(arow0 + row_of(i, q), n0 + nl, bias, v0, v1);
-        }
-        float *c = (float *)g.C + arow0 * g.ldc + n0 + nl;
-#pragma unroll
-        for (int q = 0; q < 16; ++q)
-            if (row_of(i, q) < rows) c[(long long)row_of(i, q) * g.ldc] = v[q];
+    unsigned long long bad = 0;  // outputs with a sum that is not finite: bit (j 4 + i) 4 + c
+    auto check = [&](int j, int i, int c, float v0, float v1) {
+        const bool fin = __builtin_isfinite(v0) && (NB == 1 || __builtin_isfinite(v1));
+        if (!fin && row_of(i) < rows) bad |= 1ull << ((j * 4 + i) * 4 + c);
     };
+    const bool vec4 = (g.ldc & 3) == 0;
+    // the activation is picked once per tile (picked per output, it was a
+    // branch and a wait for each of a lane's 64 outputs)
     auto tile = [&](auto &&out) {
 #pragma unroll
-        for (int j = 0; j < 2 / NB; ++j)
+        for (int j = 0; j < NJ; ++j) {
+            const int n = n0 + col_of(j);
+            float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (MODE != MODE_GATED_UP && g.bias)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) block(i, j, out);
-    };
-    auto finish = [&](auto ACT_, long long row, int n, float bias, float v0, float v1) -> float {
-        constexpr int ACT = decltype(ACT_)::value;
-        if constexpr (MODE == MODE_GATED_UP) return act_apply(ACT, v0) * v1;
-        else if constexpr (MODE == MODE_STD_UP) return dropout_h(g, row, n, act_apply(ACT, v0 + bias));
-        else return v0 + bias;
+                for (int c = 0; c < 4; ++c)
+                    if (n + c < g.N) bias[c] = g.bias[sofs + n + c];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                f32x4_t v;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float v0 = acc[i][NB == 2 ? 2 * j : j][c], v1 = acc[i][NB == 2 ? 2 * j + 1 : j][c];
+                    check(j, i, c, v0, v1);
+                    v[c] = out(arow0 + row_of(i), n + c, bias[c], v0, v1);
+                }
+                if (row_of(i) >= rows) continue;
+                float *p = (float *)g.C + (arow0 + row_of(i)) * g.ldc + n;
+                if (vec4 && n + 3 < g.N) {
+                    *(f32x4_t *)p = v;
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (n + c < g.N) p[c] = v[c];
+                }
+            }
+        }
     };
     auto tile_act = [&](auto ACT_) {
-        if (MODE == MODE_STD_UP && g.drop_p > 0.0f) {
-            tile([&](long long row, int n, float bias, float v0, float v1) { return finish(ACT_, row, n, bias, v0, v1); });
+        constexpr int ACT = decltype(ACT_)::value;
+        if constexpr (MODE == MODE_GATED_UP) {
+            tile([](long long, int, float, float v0, float v1) { return act_apply(ACT, v0) * v1; });
+        } else if constexpr (MODE == MODE_STD_UP) {
+            if (g.drop_p > 0.0f)
+                tile([&](long long row, int n, float bias, float v0, float) {
+                    return dropout_h(g, row, n, act_apply(ACT, v0 + bias));
+                });
+            else tile([](long long, int, float bias, float v0, float) { return act_apply(ACT, v0 + bias); });
         } else {
-            tile([&](long long, int, float bias, float v0, float v1) -> float {
-                if constexpr (MODE == MODE_STD_UP) return act_apply(decltype(ACT_)::value, v0 + bias);
-                else return finish(ACT_, 0, 0, bias, v0, v1);
-            });
+            tile([](long long, int, float bias, float v0, float) { return v0 + bias; });
         }
     };
     if (S > 1) {  // a K range: its raw sums, [b][row][column] of split_ws block (tile, ks)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 4; ++i) {
+                if (row_of(i) >= rows) continue;
 #pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    const int ml = row_of(i, q);
-                    if (ml >= rows) continue;
-                    const int jo = NB == 2 ? 0 : j;
-                    if (!__builtin_isfinite(acc[i][j][q])) bad |= 1ull << ((jo * 2 + i) * 16 + q);
-                    ws[((NB == 2 ? j : 0) * BM + ml) * BN + col_of(jo)] = acc[i][j][q];
-                }
+                for (int b = 0; b < NB; ++b) *(f32x4_t *)(ws + (b * BM + row_of(i)) * BN + col_of(j)) = acc[i][NB * j + b];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) check(j, i, c, acc[i][NB * j][c], acc[i][NB * j + NB - 1][c]);
+            }
     } else if constexpr (MODE == MODE_DOWN) {
         tile_act(std::integral_constant<int, MOE_ACT_IDENTITY>{});
     } else {
@@ -288,7 +308,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     while (bad) {  // once more from the fp32 rows, one K value after the other; NaN ends a sum
         const int u = __builtin_ctzll(bad);
         bad &= bad - 1;
-        const int ml = row_of((u >> 4) & 1, u & 15), nl = col_of(u >> 5), n = n0 + nl;
+        const int ml = row_of((u >> 2) & 3), nl = col_of(u >> 4) + (u & 3), n = n0 + nl;
         const float *ar = A + (arow0 + ml) * g.lda, *w0 = B0 + (long long)nl * g.ldb, *w1 = B1 + (long long)nl * g.ldb;
         float v0 = 0.0f, v1 = 0.0f;
         for (int k = kb * 32; k < ke * 32 && v0 == v0; ++k) v0 = fmaf(ar[k], w0[k], v0);
@@ -299,6 +319,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             if (NB == 2) ws[(BM + ml) * BN + nl] = v1;
             continue;
         }
+        if (n >= g.N) continue;
         float v = v0 + ((MODE != MODE_GATED_UP && g.bias) ? g.bias[sofs + n] : 0.0f);
         if (MODE != MODE_DOWN) v = act_apply(g.act, v);
         if (MODE == MODE_GATED_UP) v = v * v1;
