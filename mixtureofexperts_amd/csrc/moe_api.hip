@@ -98,7 +98,7 @@ struct moe_handle {
     long long ent_max = 0;
     long long act_rows = 0;     // rows of xp and h (bf16 kernel: max_tiles * bm, tile images)
     int ld_y = 0;               // row stride of y (elements)
-    int bm = kGemmBM;           // GEMM tile rows of this handle's kernels (scan granule)
+    int bm = kGemmBM;           // GEMM tile rows of the current call's kernels (scan granule)
     bool bf16_gemm = false;     // bf16 weights and activations: the LDS-DMA MFMA kernel
     float *logits = nullptr, *probs = nullptr, *gates = nullptr, *gate_sorted = nullptr;
     float *lse = nullptr;          // [T] per-token logsumexp of the last routing call
@@ -351,13 +351,14 @@ __global__ void fp8_rows_kernel(const uint8_t *src, int layout, int N, int K, in
 // rows [n][D] of fp32/bf16 -> compute type with row stride ld (pads
 // untouched); bm > 0: bf16 rows of one expert starting at M tile 0 of the
 // bf16 kernel's A tile image (row r: row r mod bm of tile r / bm, ld / 32 K
-// stages of 64 B, chunk q of a stage at q ^ ((row >> 2) & 3))
+// stages of 64 B, chunk q of a stage at q ^ ((row >> 2) & 3)), pads zeroed
 __global__ void convert_rows_kernel(const void *src, int src_bf16, int n, int D, int ct, void *dst, int ld, int bm) {
-    const long long total = (long long)n * D;
+    const int W = bm > 0 ? ld : D;
+    const long long total = (long long)n * W;
     for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < total;
          t += (long long)gridDim.x * blockDim.x) {
-        const long long r = t / D, c = t % D;
-        const float v = src_bf16 ? bf16_to_f32(((const uint16_t *)src)[t]) : ((const float *)src)[t];
+        const long long r = t / W, c = t % W, i = r * D + c;
+        const float v = c >= D ? 0.0f : (src_bf16 ? bf16_to_f32(((const uint16_t *)src)[i]) : ((const float *)src)[i]);
         if (ct == CT_F32) {
             ((float *)dst)[r * ld + c] = v;
         } else if (bm > 0) {
@@ -561,6 +562,33 @@ static int check_ready(moe_handle *h) {
     return MOE_OK;
 }
 
+// n-tiles of the up GEMM
+static int up_ntiles(const moe_handle *h) {
+    return h->bf16_gemm ? h->H_pad / (h->gated ? 128 : 256) : h->H_pad / kGemmBN;
+}
+// Tile rows of a call of `rows` expert rows on the bf16 kernel: 256 with bf16
+// weights where the experts average 192 rows or more and the up GEMM has four
+// rounds of work items or more (then weights are read half as often and a
+// partial tile is a small part of the work), else 128 (two workgroups per CU,
+// finer last rounds).  Whole layer, 128 / 256, us: 8 experts of 4096 / 14336, 256
+// rows 865 / 798, 1024 rows 2788 / 2487; 64 of 2048 / 1408, 96 rows 262 / 302, 192
+// rows 351 / 320, 768 rows 972 / 899; 128 standard ones of 768 / 3072, 128 rows
+// 517 / 531, 384 rows 985 / 962; 16 of 1024 / 2048 (2 to 3 rounds), 256 rows 105 /
+// 115, 512 rows 150 / 151.  fp8 weights stay on 128 (66 of 2048 / 1408, 8192
+// tokens 1082 / 1193; 8 of 4096 / 14336, 8192 tokens 4283 / 4616).
+static int tile_rows(const moe_handle *h, long long rows) {
+    const long long items = (rows / 256 + h->E) * up_ntiles(h);
+    return (h->bf16_gemm && h->wt == WT_BF16 && rows >= 192LL * h->E && items >= 4LL * h->ncu) ? 256 : kGemmBM;
+}
+
+// Expert rows of a call of T tokens, at most.
+static long long call_rows(const moe_handle *h, int T) {
+    long long rows = (long long)T * h->kc;
+    if (h->cfg.gate_kind == MOE_GATE_EXPERT_CHOICE && !h->given)
+        rows = std::min(rows, (long long)T * h->lsh + (long long)h->Er * std::min(T, h->kl));
+    return std::min(rows, (long long)h->rows_max);
+}
+
 static int m_tiles_for(const moe_handle *h, int T) {
     long long mt = (long long)T * h->kc / h->bm + h->E;
     if (mt > h->max_tiles) mt = h->max_tiles;
@@ -598,10 +626,6 @@ static int run_permute(moe_handle *h, const void *x_dev, int x_bf16, int T, int 
 // over them): 128-row tiles run two workgroups per CU.
 static int gemm_slots(const moe_handle *h) { return h->bm == 128 ? 2 * h->ncu : h->ncu; }
 
-// n-tiles of the up GEMM
-static int up_ntiles(const moe_handle *h) {
-    return h->bf16_gemm ? h->H_pad / (h->gated ? 128 : 256) : h->H_pad / kGemmBN;
-}
 // The bf16 up GEMM on 256-row tiles with an even n-tile count pairs an
 // expert's last M tile of at most 128 rows with two n-tiles (item_start).
 static bool up_pairs(const moe_handle *h) { return h->bf16_gemm && h->bm == 256 && up_ntiles(h) % 2 == 0; }
@@ -619,6 +643,7 @@ static int run_routing(moe_handle *h, const void *x_dev, int x_bf16, int T, int 
         ++h->aux_counter;
         aux_update = h->aux_counter % h->aux_update_freq == 0;
     }
+    h->bm = tile_rows(h, call_rows(h, T));
     RtArgs A{};
     RouteArgs &ra = A.r;
     if (compute_logits) {
@@ -963,16 +988,13 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
         h->rows_max = (int)std::min<long long>(h->rows_max, (long long)h->T_max * h->lsh + (long long)h->Er * cmax);
     }
     h->bf16_gemm = h->ct == CT_BF16 && (h->wt == WT_BF16 || h->wt == WT_FP8);
-    // 256-row tiles for a few large experts (at most 16, averaging at least 384
-    // rows at max_tokens); 128-row tiles, two workgroups per CU, for many or
-    // small ones (fine-grained MoE layers: skewed counts, short K), and for
-    // standard experts with fp8 weights (on 256-row tiles their up GEMM's
-    // accumulators, fp8 stage bytes and epilogue scales exceed the registers)
-    const bool fp8_std = h->wt == WT_FP8 && !h->gated;
-    h->bm = (h->bf16_gemm && !fp8_std && h->E <= 16 && (long long)h->rows_max >= 384LL * h->E) ? 256 : kGemmBM;
-    h->max_tiles = h->rows_max / h->bm + h->E + 1;
-    // bf16 kernel: xp and h are A tile images of up to max_tiles M tiles
-    h->act_rows = h->bf16_gemm ? (long long)h->max_tiles * h->bm : h->rows_max;
+    // M tiles of the calls: at most rows_max / bm + E, bm = 128 or 256 by the
+    // call's rows (tile_rows)
+    h->max_tiles = h->rows_max / kGemmBM + h->E + 1;
+    // bf16 kernel: xp and h are A tile images of up to that many M tiles
+    h->act_rows = h->bf16_gemm ? (long long)h->max_tiles * kGemmBM : h->rows_max;
+    if (tile_rows(h, h->rows_max) == 256)
+        h->act_rows = std::max(h->act_rows, (long long)(h->rows_max / 256 + h->E + 1) * 256);
     if (h->bf16_gemm) {
         A(&h->w1t, wsz * (size_t)h->E * h->w1_stride);
         if (h->gated) A(&h->w3t, wsz * (size_t)h->E * h->w1_stride);
@@ -1013,11 +1035,11 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
     // spread over the HBM channels
     h->ld_y = h->bf16_gemm ? (int)round_up(h->Dout, 64) + 64 : h->Dout;
     A((void **)&h->y, sizeof(float) * (size_t)h->rows_max * h->ld_y);
-    // tail split: at most gemm_slots partial blocks of BM x 256 floats
-    // (rem * S <= slots) for either GEMM; the fp32 kernels' K ranges: about two
+    // tail split: at most gemm_slots partial blocks of BM x 256 floats (rem * S
+    // <= slots; 2 ncu of 128 rows or ncu of 256) for either GEMM; the fp32 kernels' K ranges: about two
     // workgroups per CU of 128 x 128 floats, of 128 x 256 where the handle's
     // batches reach the f32x3 kernel
-    h->split_cap = h->bf16_gemm ? (long long)gemm_slots(h) * h->bm * 256
+    h->split_cap = h->bf16_gemm ? (long long)h->ncu * 256 * 256
                                 : 2LL * h->ncu * kGemmBM * kGemmBN * (f32x3_rows(h->max_tiles - 1, h->E) ? 2 : 1);
     A((void **)&h->split_ws, sizeof(float) * (size_t)h->split_cap);
     if (r != MOE_OK) return cleanup(r);
@@ -1565,6 +1587,7 @@ int moe_expert_forward(moe_handle *h, int32_t expert, const float *x, int32_t n,
     std::vector<int> cnt(h->E, 0), off(h->E + 1, 0);
     cnt[expert] = n;
     for (int e = 0; e < h->E; ++e) off[e + 1] = off[e] + cnt[e];
+    h->bm = tile_rows(h, std::min((long long)n * h->E, (long long)h->rows_max));  // one expert takes all rows
     const int nt = (n + h->bm - 1) / h->bm;
     std::vector<int2> tl(nt);
     for (int i = 0; i < nt; ++i) tl[i] = make_int2(expert, i * h->bm);

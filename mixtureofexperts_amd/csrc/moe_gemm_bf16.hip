@@ -628,7 +628,7 @@ struct RowOffsetPut {
 template <int BM, int WF8, int OCC>
 struct RingShape {
     static constexpr int STAGE = BM * 64 + 256 * (WF8 ? 32 : 64);
-    static constexpr int NS = (OCC == 2) ? (WF8 ? 4 : 3) : ((BM == 256 && !WF8) ? 4 : 6);
+    static constexpr int NS = (OCC == 2) ? (WF8 ? 4 : 3) : 4;
     static constexpr int BYTES = NS * STAGE;
 };
 
@@ -1192,6 +1192,7 @@ hipError_t launch_grouped_gemm_bf16(int mode, int bm, int wfp8, const GemmArgs &
     if (g.ksplit < 1 || (g.ksplit > 1 && (!g.split_ws || g.ncu < 1))) return hipErrorInvalidValue;
     if (g.ksplit > 1 && mode != MODE_DOWN && bm != 256) return hipErrorInvalidValue;
     if (wfp8 && (!g.s0 || (mode == MODE_GATED_UP && !g.s1))) return hipErrorInvalidValue;
+    // (fp8 weights: 128-row tiles only)
 #define MOE_BF16_CASE(M, B, F) \
     if (mode == M && bm == B && (wfp8 != 0) == (F != 0)) return launch_bf16_act<M, B, F>(g, s);
     MOE_BF16_CASE(MODE_GATED_UP, 256, 0)
@@ -1200,8 +1201,6 @@ hipError_t launch_grouped_gemm_bf16(int mode, int bm, int wfp8, const GemmArgs &
     MOE_BF16_CASE(MODE_GATED_UP, 128, 0)
     MOE_BF16_CASE(MODE_STD_UP, 128, 0)
     MOE_BF16_CASE(MODE_DOWN, 128, 0)
-    MOE_BF16_CASE(MODE_GATED_UP, 256, 1)
-    MOE_BF16_CASE(MODE_DOWN, 256, 1)  // (standard experts with fp8 weights take 128-row tiles)
     MOE_BF16_CASE(MODE_GATED_UP, 128, 1)
     MOE_BF16_CASE(MODE_STD_UP, 128, 1)
     MOE_BF16_CASE(MODE_DOWN, 128, 1)

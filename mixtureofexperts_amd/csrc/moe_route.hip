@@ -15,6 +15,8 @@
 #include <climits>
 #include <mutex>
 
+#include <type_traits>
+
 #include "moe_internal.h"
 
 namespace moe {
@@ -1387,17 +1389,91 @@ __device__ __forceinline__ long long xp_index(const PermuteArgs &a, long long q,
     return ((mt * a.ktt + (col >> 5)) * a.bm + lr) * 32 + chunk * 8 + (col & 7);
 }
 
+// Column of chunk u of a lane in the batch from column d0: lanes past the
+// padded row's end take its last chunk again.
+__device__ __forceinline__ int chunk_col(const PermuteArgs &a, int d0, int u, int lane) {
+    return min(d0 + u * 512 + lane * 8, a.ld_xp - 8);
+}
+
+// Columns c .. c + 7 (c a lane's chunk_col) of row t of x as bf16, the pad
+// columns [D, ld_xp) as zeros: the tile image's rows are written whole on
+// every call (its layout changes with the call's tile height, so nothing older
+// may show through).  D >= 8: the load is from column min(c, D - 8), one or two
+// vector loads at the row's own alignment (rows of an odd D are 2- or 4-byte
+// aligned; global loads take any address), and chunk_finish moves the values
+// of a chunk that D cuts down to their places.  All loads of a batch go out
+// before the first is waited for.
+template <bool XB16>
+struct ChunkRaw { u32x4_t v; };
+template <>
+struct ChunkRaw<false> { float f[8]; };
+template <bool XB16>
+__device__ __forceinline__ void chunk_load(const PermuteArgs &a, int t, int c, ChunkRaw<XB16> &r) {
+    const long long at = (long long)t * a.D + min(c, a.D - 8);
+    if constexpr (XB16) __builtin_memcpy(&r.v, (const uint16_t *)a.x + at, 16);
+    else __builtin_memcpy(r.f, (const float *)a.x + at, 32);
+}
+template <bool XB16>
+__device__ __forceinline__ u32x4_t chunk_finish(const PermuteArgs &a, int c, const ChunkRaw<XB16> &r) {
+    u32x4_t v;
+    if constexpr (XB16) {
+        v = r.v;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = f32_to_bf16(r.f[2 * k]) | ((uint32_t)f32_to_bf16(r.f[2 * k + 1]) << 16);
+    }
+    if ((a.D & 7) == 0) {
+        const bool in = c < a.D;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = in ? v[k] : 0u;
+    } else if (__any(c + 8 > a.D)) {
+        // columns by which the loaded values are too low: halves of words, then words
+        const int k = min(max(c - (a.D - 8), 0), 8);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            if (s < k) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) v[w] = (v[w] >> 16) | (w < 3 ? v[w + 1] << 16 : 0u);
+            }
+    }
+    return v;
+}
+// (D < 8: one chunk of values, by elements)
+__device__ __forceinline__ u32x4_t chunk_short(const PermuteArgs &a, int t, int c) {
+    u32x4_t v{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+        if (c + k < a.D) {
+            const long long at = (long long)t * a.D + c + k;
+            const uint32_t h = a.x_bf16 ? ((const uint16_t *)a.x)[at] : f32_to_bf16(((const float *)a.x)[at]);
+            v[k >> 1] |= h << (16 * (k & 1));
+        }
+    return v;
+}
+template <int UB, bool XB16>
+__device__ __forceinline__ void load_chunks(const PermuteArgs &a, int t, int d0, int lane, u32x4_t (&v)[UB]) {
+    constexpr int G = XB16 || UB < 2 ? UB : 2;  // chunks in flight (fp32 x: 8 registers each)
+#pragma unroll
+    for (int g = 0; g < UB; g += G) {
+        ChunkRaw<XB16> r[G];
+#pragma unroll
+        for (int u = 0; u < G; ++u) chunk_load<XB16>(a, t, chunk_col(a, d0, g + u, lane), r[u]);
+#pragma unroll
+        for (int u = 0; u < G; ++u) v[g + u] = chunk_finish<XB16>(a, chunk_col(a, d0, g + u, lane), r[u]);
+    }
+}
+
 // Store U chunks of 8 bf16 per lane into the xp row of every position the
-// token holds (row of lane j: xp row of entry j, < 0 if dropped).  Chunk u of
-// a lane is column min(d0 + 512 u + 8 lane, D - 8), the column its value was
-// loaded from: a lane past the row's end rewrites the last chunk with that
-// chunk's own value, so no store is conditional.
+// token holds (row of lane j: xp row of entry j, < 0 if dropped), each at the
+// column its value was loaded for (chunk_col): a lane past the row's end
+// rewrites the last chunk with that chunk's own value, so no store is
+// conditional.
 template <int U>
 __device__ __forceinline__ void store_row_chunk(const PermuteArgs &a, int row, int d0, int lane,
                                                 const u32x4_t (&v)[U]) {
     int cols[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) cols[u] = min(d0 + u * 512 + lane * 8, a.D - 8);
+    for (int u = 0; u < U; ++u) cols[u] = chunk_col(a, d0, u, lane);
 #pragma nounroll
     for (int j = 0; j < a.kt; ++j) {
         const int q = __shfl(row, j);
@@ -1414,18 +1490,27 @@ __device__ __forceinline__ void store_row_chunk(const PermuteArgs &a, int row, i
 // renormalisation, position), then the wave copies the token's row into
 // every position it owns, converting to the GEMM type.
 // ============================================================================
-// bf16 rows into the bf16 tile image: UB 16-byte chunks per lane per batch
-// (UB * 512 columns, the smallest power of two covering D up to 2048, so that
-// few lanes rewrite the row's last chunk), loaded together from clamped
-// in-row addresses, then stored to every position the token holds.
-__device__ __forceinline__ bool permute_bf16_rows(const PermuteArgs &a) {
-    return a.copy_rows && a.ct == CT_BF16 && a.x_bf16 && (a.D & 7) == 0;
-}
-template <int UB>
+// Rows into the bf16 tile image: UB 16-byte chunks per lane per batch (UB *
+// 512 columns, the smallest power of two covering D up to 2048, so that few
+// lanes rewrite the row's last chunk), loaded together, then stored to every
+// position the token holds.
+__device__ __forceinline__ bool permute_image_rows(const PermuteArgs &a) { return a.copy_rows && a.tiled; }
+// WHOLE: bf16 rows without pad columns (D a multiple of 64), loads only (the
+// branches of the general case cost 2 of 15 us on 16384 rows of 768)
+template <int UB, bool WHOLE>
 __device__ __forceinline__ void load_row_chunk(const PermuteArgs &a, int t, int d0, int lane, u32x4_t (&v)[UB]) {
-    const uint16_t *__restrict__ src = (const uint16_t *)a.x + (long long)t * a.D;
+    if constexpr (WHOLE) {
+        const uint16_t *__restrict__ src = (const uint16_t *)a.x + (long long)t * a.D;
 #pragma unroll
-    for (int u = 0; u < UB; ++u) v[u] = *(const u32x4_t *)(src + min(d0 + u * 512 + lane * 8, a.D - 8));
+        for (int u = 0; u < UB; ++u) __builtin_memcpy(&v[u], src + chunk_col(a, d0, u, lane), 16);
+    } else if (a.D < 8) {
+#pragma unroll
+        for (int u = 0; u < UB; ++u) v[u] = chunk_short(a, t, chunk_col(a, d0, u, lane));
+    } else if (a.x_bf16) {
+        load_chunks<UB, true>(a, t, d0, lane, v);
+    } else {
+        load_chunks<UB, false>(a, t, d0, lane, v);
+    }
 }
 
 // The entry of lane j < kt of a token (its expert id, gate and rank inside
@@ -1489,19 +1574,19 @@ __device__ __forceinline__ int permute_entries(const PermuteArgs &a, int t, int 
 }
 
 // The token's row into every xp row it owns, converting to the GEMM type.
-// bf16 rows: `first` holds the row's first batch (loaded by the caller);
+// Tile image rows: `first` holds the row's first batch (loaded by the caller);
 // each further batch is loaded before the previous one is stored.
-template <int UB>
+template <int UB, bool WHOLE>
 __device__ __forceinline__ void permute_copy(const PermuteArgs &a, int t, int lane, int row,
                                              const u32x4_t (&first)[UB]) {
-    if (permute_bf16_rows(a)) {
+    if (permute_image_rows(a)) {
         u32x4_t cur[UB];
 #pragma unroll
         for (int u = 0; u < UB; ++u) cur[u] = first[u];
         for (int d0 = 0;; d0 += 512 * UB) {
-            const bool more = d0 + 512 * UB < a.D;
+            const bool more = d0 + 512 * UB < a.ld_xp;
             u32x4_t nx[UB];
-            if (more) load_row_chunk<UB>(a, t, d0 + 512 * UB, lane, nx);
+            if (more) load_row_chunk<UB, WHOLE>(a, t, d0 + 512 * UB, lane, nx);
             store_row_chunk<UB>(a, row, d0, lane, cur);
             if (!more) break;
 #pragma unroll
@@ -1509,49 +1594,20 @@ __device__ __forceinline__ void permute_copy(const PermuteArgs &a, int t, int la
         }
         return;
     }
-    if (a.ct == CT_BF16 && !a.x_bf16 && (a.D & 7) == 0) {
-        const float *__restrict__ src = (const float *)a.x + (long long)t * a.D;
-        constexpr int U = 4;
-        for (int d0 = 0; d0 < a.D; d0 += 512 * U) {
-            u32x4_t v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int d = min(d0 + u * 512 + lane * 8, a.D - 8);
-                const float4 f0 = *(const float4 *)(src + d), f1 = *(const float4 *)(src + d + 4);
-                v[u] = u32x4_t{f32_to_bf16(f0.x) | ((uint32_t)f32_to_bf16(f0.y) << 16),
-                                  f32_to_bf16(f0.z) | ((uint32_t)f32_to_bf16(f0.w) << 16),
-                                  f32_to_bf16(f1.x) | ((uint32_t)f32_to_bf16(f1.y) << 16),
-                                  f32_to_bf16(f1.z) | ((uint32_t)f32_to_bf16(f1.w) << 16)};
-            }
-            store_row_chunk<U>(a, row, d0, lane, v);
-        }
-        return;
-    }
     for (int j = 0; j < a.kt; ++j) {
         const int p = __shfl(row, j);
         if (p < 0) continue;
-        if (a.ct == CT_BF16) {
-            uint16_t *dst = (uint16_t *)a.xp;
-            if (a.x_bf16) {
-                const uint16_t *src = (const uint16_t *)a.x + (long long)t * a.D;
-                for (int d = lane; d < a.D; d += 64) dst[xp_index(a, p, d)] = src[d];
-            } else {
-                const float *src = (const float *)a.x + (long long)t * a.D;
-                for (int d = lane; d < a.D; d += 64) dst[xp_index(a, p, d)] = f32_to_bf16(src[d]);
-            }
+        float *dst = (float *)a.xp + (long long)p * a.ld_xp;
+        if (a.x_bf16) {
+            const uint16_t *src = (const uint16_t *)a.x + (long long)t * a.D;
+            for (int d = lane; d < a.D; d += 64) dst[d] = bf16_to_f32(src[d]);
         } else {
-            float *dst = (float *)a.xp + (long long)p * a.ld_xp;
-            if (a.x_bf16) {
-                const uint16_t *src = (const uint16_t *)a.x + (long long)t * a.D;
-                for (int d = lane; d < a.D; d += 64) dst[d] = bf16_to_f32(src[d]);
+            const float *src = (const float *)a.x + (long long)t * a.D;
+            if ((a.D & 3) == 0) {
+                for (int d = lane * 4; d < a.D; d += 256)
+                    *(float4 *)(dst + d) = *(const float4 *)(src + d);
             } else {
-                const float *src = (const float *)a.x + (long long)t * a.D;
-                if ((a.D & 3) == 0) {
-                    for (int d = lane * 4; d < a.D; d += 256)
-                        *(float4 *)(dst + d) = *(const float4 *)(src + d);
-                } else {
-                    for (int d = lane; d < a.D; d += 64) dst[d] = src[d];
-                }
+                for (int d = lane; d < a.D; d += 64) dst[d] = src[d];
             }
         }
     }
@@ -1568,31 +1624,31 @@ __device__ __forceinline__ void permute_copy(const PermuteArgs &a, int t, int la
 // need are in flight before the current stores: rows of one batch (PIPE) the
 // next token's entries and first batch; longer rows (one token per wave at
 // the usual sizes) the row's next batch (permute_copy).
-template <int UB, bool PIPE>
+template <int UB, bool PIPE, bool WHOLE>
 __global__ __launch_bounds__(kPermThreads) void permute_kernel(PermuteArgs a) {
     static_assert(UB <= 4, "row batch held through the scan");
     __shared__ ScanLds L;
     const int lane = threadIdx.x & 63;
     const int t1 = min(a.T, (int)(blockIdx.x + 1) * a.tpw);
     int t = blockIdx.x * a.tpw + (threadIdx.x >> 6);
-    const bool rows16 = permute_bf16_rows(a);
+    const bool rows16 = permute_image_rows(a);
     EntryMeta m = load_meta(a, t < t1 ? t : -1, lane);
     u32x4_t cur[UB];
-    if (rows16 && t < t1) load_row_chunk<UB>(a, t, 0, lane, cur);
+    if (rows16 && t < t1) load_row_chunk<UB, WHOLE>(a, t, 0, lane, cur);
     scan_block(a.s, (int)(((long long)blockIdx.x * a.tpw) / a.rb), L, blockIdx.x == 0);
     for (; t < t1; t += kPermThreads / 64) {
         const int tn = t + kPermThreads / 64;
         const EntryMeta mn = load_meta(a, tn < t1 ? tn : -1, lane);
         u32x4_t nxt[PIPE ? UB : 1];
-        if (PIPE && rows16 && tn < t1) load_row_chunk<PIPE ? UB : 1>(a, tn, 0, lane, nxt);
+        if (PIPE && rows16 && tn < t1) load_row_chunk<PIPE ? UB : 1, WHOLE>(a, tn, 0, lane, nxt);
         const int row = permute_entries(a, t, lane, L, m);
-        if (a.copy_rows) permute_copy<UB>(a, t, lane, row, cur);
+        if (a.copy_rows) permute_copy<UB, WHOLE>(a, t, lane, row, cur);
         m = mn;
         if constexpr (PIPE) {
 #pragma unroll
             for (int u = 0; u < UB; ++u) cur[u] = nxt[u];
         } else if (rows16 && tn < t1) {
-            load_row_chunk<UB>(a, tn, 0, lane, cur);
+            load_row_chunk<UB, WHOLE>(a, tn, 0, lane, cur);
         }
     }
 }
@@ -1600,8 +1656,7 @@ __global__ __launch_bounds__(kPermThreads) void permute_kernel(PermuteArgs a) {
 // Permute for more slots per token than a wave has lanes (ExpertChoiceGating
 // with min(capacity, E) > 64; kt <= MOE_MAX_EXPERTS): lane l owns entries l,
 // l + 64, ... (kWideEnt of them); same finalisation as permute_kernel, then
-// one row copy per kept entry, element by element (most of these slots are
-// empty).
+// one row copy per kept entry (most of these slots are empty).
 constexpr int kWideEnt = MOE_MAX_EXPERTS / 64;
 
 __device__ __forceinline__ void permute_wide_token(const PermuteArgs &a, int t, int lane, const ScanLds &L) {
@@ -1667,12 +1722,18 @@ __device__ __forceinline__ void permute_wide_token(const PermuteArgs &a, int t, 
         for (int l = 0; l < 64 && 64 * c + l < a.kt; ++l) {
             const int p = __shfl(row[c], l);
             if (p < 0) continue;
-            for (int d = lane; d < a.D; d += 64) {
-                const float v = a.x_bf16 ? bf16_to_f32(((const uint16_t *)a.x)[(long long)t * a.D + d])
-                                         : ((const float *)a.x)[(long long)t * a.D + d];
-                if (a.ct == CT_BF16) ((uint16_t *)a.xp)[xp_index(a, p, d)] = f32_to_bf16(v);
-                else ((float *)a.xp)[(long long)p * a.ld_xp + d] = v;
+            if (a.tiled) {
+                for (int d0 = 0; d0 < a.ld_xp; d0 += 512) {
+                    u32x4_t v[1];
+                    load_row_chunk<1, false>(a, t, d0, lane, v);
+                    *(u32x4_t *)((uint16_t *)a.xp + xp_index(a, p, chunk_col(a, d0, 0, lane))) = v[0];
+                }
+                continue;
             }
+            for (int d = lane; d < a.D; d += 64)
+                ((float *)a.xp)[(long long)p * a.ld_xp + d] =
+                    a.x_bf16 ? bf16_to_f32(((const uint16_t *)a.x)[(long long)t * a.D + d])
+                             : ((const float *)a.x)[(long long)t * a.D + d];
         }
 }
 
@@ -1696,11 +1757,20 @@ hipError_t launch_permute(PermuteArgs a, hipStream_t s) {
     a.tpw = kPermTokens;
     while (a.tpw * 2 <= a.rb && a.tpw < 4 * kPermTokens && (a.T + a.tpw - 1) / a.tpw > 512) a.tpw *= 2;
     const int nwg = (a.T + a.tpw - 1) / a.tpw;
-    if (a.kt > 64) hipLaunchKernelGGL(permute_wide_kernel, dim3(nwg), dim3(kPermThreads), 0, s, a);
-    else if (a.D > 2048) hipLaunchKernelGGL((permute_kernel<4, false>), dim3(nwg), dim3(kPermThreads), 0, s, a);
-    else if (a.D > 1024) hipLaunchKernelGGL((permute_kernel<4, true>), dim3(nwg), dim3(kPermThreads), 0, s, a);
-    else if (a.D > 512) hipLaunchKernelGGL((permute_kernel<2, true>), dim3(nwg), dim3(kPermThreads), 0, s, a);
-    else hipLaunchKernelGGL((permute_kernel<1, true>), dim3(nwg), dim3(kPermThreads), 0, s, a);
+    if (a.kt > 64) {
+        hipLaunchKernelGGL(permute_wide_kernel, dim3(nwg), dim3(kPermThreads), 0, s, a);
+        return hipGetLastError();
+    }
+    auto launch = [&](auto WHOLE_) {
+        constexpr bool W = decltype(WHOLE_)::value;
+        const dim3 grid(nwg), block(kPermThreads);
+        if (a.D > 2048) hipLaunchKernelGGL((permute_kernel<4, false, W>), grid, block, 0, s, a);
+        else if (a.D > 1024) hipLaunchKernelGGL((permute_kernel<4, true, W>), grid, block, 0, s, a);
+        else if (a.D > 512) hipLaunchKernelGGL((permute_kernel<2, true, W>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((permute_kernel<1, true, W>), grid, block, 0, s, a);
+    };
+    if (a.x_bf16 && a.D == a.ld_xp) launch(std::true_type{});
+    else launch(std::false_type{});
     return hipGetLastError();
 }
 

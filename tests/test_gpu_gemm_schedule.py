@@ -82,3 +82,66 @@ def test_expert_forward_paired_and_split(moe, oracle, n):
         assert np.array_equal(y.view(np.uint32), y2.view(np.uint32))
     finally:
         c.dev.close()
+
+
+@pytest.mark.parametrize("etype,act,H", [("gated", "silu", 2816), ("standard", "gelu", 5632)])
+def test_256_row_tiles_and_their_change_between_calls(moe, oracle, etype, act, H):
+    # 16 experts averaging 512 rows with 22 n-tiles: at least four rounds of
+    # up items, so 256-row tiles, several experts ending in a tile of at most
+    # 128 rows (paired items); calls of fewer tokens on the same handle take
+    # 128-row tiles.  D = 100 ends inside a K stage: the pads of either
+    # layout must not show what the other left there, an infinity or a NaN
+    # included
+    rng = np.random.default_rng(83)
+    bias = (rng.standard_normal(16) * 0.6).astype(np.float32)
+    c = Case(moe, oracle, T=4096, D=100, H=H, Dout=72, E=16, k=2, expert_type=etype, act=act, wdtype="bf16",
+             xdtype="bf16", seed=83, router_bias=bias)
+    try:
+        print(f"256-row tiles {etype} H={H}", flush=True)
+        big, loss, res = c.run(training=True)
+        w, paired = _up_items(res["counts"], 22)
+        assert paired > 0 and w % 256 != 0  # (by rows / 256 + experts M tiles the rule counts 48 * 22 items)
+        check_case(c, TOL["bf16"])
+        check_case(c, TOL["bf16"], T=300)
+        small = c.run(training=True, T=300)[0]
+        x = c.x_dev.copy()
+        x[::7, 99], x[::5, 3] = 0x7f80, 0x7fc0  # +Inf and NaN bit patterns
+        c.dev.forward(np.ascontiguousarray(x), c.xcode, True)
+        again = c.run(training=True, T=300)[0]
+        assert np.array_equal(again.view(np.uint32), small.view(np.uint32))
+        c.dev.forward(np.ascontiguousarray(x[:300]), c.xcode, True)
+        again = c.run(training=True)[0]
+        assert np.array_equal(again.view(np.uint32), big.view(np.uint32))
+    finally:
+        c.dev.close()
+
+
+@pytest.mark.parametrize("n", [600, 700])
+def test_expert_forward_256_row_tiles(moe, oracle, n):
+    # one expert's rows on such a handle: two full tiles and a paired one of 88
+    # rows, or an unpaired one of 188
+    c = Case(moe, oracle, T=4096, D=100, H=2816, E=16, k=2, wdtype="bf16", xdtype="bf16", seed=84)
+    try:
+        print(f"expert_forward 256-row tiles, 22 n-tiles, n={n}", flush=True)
+        x = np.ascontiguousarray(c.x[:n])
+        y = c.dev.expert_forward(5, x)
+        ex = c.ex[5]
+        xd = x.astype(np.float64)
+        g, u = xd @ ex["w1"].T.astype(np.float64), xd @ ex["w3"].T.astype(np.float64)
+        h = _bf16_round(oracle, (g / (1.0 + np.exp(-g))) * u).astype(np.float64)
+        err = rel_err(y, h @ ex["w2"].T.astype(np.float64))
+        assert err <= TOL["bf16"], err
+    finally:
+        c.dev.close()
+
+
+@pytest.mark.parametrize("D,xdtype", [(5, "bf16"), (9, "bf16"), (63, "f32"), (100, "f32"), (513, "bf16"), (1031, "bf16"),
+                                      (2052, "f32"), (2055, "bf16")])
+def test_permute_rows_of_any_width(moe, oracle, D, xdtype):
+    # the tile image's rows: widths below one 16-byte chunk, cut inside a
+    # chunk, past one batch of chunks, of rows at 2- and 4-byte alignment
+    c = Case(moe, oracle, T=70, D=D, H=64, Dout=64, E=4, k=2, wdtype="bf16", xdtype=xdtype, seed=90 + D)
+    try:
+        check_case(c, TOL["bf16"])
+    finally:
+        c.dev.close()
