@@ -272,7 +272,13 @@ __device__ __forceinline__ void load_plan(const GemmArgs &g, const TileJob &jb, 
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
         const int r = w * (BMA / NWAVE) + 16 * i;
-        gsrc[i] = Ab + (long long)r * ROWB;
+        // 16 rows past the tile's valid ones: every lane reads the same 16 bytes
+        // (the products of those rows are not used, the load itself keeps the
+        // vmcnt arithmetic).  With the h rows past the valid ones left
+        // unwritten (store_staged), us: 48 tokens on 8 experts of 4096 / 14336 470
+        // -> 441, 517 on 66 fp8 ones of 2048 / 1408 184 -> 169, 16384 on 128 of
+        // 768 / 3072 407 -> 389
+        gsrc[i] = r < jb.rows ? Ab + (long long)r * ROWB : Ab - lane * 16;
         ldst[i] = r * ROWB;
     }
     constexpr int BR = WF8 ? 32 : 16;  // B-tile rows per load
@@ -482,7 +488,7 @@ struct StagePut {
 
 // Stores the staged tile.  Up GEMMs: h goes out as the down GEMM's A tile
 // image, in which the tile's CW / 64 K stages of 64-B rows are one contiguous
-// region (all BM rows, including rows past the valid ones): thread t writes
+// region (the valid rows of it): thread t writes
 // 16-byte units t, t + NT, ... (NT threads), unit u being chunk position u & 3 of row
 // (u >> 2) mod BM of stage block u / (4 BM).  Down GEMM: y rows; thread t
 // copies chunk t mod CH of rows t / CH + k (NT / CH), valid rows only and
@@ -506,7 +512,10 @@ __device__ __forceinline__ void store_staged(const GemmArgs &g, const TileJob &j
                 v[q] = *(const MOE_LDS_AS u32x4_t *)(row_addr(r) + ((ch ^ (r & (CH - 1))) << 4));
             }
 #pragma unroll
-            for (int q = 0; q < U; ++q) *(u32x4_t *)(base + (long long)(u0 + q * NT + threadIdx.x) * 16) = v[q];
+            for (int q = 0; q < U; ++q) {
+                const int u = u0 + q * NT + (int)threadIdx.x;
+                if ((u >> 2) % BM < jb.rows) *(u32x4_t *)(base + (long long)u * 16) = v[q];
+            }
         }
     } else {
         constexpr int RPP = NT / CH;  // rows per pass of the workgroup
@@ -556,7 +565,8 @@ __device__ __forceinline__ void store_staged_pair(const GemmArgs &g, const TileJ
             const int u = u0 + q * NT + (int)threadIdx.x;
             const int hf = u / NUH, up = u - hf * NUH;
             uint8_t *base = (uint8_t *)g.C + ((long long)jb.mt * KTT + (jb.n0 + hf * NTW) / 32) * BM * 64;
-            *(u32x4_t *)(base + (long long)(up / (4 * BMA)) * BM * 64 + (up % (4 * BMA)) * 16) = v[q];
+            if ((up >> 2) % BMA < jb.rows)
+                *(u32x4_t *)(base + (long long)(up / (4 * BMA)) * BM * 64 + (up % (4 * BMA)) * 16) = v[q];
         }
     }
 }
@@ -571,18 +581,17 @@ struct RowOffsetPut {
     }
 };
 
-// Prologue: this wave's NL loads of stages 0 .. NS-2 (clamped to the last
-// stage), stage s into slot s.
-#define MOE_PROLOGUE_LOADS(NS, NL, KT)                                       \
-    _Pragma("unroll") for (int s0 = 0; s0 < NS - 1; ++s0) {                  \
+// Prologue: this wave's NL loads of stages 0 .. NS-2 and the first NL1 of
+// stage NS-1 (clamped to the last stage), stage s into slot s.
+#define MOE_PROLOGUE_LOADS(NS, NL, NL1, KT)                                  \
+    _Pragma("unroll") for (int s0 = 0; s0 < NS; ++s0) {                      \
         const int kt = min(s0, KT - 1);                                      \
-        _Pragma("unroll") for (int i = 0; i < NL; ++i) {                     \
+        _Pragma("unroll") for (int i = 0; i < (s0 < NS - 1 ? NL : NL1); ++i) { \
             switch (s0) {                                                    \
             case 0: dma(ic<0>{}, kt, i); break;                              \
             case 1: dma(ic<1>{}, kt, i); break;                              \
             case 2: dma(ic<2>{}, kt, i); break;                              \
-            case 3: dma(ic<3>{}, kt, i); break;                              \
-            default: dma(ic<4>{}, kt, i); break;                             \
+            default: dma(ic<3>{}, kt, i); break;                             \
             }                                                                \
         }                                                                    \
     }
@@ -597,14 +606,10 @@ struct RowOffsetPut {
             stage(ic<1>{}, st + 1);                                               \
             stage(ic<2 % NS>{}, st + 2);                                          \
             if constexpr (NS > 3) stage(ic<3 % NS>{}, st + 3);                    \
-            if constexpr (NS > 4) stage(ic<4 % NS>{}, st + 4);                    \
-            if constexpr (NS > 5) stage(ic<5 % NS>{}, st + 5);                    \
         }                                                                         \
         if (st < KT) stage(ic<0>{}, st);                                          \
         if (st + 1 < KT) stage(ic<1 % NS>{}, st + 1);                             \
         if constexpr (NS > 3) if (st + 2 < KT) stage(ic<2 % NS>{}, st + 2);       \
-        if constexpr (NS > 4) if (st + 3 < KT) stage(ic<3 % NS>{}, st + 3);       \
-        if constexpr (NS > 5) if (st + 4 < KT) stage(ic<4 % NS>{}, st + 4);       \
     }
 
 // ============================================================================
@@ -668,7 +673,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
     constexpr int RING = RingShape<BM, WF8, OCC>::BYTES;
     // LDS ring slots (<= 144 KB per CU)
     constexpr int NS = PAIR ? RING / STAGE : RingShape<BM, WF8, OCC>::NS;
-    static_assert(NS >= 3 && NS <= 6, "ring depth");
+    static_assert(NS >= 3 && NS <= 4, "ring depth");
     constexpr int MW = BMA / 64;         // waves along M, 64 rows each
     constexpr int WN = 128;              // wave tile columns (2 waves along N)
     constexpr int IM = 4;                // 16-row blocks per wave
@@ -677,7 +682,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
     constexpr int LA = BMA / (16 * NWAVE);  // A loads (16 rows each) per wave per stage
     constexpr int LB = BRW / ((WF8 ? 32 : 16) * NWAVE);  // B loads per wave per stage
     constexpr int NL = LA + LB;          // 16-byte loads per lane per stage
-    constexpr int NL0 = NL / 2;          // of which issued in a stage's first sub-step
+    constexpr int NL1 = NL - NL / 2;     // of which issued in the half stage in which the slot becomes free
     static_assert(NS * STAGE <= RING && RING * OCC <= 160 * 1024, "LDS");
     auto slot = [&](auto J_) -> MOE_LDS_AS uint8_t * {
         constexpr int J = decltype(J_)::value;
@@ -724,22 +729,26 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
     u32x2_t braw[2][JH];  // WF8: the weight bytes, widened when they are used
 
     // ---- main loop --------------------------------------------------------------
-    // Stage s (32 K columns) lives in ring slot s % NS and is loaded NS - 1
-    // stages ahead.  Its MFMAs run in two halves of the wave's columns, rows in
+    // Stage s (32 K columns) lives in ring slot s % NS and is loaded NS stages
+    // ahead.  Its MFMAs run in two halves of the wave's columns, rows in
     // order; a row block's fragment is replaced by the next stage's once the
     // second half is past it.  Per stage:
-    //   half 0: MFMAs of columns [0, JH)  | LDS reads of (s, columns [JH, JN))       | loads of stage s+NS-1, first half
+    //   half 0: MFMAs of columns [0, JH)  | LDS reads of (s, columns [JH, JN))       | loads NL1 .. NL-1 of stage s-1+NS
     //   wait until this wave's loads of stage s+1 landed; barrier (every wave's have)
-    //   half 1: MFMAs of columns [JH, JN) | LDS reads of (s+1, rows, columns [0, JH)) | loads of stage s+NS-1, second half
-    // Stage s+NS-1 goes to the slot of stage s-1, whose last reads (its half 0)
-    // ended before the barrier of stage s-1.  Past the last stage
-    // the loads repeat stage KT-1 (in bounds, into a slot nothing reads again),
-    // which keeps the vmcnt arithmetic exact: when the barrier of stage s is
-    // reached, the loads issued after those of stage s+1 are NS-3 whole stages
-    // and the first NL0 loads of stage s+NS-1.
-    constexpr int AFTER = (NS - 3) * NL + NL0;
-    MOE_PROLOGUE_LOADS(NS, NL, KT)
-    wait_vmcnt<(NS - 2) * NL>();  // stage 0 landed
+    //   half 1: MFMAs of columns [JH, JN) | LDS reads of (s+1, rows, columns [0, JH)) | loads 0 .. NL1-1 of stage s+NS
+    // Nothing of slot s is read after the barrier of stage s (the rows and the
+    // first columns are read in half 1 of stage s-1, the rest in half 0), so
+    // stage s+NS goes there from half 1 on: between NS-2 and NS-1 whole stages
+    // are in flight, half a stage more than when stage s filled slot s-1 (up
+    // GEMM of 128 standard experts of 768 / 3072, 16384 rows: 186 -> 169 us; of 8 of
+    // 4096 / 14336, 8192 rows: 1625 -> 1595).  Past the last
+    // stage the loads repeat stage KT-1 (in bounds, into a slot nothing reads
+    // again), which keeps the vmcnt arithmetic exact: when the barrier of stage
+    // s is reached, the loads issued after those of stage s+1 are NS-2 whole
+    // stages.
+    constexpr int AFTER = (NS - 2) * NL;
+    MOE_PROLOGUE_LOADS(NS, NL, NL1, KT)
+    wait_vmcnt<(NS - 2) * NL + NL1>();  // stage 0 landed
     barrier_lds();
 
     // The loop of a wave whose first NV 32-row blocks hold rows of the tile:
@@ -779,11 +788,10 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
         auto stage = [&](auto J_, int st) {
             constexpr int J = decltype(J_)::value;
             using Jn = ic<(J + 1) % NS>;       // slot of stage s+1
-            using Jl = ic<(J + NS - 1) % NS>;  // slot of stage s-1 = s+NS-1
-            const int kl = min(st + NS - 1, KT - 1);
+            using Jp = ic<(J + NS - 1) % NS>;  // slot of stages s-1 and s-1+NS
             read_b(J_, 1);
 #pragma unroll
-            for (int t = 0; t < NL0; ++t) dma(Jl{}, kl, t);
+            for (int t = NL1; t < NL; ++t) dma(Jp{}, min(st - 1 + NS, KT - 1), t);
             widen(0);
 #pragma unroll
             for (int i = 0; i < NF; ++i) row_mfmas(i, 0);
@@ -797,7 +805,7 @@ __device__ __forceinline__ void tile_body(const GemmArgs &g, const TileJob &jb, 
             barrier_lds();
             read_b(Jn{}, 0);
 #pragma unroll
-            for (int t = NL0; t < NL; ++t) dma(Jl{}, kl, t);
+            for (int t = 0; t < NL1; ++t) dma(J_, min(st + NS, KT - 1), t);
             widen(1);
 #pragma unroll
             for (int i = 0; i < NF; ++i) {
