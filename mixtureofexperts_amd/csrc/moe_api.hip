@@ -128,6 +128,11 @@ struct moe_handle {
     int ncu = 256;              // compute units: workgroup slots of one GEMM round
     void *x_dev = nullptr;
     float *out_dev = nullptr;
+    // pinned host memory of the host-buffer calls: kHostPin bytes each for x,
+    // out and the routing's rows, then the scalars and counts.  Made by the
+    // first of them; pin_busy from a call's first copy to the end of its wait.
+    uint8_t *pin = nullptr;
+    bool pin_failed = false, pin_busy = false;
 
     // AuxiliaryFreeLoss state (src/balancing/auxiliary_free.jl:11-20): bias and
     // momentum on the device, the update counter on the host
@@ -165,6 +170,8 @@ static int dalloc(moe_handle *h, void **p, size_t bytes) {
 }
 
 static void free_all(moe_handle *h) {
+    if (h->pin) (void)hipHostFree(h->pin);
+    h->pin = nullptr;
     for (void *p : h->allocs) (void)hipFree(p);
     h->allocs.clear();
 }
@@ -872,6 +879,33 @@ static int forward_locked(moe_handle *h, const void *x_dev, int x_dtype, int T, 
     return MOE_OK;
 }
 
+// x, out and the routing's rows of at most this many bytes pass through the
+// handle's pinned memory.  A copy from or to pageable memory is staged by the
+// runtime and waited for by the calling thread; four or five of them were
+// 50 of the 155 us of a 32-token layer call (now 104) and 43 of the 78 us of a
+// one-token decode call (now 36).  Larger ones keep the runtime's staged
+// copies, which overlap the host's and the device's halves.
+constexpr size_t kHostPin = 256 * 1024;
+
+// The pinned memory, or null (then the copies go straight from and to the
+// caller's memory).
+static uint8_t *host_pin(moe_handle *h) {
+    if (!h->pin && !h->pin_failed) {
+        void *p = nullptr;
+        if (hipHostMalloc(&p, 3 * kHostPin + sizeof(float) * (8 + (size_t)h->E), hipHostMallocDefault) == hipSuccess) {
+            h->pin = (uint8_t *)p;
+        } else {
+            (void)hipGetLastError();
+            h->pin_failed = true;
+        }
+    }
+    if (h->pin && h->pin_busy) {  // an earlier call failed between its copies and its wait
+        (void)hipStreamSynchronize(h->stream);
+        h->pin_busy = false;
+    }
+    return h->pin;
+}
+
 static int ensure_io_buffers(moe_handle *h) {
     if (!h->x_dev) {
         int r = dalloc(h, &h->x_dev, sizeof(float) * (size_t)h->T_max * h->D);
@@ -1014,14 +1048,15 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
     h->nsup_max = (h->nblk_max + kSuper - 1) / kSuper;
     A((void **)&h->sup_cnt2, sizeof(int) * 2 * (size_t)h->nsup_max * h->ldc);
     A((void **)&h->sup_p2, sizeof(unsigned long long) * 2 * (size_t)h->nsup_max * h->ldc);
-    A((void **)&h->counts, sizeof(int) * E);
     A((void **)&h->offsets, sizeof(int) * (E + 1));
     A((void **)&h->cap, sizeof(int));
     A((void **)&h->tiles, sizeof(int2) * (size_t)h->max_tiles);
     A((void **)&h->num_tiles, sizeof(int));
     A((void **)&h->tile_start, sizeof(int) * (E + 1));
     A((void **)&h->item_start, sizeof(int) * (E + 1));
-    A((void **)&h->scalars, sizeof(float) * 8);
+    // the scalars, then the counts (read back together)
+    A((void **)&h->scalars, sizeof(float) * (8 + E));
+    h->counts = (int *)(h->scalars + 8);
     if (cfg->gate_kind == MOE_GATE_EXPERT_CHOICE) A((void **)&h->ec_sel, sizeof(uint16_t) * T * E);
     A((void **)&h->aux_bias, sizeof(float) * aux_free_len(h));
     A((void **)&h->aux_mom, sizeof(float) * aux_free_len(h));
@@ -1544,27 +1579,44 @@ static int forward_host_locked(moe_handle *h, const void *x, int32_t x_dtype, in
     r = join_stream(h, s);
     if (r != MOE_OK) return r;
     const size_t xbytes = (x_dtype == MOE_BF16 ? 2 : 4) * (size_t)T * h->D;
-    HIP_TRY(h, hipMemcpyAsync(h->x_dev, x, xbytes, hipMemcpyHostToDevice, s));
+    const size_t obytes = sizeof(float) * (size_t)T * h->Dout;
+    uint8_t *pin = host_pin(h);
+    h->pin_busy = pin != nullptr;
+    if (pin && xbytes <= kHostPin) {
+        memcpy(pin, x, xbytes);
+        HIP_TRY(h, hipMemcpyAsync(h->x_dev, pin, xbytes, hipMemcpyHostToDevice, s));
+    } else {
+        HIP_TRY(h, hipMemcpyAsync(h->x_dev, x, xbytes, hipMemcpyHostToDevice, s));
+    }
     h->keep_rows = aux && (aux->logits || aux->probs);
-    r = forward_locked(h, h->x_dev, x_dtype, T, training, h->out_dev, nullptr, s);
+    // a small out is written by the combine straight into the pinned memory
+    float *opin = (pin && obytes <= kHostPin) ? (float *)(pin + kHostPin) : nullptr;
+    r = forward_locked(h, h->x_dev, x_dtype, T, training, opin ? opin : h->out_dev, nullptr, s);
     if (r != MOE_OK) return r;
-    HIP_TRY(h, hipMemcpyAsync(out, h->out_dev, sizeof(float) * (size_t)T * h->Dout, hipMemcpyDeviceToHost, s));
-    float sc[4] = {0, 0, 0, 0};
-    HIP_TRY(h, hipMemcpyAsync(sc, h->scalars, sizeof(float) * 4, hipMemcpyDeviceToHost, s));
+    if (!opin) HIP_TRY(h, hipMemcpyAsync(out, h->out_dev, obytes, hipMemcpyDeviceToHost, s));
+    // the scalars and the counts behind them, in one copy
+    float sc_own[4] = {0, 0, 0, 0};
+    const float *sc = pin ? (const float *)(pin + 3 * kHostPin) : sc_own;
+    if (pin) HIP_TRY(h, hipMemcpyAsync(pin + 3 * kHostPin, h->scalars, sizeof(float) * (8 + (size_t)h->E), hipMemcpyDeviceToHost, s));
+    else HIP_TRY(h, hipMemcpyAsync(sc_own, h->scalars, sizeof(float) * 4, hipMemcpyDeviceToHost, s));
     const size_t nk = (size_t)T * h->kc;
     if (aux) {
         if (aux->logits) HIP_TRY(h, hipMemcpyAsync(aux->logits, h->logits, sizeof(float) * (size_t)T * h->Er, hipMemcpyDeviceToHost, s));
         if (aux->probs) HIP_TRY(h, hipMemcpyAsync(aux->probs, h->probs, sizeof(float) * (size_t)T * h->Er, hipMemcpyDeviceToHost, s));
         if (aux->indices) HIP_TRY(h, hipMemcpyAsync(aux->indices, h->idx, sizeof(int) * nk, hipMemcpyDeviceToHost, s));
         if (aux->gates) HIP_TRY(h, hipMemcpyAsync(aux->gates, h->gates, sizeof(float) * nk, hipMemcpyDeviceToHost, s));
-        if (aux->counts) HIP_TRY(h, hipMemcpyAsync(aux->counts, h->counts, sizeof(int) * h->E, hipMemcpyDeviceToHost, s));
+        if (aux->counts && !pin)
+            HIP_TRY(h, hipMemcpyAsync(aux->counts, h->counts, sizeof(int) * h->E, hipMemcpyDeviceToHost, s));
         if (aux->offsets) HIP_TRY(h, hipMemcpyAsync(aux->offsets, h->offsets, sizeof(int) * (h->E + 1), hipMemcpyDeviceToHost, s));
         if (aux->perm) HIP_TRY(h, hipMemcpyAsync(aux->perm, h->perm, sizeof(int) * nk, hipMemcpyDeviceToHost, s));
     }
     HIP_TRY(h, hipStreamSynchronize(s));
     settle(h);
+    h->pin_busy = false;
+    if (opin) memcpy(out, opin, obytes);
     if (loss) *loss = sc[2];
     if (aux) {
+        if (aux->counts && pin) memcpy(aux->counts, sc + 8, sizeof(int) * h->E);
         if (aux->switch_loss) *aux->switch_loss = sc[0];
         if (aux->z_loss) *aux->z_loss = sc[1];
         if (aux->mean_entropy) *aux->mean_entropy = sc[3];
@@ -1720,15 +1772,33 @@ int moe_decode(moe_handle *h, const float *xb, int32_t n, float *out, float *log
     hipStream_t s = h->stream;
     r = join_stream(h, s);
     if (r != MOE_OK) return r;
-    HIP_TRY(h, hipMemcpyAsync(h->x_dev, xb, sizeof(float) * (size_t)n * h->D, hipMemcpyHostToDevice, s));
-    r = decode_locked(h, (const float *)h->x_dev, n, h->out_dev, s);
+    // through the pinned memory where x, out and the routing's rows fit (host_pin)
+    const size_t xbytes = sizeof(float) * (size_t)n * h->D, obytes = sizeof(float) * (size_t)n * h->Dout;
+    const size_t lbytes = sizeof(float) * (size_t)n * h->Er, kbytes = sizeof(int) * (size_t)n * h->kt;
+    uint8_t *pin = host_pin(h);
+    if (xbytes > kHostPin || obytes > kHostPin || lbytes + 2 * kbytes > kHostPin) pin = nullptr;
+    h->pin_busy = pin != nullptr;
+    if (pin) memcpy(pin, xb, xbytes);
+    HIP_TRY(h, hipMemcpyAsync(h->x_dev, pin ? (const void *)pin : xb, xbytes, hipMemcpyHostToDevice, s));
+    float *o = pin ? (float *)(pin + kHostPin) : h->out_dev;
+    uint8_t *rows = pin ? pin + 2 * kHostPin : nullptr;
+    void *lo = pin ? (void *)rows : logits, *io = pin ? (void *)(rows + lbytes) : indices,
+         *go = pin ? (void *)(rows + lbytes + kbytes) : gates;
+    r = decode_locked(h, (const float *)h->x_dev, n, o, s);
     if (r != MOE_OK) return r;
-    HIP_TRY(h, hipMemcpyAsync(out, h->out_dev, sizeof(float) * (size_t)n * h->Dout, hipMemcpyDeviceToHost, s));
-    if (logits) HIP_TRY(h, hipMemcpyAsync(logits, h->logits, sizeof(float) * (size_t)n * h->Er, hipMemcpyDeviceToHost, s));
-    if (indices) HIP_TRY(h, hipMemcpyAsync(indices, h->idx, sizeof(int) * (size_t)n * h->kt, hipMemcpyDeviceToHost, s));
-    if (gates) HIP_TRY(h, hipMemcpyAsync(gates, h->gates, sizeof(float) * (size_t)n * h->kt, hipMemcpyDeviceToHost, s));
+    if (!pin) HIP_TRY(h, hipMemcpyAsync(out, o, obytes, hipMemcpyDeviceToHost, s));
+    if (logits) HIP_TRY(h, hipMemcpyAsync(lo, h->logits, lbytes, hipMemcpyDeviceToHost, s));
+    if (indices) HIP_TRY(h, hipMemcpyAsync(io, h->idx, kbytes, hipMemcpyDeviceToHost, s));
+    if (gates) HIP_TRY(h, hipMemcpyAsync(go, h->gates, kbytes, hipMemcpyDeviceToHost, s));
     HIP_TRY(h, hipStreamSynchronize(s));
     settle(h);
+    if (pin) {
+        h->pin_busy = false;
+        memcpy(out, o, obytes);
+        if (logits) memcpy(logits, lo, lbytes);
+        if (indices) memcpy(indices, io, kbytes);
+        if (gates) memcpy(gates, go, kbytes);
+    }
     return MOE_OK;
 }
 
