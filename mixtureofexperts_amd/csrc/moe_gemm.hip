@@ -295,7 +295,13 @@ static hipError_t launch_f32x3(const GemmArgs &g, hipStream_t s) {
     constexpr int BN = MODE == MODE_GATED_UP ? 128 : 256;
     long long total = (long long)g.m_tiles_grid * g.n_tiles * g.ksplit;
     total = (total + 7) / 8 * 8;
-    hipLaunchKernelGGL((grouped_gemm_f32x3_kernel<MODE>), dim3((unsigned)total), dim3(512), 0, s, g);
+    // Running sums where they are faster and no less accurate than the fp32
+    // MFMA: K of 512 or more (error of a 512 / 1024 gated layer 6.4e-7, fp32 MFMA
+    // 8.5e-7) and 128 x 128 tiles for every CU, where neither kernel cuts K into
+    // ranges
+    if (g.K >= 512 && g.ksplit == 1 && (long long)g.m_tiles_grid * g.n_tiles * (BN / 128) >= g.ncu)
+        hipLaunchKernelGGL((grouped_gemm_f32x3_kernel<MODE, false>), dim3((unsigned)total), dim3(512), 0, s, g);
+    else hipLaunchKernelGGL((grouped_gemm_f32x3_kernel<MODE, true>), dim3((unsigned)total), dim3(512), 0, s, g);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && g.ksplit > 1) {
         hipLaunchKernelGGL((fold_f32_kernel<MODE, BN>), dim3((unsigned)(g.m_tiles_grid * g.n_tiles), kGemmBM * BN / 256),

@@ -38,6 +38,18 @@
 // NaN or infinite sums, and every output that is not finite is recomputed
 // from the fp32 operands, one K value after the other.
 //
+// STAGE_SUMS: the six products of a stage start from zero, the smallest first,
+// and are added to the running sum with one rounded addition.  The matrix unit
+// cuts every sum off (towards zero: a bias), so six sums of the running size
+// per 32 K cost more accuracy at small K than grouped_gemm_kernel's 16 of
+// random sign: error against 64 bits at 300 / 300 gated 2.5e-7 there, 5.0e-7 with
+// running sums, 1.6e-7 with stage sums; 64 / 64 2.0e-7, 2.9e-7, 1.0e-7; 128 / 256
+// standard 1.8e-7, 3.4e-7, 1.2e-7; 768 / 3072 standard 11.3e-7, 9.9e-7,
+// 2.6e-7.
+// The additions wait for the matrix unit and cost 6 % where it is the bound
+// (768 / 3072 standard, 4096 tokens: 427 -> 453 us), 0 to 2 % elsewhere, so the running sums
+// stay for large calls of large K (launch_f32x3).
+//
 // K split (g.ksplit = S > 1): as in grouped_gemm_kernel, blocks of BM x 256
 // floats.
 
@@ -64,7 +76,7 @@ __device__ __forceinline__ void split8(const f32x4_t &a, const f32x4_t &b, u32x4
     }
 }
 
-template <int MODE>
+template <int MODE, bool STAGE_SUMS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void grouped_gemm_f32x3_kernel(GemmArgs g) {
     constexpr int NB = (MODE == MODE_GATED_UP) ? 2 : 1;
     constexpr int BM = kGemmBM, BR = 256;         // tile rows, weight rows
@@ -169,14 +181,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                                                            (NB == 2 ? j * 128 + hf * 16 : (2 * hf + j) * 16) * 64);
         };
         auto row_mfmas = [&](int i, int hf) {
+            f32x4_t t2[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) t2[j] = STAGE_SUMS ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : acc[i][2 * hf + j];
 #pragma unroll
             for (int t = 0; t < 6; ++t) {
-                constexpr int PA[6] = {0, 0, 1, 1, 0, 2}, PB[6] = {0, 1, 0, 1, 2, 0};
+                constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    acc[i][2 * hf + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[hf][j][PB[t]], fa[i][PA[t]],
-                                                                                 acc[i][2 * hf + j], 0, 0, 0);
+                    t2[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[hf][j][PB[t]], fa[i][PA[t]], t2[j], 0, 0, 0);
             }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][2 * hf + j] = STAGE_SUMS ? acc[i][2 * hf + j] + t2[j] : t2[j];
         };
         // after each pair of MFMAs: VA vector instructions of the split, an LDS
         // read, at the end the LDS writes
@@ -203,7 +219,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int i = 0; i < NF; ++i) row_mfmas(i, 0);
             if constexpr (NV > 0)
-                interleave(std::integral_constant<int, 10 / NV>{}, std::integral_constant<int, 6>{},
+                interleave(std::integral_constant<int, (STAGE_SUMS ? 12 : 10) / NV>{}, std::integral_constant<int, 6>{},
                            std::integral_constant<int, 6>{});
             barrier();
             read_b(cur ^ 1, 0);
@@ -215,7 +231,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 read_a(cur ^ 1, i);
             }
             if constexpr (NV > 0)
-                interleave(std::integral_constant<int, 6 / NV>{}, std::integral_constant<int, 6 * NF>{},
+                interleave(std::integral_constant<int, (STAGE_SUMS ? 8 : 6) / NV>{}, std::integral_constant<int, 6 * NF>{},
                            std::integral_constant<int, 3>{});
         }
     };

@@ -51,6 +51,29 @@ def test_f32x3_layer(moe, oracle, T, D, H, Dout, E, k, etype, act):
         c.dev.close()
 
 
+@pytest.mark.parametrize("T,D,H,E,k,etype,act", [
+    (192, 64, 64, 4, 1, "gated", "silu"),       # two stages per sum
+    (128, 128, 256, 4, 2, "standard", "gelu"),
+    (128, 300, 300, 4, 2, "gated", "silu"),     # a partial last stage
+    (600, 480, 448, 3, 2, "gated", "silu"),     # the largest K below the running sums', both row blocks
+])
+def test_f32x3_small_k(moe, oracle, T, D, H, E, k, etype, act):
+    # Small K: as accurate as the fp32 matrix unit (2.0e-7, 1.8e-7 and 2.5e-7 on the
+    # first three).  Per GEMM sqrt(K / 32) 2^-25 for the rounded additions of the
+    # stages (1.2e-7 at 480) and, since stage sums are cut off, at most 2^-23 of a stage, random
+    # over them: about 0.6 x 2^-23; h rounds once more.  Two GEMMs in
+    # turn and the gates: below 10 x 2^-25.
+    c = Case(moe, oracle, T=T, D=D, H=H, E=E, k=k, gate="switch" if k == 1 else "topk", expert_type=etype, act=act,
+             wdtype="f32", seed=700 + D)
+    try:
+        out, _, res = c.run(training=True)
+        ref = exact_forward(c, res["indices"], res["gates"])
+        err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+        assert err <= 10 * 2.0 ** -25, err
+    finally:
+        c.dev.close()
+
+
 @pytest.mark.parametrize("H", [96, 2816])
 def test_f32x3_infinities_and_nan(moe, oracle, H):
     # values whose parts overflow or are not finite: the outputs they enter
