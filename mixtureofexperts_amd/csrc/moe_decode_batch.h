@@ -284,6 +284,19 @@ __device__ __forceinline__ float wave_total(const f32x4_t *red, int nwave, int q
     return s;
 }
 
+// A bf16 weight row with K fp32 values, one after the other: an output whose
+// sum is not finite is recomputed by it.  An infinite weight gives NaN with
+// the zero parts of a finite x (and infinities of both signs with parts of
+// both signs), where the product itself is an infinity.
+template <typename X>
+__device__ __forceinline__ float row_serial(const uint16_t *w, int K, X x) {
+#pragma clang fp contract(off)
+    float s = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < K; ++k) s = s + bf16_to_f32(w[k]) * x(k);
+    return s;
+}
+
 constexpr int kUpWaves = 4;
 constexpr int kBatchNT = 2;  // column tiles of 16 entries per pass over the weights
 
@@ -307,6 +320,11 @@ __device__ __forceinline__ void up_tile(const DecodeArgs &a, const DecodeBatch &
             if constexpr (WF8) {
                 g = g * a.s1[(long long)e * a.Hpad + r0 + r];
                 up = up * a.s3[(long long)e * a.Hpad + r0 + r];
+            } else if (r0 + r < a.H && !(__builtin_isfinite(g) && __builtin_isfinite(up))) {
+                const float *x = a.x + (long long)(L.list[j0 + c] / a.kt) * a.D;
+                const long long wo = (long long)e * a.w1_stride + (long long)(r0 + r) * a.Dpad;
+                g = row_serial((const uint16_t *)a.w1 + wo, a.D, [&](int k) { return x[k]; });
+                up = row_serial((const uint16_t *)a.w3 + wo, a.D, [&](int k) { return x[k]; });
             }
             // pad rows: 0 whatever x holds
             const float h = r0 + r < a.H ? (g * (1.0f / (1.0f + expf(-g)))) * up : 0.0f;
@@ -333,7 +351,15 @@ __device__ __forceinline__ void down_tile(const DecodeArgs &a, const DecodeBatch
         const int c = u >> 5, r = u & 31;
         if (r0 + r >= a.Dout) continue;
         float y = wave_total<1, NT>(red, NW, 0, r, c);
-        if constexpr (WF8) y = y * a.s2[(long long)e * a.Dout_npad + r0 + r];
+        if constexpr (WF8) {
+            y = y * a.s2[(long long)e * a.Dout_npad + r0 + r];
+        } else if (!__builtin_isfinite(y)) {
+            const uint16_t *h = b.hs + (long long)L.list[j0 + c] * 3 * a.Hpad;
+            y = row_serial((const uint16_t *)a.w2 + (long long)e * a.w2_stride + (long long)(r0 + r) * a.Hpad, a.H,
+                           [&](int k) {
+                               return (bf16_to_f32(h[k + 2 * a.Hpad]) + bf16_to_f32(h[k + a.Hpad])) + bf16_to_f32(h[k]);
+                           });
+        }
         b.y[(long long)L.list[j0 + c] * a.Dout + r0 + r] = y;
     }
 }

@@ -73,3 +73,29 @@ def test_decode_grouped_independent_of_the_batch(moe, oracle, wdtype, n):
         assert np.isnan(o[7]).all()
     finally:
         c.dev.close()
+
+
+@pytest.mark.parametrize("wdtype,T,D,H", [("bf16", 40, 512, 700), ("bf16", 70, 260, 300), ("f32", 40, 512, 700)])
+def test_decode_grouped_infinite_weights(moe, oracle, wdtype, T, D, H):
+    # an infinite weight gives the infinities of its products, as in a single
+    # call, and not the NaN of infinity times a part of x that is 0
+    c = Case(moe, oracle, T=T, D=D, H=H, E=4, k=2, wdtype=wdtype, seed=91, max_tokens=2 * T)
+    try:
+        for e, (name, r, col) in enumerate([("w2", 3, 5), ("w3", 7, 2), ("w2", D - 1, H - 1)]):
+            ex = c.ex[e]
+            ex[name] = ex[name].copy()
+            ex[name][r, col] = np.inf
+            c.dev.set_expert(e, ex["w1"], ex["w2"], ex["w3"])  # fp32 source: bf16 values stay as they are
+        x = np.ascontiguousarray(np.round(c.x * 4) / 4)  # at most 8 bits: the lower parts of x are 0
+        x[x == 0] = 0.25
+        out, logits, idx, _ = c.dev.decode(x)
+        with np.errstate(all="ignore"):
+            ref, ridx, _, _ = oracle.decode_ffn(x, c.wr, c.ex, k=2, logits=logits)
+        assert np.array_equal(idx, ridx)
+        assert np.isinf(ref).any() and np.isfinite(ref).any()
+        assert np.array_equal(np.isnan(out), np.isnan(ref))
+        assert np.array_equal(out[np.isinf(ref)], ref[np.isinf(ref)])
+        ok = np.isfinite(ref)
+        assert rel_err(out[ok], ref[ok]) <= TOL
+    finally:
+        c.dev.close()
