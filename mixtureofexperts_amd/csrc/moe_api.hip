@@ -1713,10 +1713,16 @@ static int decode_wide_route(const moe_handle *h) { return (long long)h->D * h->
 // Whether a decode call of n tokens runs grouped by expert (four launches)
 // instead of token by token (two launches, the routing repeated by every
 // block).  Measured by the multiply-adds of the call's expert products, n kt
-// 3 D H, both ways in us: fp32 / bf16, one token: 13 M 15 / 17, 25 M 23 / 23
-// and 16 / 19, 50 M 52 / 41 and 36 / 28; several: 17 M 14 / 16 and 11 / 16,
-// 25 M 27 / 18 and 25 / 18, 34 M 22 / 17 and 16 / 16; fp8: 8 M 13 / 16, 13 M
-// 19 / 16, 17 M 20 / 16.
+// 3 D H, both ways in us (token by token / grouped).
+// fp32, several tokens: from 28 M on where a row is 320 long or more (26 M 38 /
+// 55, 27 M 53 / 62, 34 M 22 / 17, 72 M 52 / 37); shorter rows are bound by the
+// per-entry reductions, which the groups run in series, up to about 170 M (D
+// 136 to 224: 33 M 33 / 43, 47 M 42 / 60, 119 M 101 / 129, 161 M 143 / 167, 189 M
+// 162 / 139, 223 M 200 / 163).
+// bf16, two to four tokens: few weights are shared (25 M 23 / 28, 39 M 28 / 34,
+// 59 M 33 / 36); more: 25 M 25 / 18, 37 M 33 / 30.
+// One token: fp32 25 M 23 / 23, 50 M 52 / 41; bf16 25 M 16 / 19, 50 M 36 / 28.
+// fp8: 8 M 13 / 16, 13 M 19 / 16, 17 M 20 / 16.
 static bool decode_batched(const moe_handle *h, int n) {
     const int c = std::min(n, kDecodeChunk);
     // workspace: y of every entry; bf16 / fp8: x in the split workspace and h
@@ -1725,7 +1731,11 @@ static bool decode_batched(const moe_handle *h, int n) {
     if (h->wt != WT_F32 && (6LL * c * h->D_pad > 4 * h->split_cap || 3LL * c * h->kt > h->act_rows)) return false;
     if (decode_wide_route(h)) return true;
     const long long mac = (long long)n * h->kt * 3 * h->D * h->H;
-    return mac >= (h->wt == WT_FP8 ? 12000000LL : (n == 1 ? 40000000LL : 24000000LL));
+    if (h->wt == WT_FP8) return mac >= 12000000LL;
+    if (h->wt == WT_F32 && h->D < 320) return mac >= 170000000LL;
+    if (n == 1) return mac >= 40000000LL;
+    if (h->wt == WT_F32) return mac >= 28000000LL;
+    return mac >= (n <= 4 ? 60000000LL : 24000000LL);
 }
 
 static int decode_locked(moe_handle *h, const float *x_dev, int n, float *out_dev, hipStream_t s,

@@ -20,6 +20,7 @@ TOL = 1e-5
 @pytest.mark.parametrize("D,H,Dout,E,k,lsh,n", [
     (512, 1376, 512, 8, 2, 0, 16),   # groups of at most 16
     (260, 300, 90, 2, 1, 0, 130),    # about 32 per group and chunk; sizes off every tile; three chunks, the last of 2
+    (324, 331, 90, 2, 1, 0, 130),    # the same with rows long enough for fp32 to run grouped
     (1000, 700, 40, 5, 2, 1, 65),    # a shared expert that takes whole chunks of 64, then one token
     (200, 330, 200, 3, 3, 0, 41),    # every expert takes all 41 tokens (three column tiles)
     (128, 96, 160, 40, 12, 3, 64),   # 15 slots per token: the index list at its largest but one
