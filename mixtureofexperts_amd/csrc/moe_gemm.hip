@@ -332,6 +332,16 @@ static int f32_ksplit(const GemmArgs &g, int nb) {
 // 1024, 16 rows 132 / 137, 32 rows 219 / 142.
 bool f32x3_rows(int m_tiles_grid, int E) { return 4LL * (m_tiles_grid - E) >= E; }
 
+// ... and layers of 96 tiles of 128 x 128 or more in the larger of their two
+// GEMMs (K here is the other one's columns): fewer leave CUs idle in 128 x 256
+// tiles, with too few stages of K to cut into ranges.  Whole layer,
+// grouped_gemm_kernel / f32x3, us, by those tiles: 20 (171 / 529, 3 experts) 46 /
+// 62, 45 (351 / 176) 82 / 97, 72 (98 / 131, 15 experts) 64 / 69, 98 (117 / 113, 36
+// experts) 95 / 89, 180 (117 / 749) 91 / 77, 290 (107 / 3597) 99 / 77.
+static bool f32x3_tiles(const GemmArgs &g) {
+    return (long long)g.m_tiles_grid * std::max(g.n_tiles, (g.K + 127) / 128) >= 96;
+}
+
 // K ranges of the f32x3 kernel over one workgroup per CU: the S whose rounds
 // of 1 / S tiles end first (the fold as 8 % of a tile), each range of eight
 // stages or more (1001 / 2731 gated, 144 down tiles of 88 stages: S = 3, one
@@ -355,7 +365,7 @@ static int f32x3_ksplit(const GemmArgs &g) {
 hipError_t launch_grouped_gemm_f32(int mode, const GemmArgs &g0, hipStream_t s) {
     if (g0.m_tiles_grid <= 0 || g0.n_tiles <= 0) return hipSuccess;
     GemmArgs g = g0;
-    if (f32x3_rows(g.m_tiles_grid, g.E)) {
+    if (f32x3_rows(g.m_tiles_grid, g.E) && f32x3_tiles(g)) {
         // n_tiles counts 128 output columns; standard and down tiles take 256
         if (mode != MODE_GATED_UP) g.n_tiles = (g.n_tiles + 1) / 2;
         g.ksplit = f32x3_ksplit(g);

@@ -30,10 +30,12 @@ def exact_forward(c, idx, gates):
     return out
 
 
+# each layer has 96 tiles of 128 x 128 or more in one of its GEMMs, from where
+# on the kernel is chosen
 @pytest.mark.parametrize("T,D,H,Dout,E,k,etype,act", [
-    (512, 100, 330, 90, 8, 2, "gated", "silu"),       # partial tiles, pads in every dimension
-    (64, 64, 128, 260, 2, 1, "gated", "gelu"),        # about 32 rows per expert: one row block, two K stages
-    (1000, 330, 260, 512, 3, 2, "standard", "gelu"),  # both row blocks, std tiles of 256 columns, biases
+    (2048, 100, 330, 90, 32, 2, "gated", "silu"),     # partial tiles, pads in every dimension
+    (3072, 64, 128, 260, 96, 1, "gated", "gelu"),     # about 32 rows per expert: one row block, two K stages
+    (4000, 330, 260, 512, 12, 2, "standard", "gelu"),  # both row blocks, std tiles of 256 columns, biases
     (300, 2816, 64, 64, 2, 2, "standard", "relu"),    # a K split of a small tile grid (88 stages)
     (700, 64, 2816, 40, 2, 1, "gated", "identity"),   # ... of the down GEMM
 ])
@@ -52,10 +54,10 @@ def test_f32x3_layer(moe, oracle, T, D, H, Dout, E, k, etype, act):
 
 
 @pytest.mark.parametrize("T,D,H,E,k,etype,act", [
-    (192, 64, 64, 4, 1, "gated", "silu"),       # two stages per sum
-    (128, 128, 256, 4, 2, "standard", "gelu"),
-    (128, 300, 300, 4, 2, "gated", "silu"),     # a partial last stage
-    (600, 480, 448, 3, 2, "gated", "silu"),     # the largest K below the running sums', both row blocks
+    (4608, 64, 64, 96, 1, "gated", "silu"),     # two stages per sum
+    (2048, 128, 256, 64, 2, "standard", "gelu"),
+    (1024, 300, 300, 32, 2, "gated", "silu"),   # a partial last stage
+    (2400, 480, 448, 12, 2, "gated", "silu"),   # the largest K below the running sums', both row blocks
 ])
 def test_f32x3_small_k(moe, oracle, T, D, H, E, k, etype, act):
     # Small K: as accurate as the fp32 matrix unit (2.0e-7, 1.8e-7 and 2.5e-7 on the
@@ -74,13 +76,13 @@ def test_f32x3_small_k(moe, oracle, T, D, H, E, k, etype, act):
         c.dev.close()
 
 
-@pytest.mark.parametrize("H", [96, 2816])
-def test_f32x3_infinities_and_nan(moe, oracle, H):
+@pytest.mark.parametrize("T,H", [(12800, 96), (200, 6400)])
+def test_f32x3_infinities_and_nan(moe, oracle, T, H):
     # values whose parts overflow or are not finite: the outputs they enter
     # are the ones a sequence of fp32 operations gives, the others keep their
     # bits.  Identity experts whose first output columns copy x (w1 = 1 on one
-    # input, w2 = 1 on one unit), the rest random.  H = 2816: K ranges.
-    T, D = 200, 64
+    # input, w2 = 1 on one unit), the rest random.  H = 6400: K ranges.
+    D = 64
     c = Case(moe, oracle, T=T, D=D, H=H, E=2, k=1, gate="switch", expert_type="standard", act="identity", wdtype="f32",
              seed=61, max_tokens=T)
     try:
