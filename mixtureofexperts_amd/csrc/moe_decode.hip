@@ -29,22 +29,6 @@
 
 namespace moe {
 
-// 4 consecutive weights (element offset `o`, a multiple of 4) as fp32
-template <int WT>
-__device__ __forceinline__ float4 load_w4(const void *w, long long o) {
-    if constexpr (WT == WT_F32) {
-        return *(const float4 *)((const float *)w + o);
-    } else if constexpr (WT == WT_BF16) {
-        const uint2 q = *(const uint2 *)((const uint16_t *)w + o);
-        return make_float4(__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xffff0000u), __uint_as_float(q.y << 16),
-                           __uint_as_float(q.y & 0xffff0000u));
-    } else {
-        const uint32_t q = *(const uint32_t *)((const uint8_t *)w + o);
-        return make_float4(fp8e4m3_to_f32((uint8_t)q), fp8e4m3_to_f32((uint8_t)(q >> 8)),
-                           fp8e4m3_to_f32((uint8_t)(q >> 16)), fp8e4m3_to_f32((uint8_t)(q >> 24)));
-    }
-}
-
 // ---- routing of one token by a block of NW waves --------------------------------
 template <int NW>
 struct DecodeRouteLds {

@@ -284,17 +284,36 @@ __device__ __forceinline__ float wave_total(const f32x4_t *red, int nwave, int q
     return s;
 }
 
-// A bf16 weight row with K fp32 values, one after the other: an output whose
-// sum is not finite is recomputed by it.  An infinite weight gives NaN with
-// the zero parts of a finite x (and infinities of both signs with parts of
-// both signs), where the product itself is an infinity.
-template <typename X>
-__device__ __forceinline__ float row_serial(const uint16_t *w, int K, X x) {
-#pragma clang fp contract(off)
+// A bf16 weight row with 4 nch fp32 values (x4(c): chunk c of four), by a whole
+// wave in a single call's arithmetic: an output whose sum is not finite is
+// recomputed by it.  An infinite weight gives NaN with the zero parts of a
+// finite x (and infinities of both signs with parts of both signs), where the
+// product itself is an infinity.  One infinity or NaN in x makes every row of
+// its token's experts such an output, in the same launches as the other
+// tokens, so the row is read in coalesced chunks, eight per lane in flight, up
+// to the first batch that makes it NaN.  Sixteen tokens on a 4096 / 14336
+// layer, us: 515; one of them with a NaN 620, with an infinity 710 (3530 and
+// 4670 by one thread per row and one load per value).
+template <typename X4>
+__device__ __forceinline__ float wave_row_bf16(const uint16_t *w, int nch, X4 x4) {
+    const int lane = threadIdx.x & 63;
     float s = 0.0f;
-#pragma unroll 1
-    for (int k = 0; k < K; ++k) s = s + bf16_to_f32(w[k]) * x(k);
-    return s;
+    for (int c0 = 0; c0 < nch; c0 += 64 * 8) {
+        float4 wv[8], xv[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int c = min(c0 + 64 * u + lane, nch - 1);
+            wv[u] = load_w4<WT_BF16>(w, 4 * c);
+            xv[u] = x4(c);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const bool v = c0 + 64 * u + lane < nch;
+            s = dot4_acc(s, zero_unless(v, wv[u]), zero_unless(v, xv[u]));
+        }
+        if (__any(s != s)) break;  // the row's sum is NaN
+    }
+    return wave_sum(s);
 }
 
 constexpr int kUpWaves = 4;
@@ -308,9 +327,12 @@ __device__ __forceinline__ void up_tile(const DecodeArgs &a, const DecodeBatch &
     const void *img[2] = {b.w1t, b.w3t};
     decode_tile<WF8, 2, kNPadGated, NT, P>(img, a.w1_stride, e, r0, a.Dpad, b.xs, false, a.kt, L, m, j0, kUpWaves, red);
     __syncthreads();
-    // thread: column c, rows 2 rr, 2 rr + 1 (one 4-byte store per part)
-    for (int u = threadIdx.x; u < 16 * min(m - j0, 16 * NT); u += 64 * kUpWaves) {
-        const int c = u >> 4, rr = (u & 15) * 2;
+    // thread: column c, rows 2 rr, 2 rr + 1 (one 4-byte store per part); whole
+    // waves run each pass, for wave_row_bf16
+    const int lane = threadIdx.x & 63, nu = 16 * min(m - j0, 16 * NT);
+    for (int u0 = threadIdx.x - lane; u0 < nu; u0 += 64 * kUpWaves) {
+        const bool on = u0 + lane < nu;
+        const int u = on ? u0 + lane : u0, c = u >> 4, rr = (u & 15) * 2;
         uint32_t part[3] = {0u, 0u, 0u};
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
@@ -320,11 +342,20 @@ __device__ __forceinline__ void up_tile(const DecodeArgs &a, const DecodeBatch &
             if constexpr (WF8) {
                 g = g * a.s1[(long long)e * a.Hpad + r0 + r];
                 up = up * a.s3[(long long)e * a.Hpad + r0 + r];
-            } else if (r0 + r < a.H && !(__builtin_isfinite(g) && __builtin_isfinite(up))) {
-                const float *x = a.x + (long long)(L.list[j0 + c] / a.kt) * a.D;
-                const long long wo = (long long)e * a.w1_stride + (long long)(r0 + r) * a.Dpad;
-                g = row_serial((const uint16_t *)a.w1 + wo, a.D, [&](int k) { return x[k]; });
-                up = row_serial((const uint16_t *)a.w3 + wo, a.D, [&](int k) { return x[k]; });
+            } else {
+                unsigned long long bad =
+                    __ballot(on && r0 + r < a.H && !(__builtin_isfinite(g) && __builtin_isfinite(up)));
+                while (bad) {
+                    const int l = __builtin_ctzll(bad), ub = u0 + l, rb = r0 + (ub & 15) * 2 + k;
+                    bad &= bad - 1;
+                    const float4 *x = (const float4 *)(a.x + (long long)(L.list[j0 + (ub >> 4)] / a.kt) * a.D);
+                    const long long wo = (long long)e * a.w1_stride + (long long)rb * a.Dpad;
+                    auto x4 = [&](int i) { return x[i]; };
+                    const float gb = wave_row_bf16((const uint16_t *)a.w1 + wo, a.D >> 2, x4);
+                    const float vb = wave_row_bf16((const uint16_t *)a.w3 + wo, a.D >> 2, x4);
+                    g = lane == l ? gb : g;
+                    up = lane == l ? vb : up;
+                }
             }
             // pad rows: 0 whatever x holds
             const float h = r0 + r < a.H ? (g * (1.0f / (1.0f + expf(-g)))) * up : 0.0f;
@@ -333,6 +364,7 @@ __device__ __forceinline__ void up_tile(const DecodeArgs &a, const DecodeBatch &
 #pragma unroll
             for (int q = 0; q < 3; ++q) part[q] |= (uint32_t)p3[q] << (16 * k);
         }
+        if (!on) continue;
         uint16_t *dst = b.hs + (long long)L.list[j0 + c] * 3 * a.Hpad + r0 + rr;
 #pragma unroll
         for (int q = 0; q < 3; ++q) *(uint32_t *)(dst + (long long)q * a.Hpad) = part[q];
@@ -347,20 +379,30 @@ __device__ __forceinline__ void down_tile(const DecodeArgs &a, const DecodeBatch
     const void *img[1] = {b.w2t};
     decode_tile<WF8, 1, kNPad, NT, P>(img, a.w2_stride, e, r0, a.Hpad, b.hs, true, a.kt, L, m, j0, NW, red);
     __syncthreads();
-    for (int u = threadIdx.x; u < 32 * min(m - j0, 16 * NT); u += 64 * NW) {
-        const int c = u >> 5, r = u & 31;
-        if (r0 + r >= a.Dout) continue;
+    const int lane = threadIdx.x & 63, nu = 32 * min(m - j0, 16 * NT);
+    for (int u0 = threadIdx.x - lane; u0 < nu; u0 += 64 * NW) {  // whole waves, for wave_row_bf16
+        const int u = min(u0 + lane, nu - 1), c = u >> 5, r = u & 31;
+        const bool on = u0 + lane < nu && r0 + r < a.Dout;
         float y = wave_total<1, NT>(red, NW, 0, r, c);
         if constexpr (WF8) {
             y = y * a.s2[(long long)e * a.Dout_npad + r0 + r];
-        } else if (!__builtin_isfinite(y)) {
-            const uint16_t *h = b.hs + (long long)L.list[j0 + c] * 3 * a.Hpad;
-            y = row_serial((const uint16_t *)a.w2 + (long long)e * a.w2_stride + (long long)(r0 + r) * a.Hpad, a.H,
-                           [&](int k) {
-                               return (bf16_to_f32(h[k + 2 * a.Hpad]) + bf16_to_f32(h[k + a.Hpad])) + bf16_to_f32(h[k]);
-                           });
+        } else {
+            unsigned long long bad = __ballot(on && !__builtin_isfinite(y));
+            while (bad) {
+                const int l = __builtin_ctzll(bad), ub = u0 + l;
+                bad &= bad - 1;
+                const uint16_t *h = b.hs + (long long)L.list[j0 + (ub >> 5)] * 3 * a.Hpad;
+                auto h4 = [&](int i) {
+                    const float4 p0 = load_w4<WT_BF16>(h, 4 * i), p1 = load_w4<WT_BF16>(h, a.Hpad + 4 * i),
+                                 p2 = load_w4<WT_BF16>(h, 2 * a.Hpad + 4 * i);
+                    return make_float4((p2.x + p1.x) + p0.x, (p2.y + p1.y) + p0.y, (p2.z + p1.z) + p0.z, (p2.w + p1.w) + p0.w);
+                };
+                const float yb = wave_row_bf16((const uint16_t *)a.w2 + (long long)e * a.w2_stride +
+                                                   (long long)(r0 + (ub & 31)) * a.Hpad, a.Hpad >> 2, h4);
+                y = lane == l ? yb : y;
+            }
         }
-        b.y[(long long)L.list[j0 + c] * a.Dout + r0 + r] = y;
+        if (on) b.y[(long long)L.list[j0 + c] * a.Dout + r0 + r] = y;
     }
 }
 

@@ -100,3 +100,38 @@ def test_decode_grouped_infinite_weights(moe, oracle, wdtype, T, D, H):
         assert rel_err(out[ok], ref[ok]) <= TOL
     finally:
         c.dev.close()
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, 3.4e38])
+def test_decode_grouped_is_not_held_up_by_one_token(moe, oracle, value):
+    # one token whose every product is not finite: the other tokens' results
+    # keep their bits and the call its time.  That token's rows (2 x 4096 of
+    # 4096 values, 4096 of 4096) are 100 MB of reads that the L2 and Infinity
+    # Cache hold, about the call's own: 1.3 to 2.2 x the time; one thread per row
+    # with one load per value took 16 x (4 x for the large finite value)
+    import time
+
+    c = Case(moe, oracle, T=16, D=4096, H=4096, E=2, k=1, gate="switch", wdtype="bf16", seed=93, max_tokens=32)
+    try:
+        print(f"grouped decode, one token with {value}", flush=True)
+        x = np.ascontiguousarray(c.x)
+        bad = x.copy()
+        bad[3, 17] = value
+
+        def fastest(a):
+            best = 1e9
+            for _ in range(8):
+                t0 = time.perf_counter()
+                c.dev.decode(a)
+                best = min(best, time.perf_counter() - t0)
+            return best
+
+        out, o = c.dev.decode(x)[0], c.dev.decode(bad)[0]
+        keep = np.arange(16) != 3
+        assert np.array_equal(o[keep].view(np.uint32), out[keep].view(np.uint32))
+        assert not np.isfinite(o[3]).all()
+        clean, held = fastest(x), fastest(bad)
+        print(f"{clean * 1e6:.0f} us, {held * 1e6:.0f} us", flush=True)
+        assert held <= 4 * clean, (clean, held)
+    finally:
+        c.dev.close()
