@@ -35,8 +35,8 @@
 // ((r >> 2) & 3), as in the bf16 kernel.
 //
 // Infinities, NaN and values that round up to an infinity: their parts give
-// NaN or infinite sums, and every output that is not finite is recomputed
-// from the fp32 operands, one K value after the other.
+// NaN or infinite sums, and a wave that holds such a sum takes it from fp32
+// MFMAs over the fp32 operands (redo).
 //
 // STAGE_SUMS: the six products of a stage start from zero, the smallest first,
 // and are added to the running sum with one rounded addition.  The matrix unit
@@ -247,12 +247,57 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // first column of the lane in column block j (gated: of h, from blocks 2 j and 2 j + 1)
     auto col_of = [&](int j) { return wn * (NB == 2 ? 32 : 64) + j * 16 + 4 * q4; };
     constexpr int NJ = 4 / NB;
+
+    // redo: the wave's 64 x 64 sums on v_mfma_f32_16x16x4_f32, operands straight
+    // from memory; those that were not finite are replaced.  It takes about
+    // four times the tile's own MFMAs and runs for whole waves, whatever the
+    // number of such sums: 768 / 3072 standard, 4096 tokens, us a call: 545; with
+    // an infinity in one row 945, in every row 1300 (1720 and 46070 by one lane
+    // per output and one K value after the other).
+    bool fin = true;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) fin = fin && (__builtin_isfinite(acc[i][j][c]) || row_of(i) >= rows);
+    if (__any(!fin)) {
+        const float *ap[4], *bp[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ap[i] = A + (arow0 + min(row_of(i), rows - 1)) * g.lda + 4 * q4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            bp[j] = NB == 2 ? ((j & 1) ? B1 : B0) + (long long)(wn * 32 + (j >> 1) * 16 + r16) * g.ldb + 4 * q4
+                            : B0 + (long long)(wn * 64 + j * 16 + r16) * g.ldb + 4 * q4;
+        f32x4_t sum[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (int k = kb * 32; k < ke * 32; k += 16) {  // lane (r16, q4): K k + 4 q4 .. + 3 of its rows
+            f32x4_t av[4], bv[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) av[i] = *(const f32x4_t *)(ap[i] + k);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) bv[j] = *(const f32x4_t *)(bp[j] + k);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j][t], av[i][t], sum[i][j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[i][j][c] = __builtin_isfinite(acc[i][j][c]) ? acc[i][j][c] : sum[i][j][c];
+    }
+
     float *ws = S > 1 ? g.split_ws + ((long long)(mt * g.n_tiles + nt) * S + ks) * (BM * BR) : nullptr;
-    unsigned long long bad = 0;  // outputs with a sum that is not finite: bit (j 4 + i) 4 + c
-    auto check = [&](int j, int i, int c, float v0, float v1) {
-        const bool fin = __builtin_isfinite(v0) && (NB == 1 || __builtin_isfinite(v1));
-        if (!fin && row_of(i) < rows) bad |= 1ull << ((j * 4 + i) * 4 + c);
-    };
     const bool vec4 = (g.ldc & 3) == 0;
     // the activation is picked once per tile (picked per output, it was a
     // branch and a wait for each of a lane's 64 outputs)
@@ -271,7 +316,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     const float v0 = acc[i][NB == 2 ? 2 * j : j][c], v1 = acc[i][NB == 2 ? 2 * j + 1 : j][c];
-                    check(j, i, c, v0, v1);
                     v[c] = out(arow0 + row_of(i), n + c, bias[c], v0, v1);
                 }
                 if (row_of(i) >= rows) continue;
@@ -308,8 +352,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 if (row_of(i) >= rows) continue;
 #pragma unroll
                 for (int b = 0; b < NB; ++b) *(f32x4_t *)(ws + (b * BM + row_of(i)) * BN + col_of(j)) = acc[i][NB * j + b];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) check(j, i, c, acc[i][NB * j][c], acc[i][NB * j + NB - 1][c]);
             }
     } else if constexpr (MODE == MODE_DOWN) {
         tile_act(std::integral_constant<int, MOE_ACT_IDENTITY>{});
@@ -320,26 +362,5 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         case MOE_ACT_RELU: tile_act(std::integral_constant<int, MOE_ACT_RELU>{}); break;
         default: tile_act(std::integral_constant<int, MOE_ACT_IDENTITY>{});
         }
-    }
-    while (bad) {  // once more from the fp32 rows, one K value after the other; NaN ends a sum
-        const int u = __builtin_ctzll(bad);
-        bad &= bad - 1;
-        const int ml = row_of((u >> 2) & 3), nl = col_of(u >> 4) + (u & 3), n = n0 + nl;
-        const float *ar = A + (arow0 + ml) * g.lda, *w0 = B0 + (long long)nl * g.ldb, *w1 = B1 + (long long)nl * g.ldb;
-        float v0 = 0.0f, v1 = 0.0f;
-        for (int k = kb * 32; k < ke * 32 && v0 == v0; ++k) v0 = fmaf(ar[k], w0[k], v0);
-        if (NB == 2)
-            for (int k = kb * 32; k < ke * 32 && v1 == v1; ++k) v1 = fmaf(ar[k], w1[k], v1);
-        if (S > 1) {
-            ws[ml * BN + nl] = v0;
-            if (NB == 2) ws[(BM + ml) * BN + nl] = v1;
-            continue;
-        }
-        if (n >= g.N) continue;
-        float v = v0 + ((MODE != MODE_GATED_UP && g.bias) ? g.bias[sofs + n] : 0.0f);
-        if (MODE != MODE_DOWN) v = act_apply(g.act, v);
-        if (MODE == MODE_GATED_UP) v = v * v1;
-        if (MODE == MODE_STD_UP) v = dropout_h(g, arow0 + ml, n, v);
-        ((float *)g.C)[(arow0 + ml) * g.ldc + n] = v;
     }
 }

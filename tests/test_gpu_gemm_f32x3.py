@@ -116,3 +116,46 @@ def test_f32x3_infinities_and_nan(moe, oracle, T, H):
         assert np.array_equal(o[keep], x[keep])
     finally:
         c.dev.close()
+
+
+@pytest.mark.parametrize("etype,H", [("standard", 4096), ("gated", 2048)])
+def test_f32x3_calls_with_infinities_take_their_time(moe, oracle, etype, H):
+    # positive weights, so that an infinity in x is one in every output of
+    # its row; in one row and in all of them.  Redone sums take about four
+    # times a tile's own MFMAs, a part of this host call: 1.4 x its time; one
+    # lane per output and one K value after the other took 5 x with one such
+    # row, 28 and 38 x with all
+    import time
+
+    T, D = 512, 512
+    c = Case(moe, oracle, T=T, D=D, H=H, E=2, k=1, gate="switch", expert_type=etype, act="identity", wdtype="f32", seed=63)
+    try:
+        print(f"f32x3 calls with infinities {etype} H={H}", flush=True)
+        for e in range(2):
+            w = c.ex[e]
+            c.dev.set_expert(e, np.abs(w["w1"]), np.abs(w["w2"]), None if w["w3"] is None else np.abs(w["w3"]), w["b1"], w["b2"])
+
+        def forward(x):
+            return c.dev.forward_routed(x, 0, False, 1 + np.arange(T, dtype=np.int32)[:, None] % 2, np.ones((T, 1), np.float32))[0]
+
+        def fastest(x):
+            best = 1e9
+            for _ in range(6):
+                t0 = time.perf_counter()
+                forward(x)
+                best = min(best, time.perf_counter() - t0)
+            return best
+
+        x = np.ascontiguousarray(c.x)
+        out, clean = forward(x), fastest(x)
+        one, every = x.copy(), x.copy()
+        one[5, 300], every[:, 300] = np.inf, np.inf
+        for bad in (one, every):
+            o, held = forward(bad), fastest(bad)
+            rows = np.isinf(bad).any(axis=1)
+            assert np.array_equal(o[~rows].view(np.uint32), out[~rows].view(np.uint32))
+            assert np.all(o[rows] == np.inf)
+            print(f"{rows.sum()} rows: {clean * 1e6:.0f} us, {held * 1e6:.0f} us", flush=True)
+            assert held <= 5 * clean, (clean, held)
+    finally:
+        c.dev.close()
