@@ -596,10 +596,15 @@ static long long call_rows(const moe_handle *h, int T) {
     return std::min(rows, (long long)h->rows_max);
 }
 
-static int m_tiles_for(const moe_handle *h, int T) {
-    long long mt = (long long)T * h->kc / h->bm + h->E;
-    if (mt > h->max_tiles) mt = h->max_tiles;
-    return (int)mt;
+// What a call's expert GEMMs run over: its rows, at most, the experts that
+// hold them, and its M tiles, at most.
+struct ExpertRows {
+    long long rows;
+    int experts, m_tiles;
+};
+static ExpertRows expert_rows(const moe_handle *h, int T) {
+    const long long rows = call_rows(h, T);
+    return {rows, h->E, (int)std::min<long long>(rows / h->bm + h->E, h->max_tiles)};
 }
 
 enum { PERMUTE_NONE = 0, PERMUTE_INDEX = 1, PERMUTE_ROWS = 2 };
@@ -745,7 +750,7 @@ static int run_routing(moe_handle *h, const void *x_dev, int x_bf16, int T, int 
     return MOE_OK;
 }
 
-static GemmArgs up_args(moe_handle *h, int mt_grid, bool training) {
+static GemmArgs up_args(moe_handle *h, const ExpertRows &er, bool training) {
     GemmArgs g{};
     if (training && !h->gated && h->drop_p > 0.0f) {
         // Dropout(p) on h in training (src/experts/standard.jl:49-51), one
@@ -771,7 +776,7 @@ static GemmArgs up_args(moe_handle *h, int mt_grid, bool training) {
     // round, folded by fold_up_kernel
     g.ksplit = (h->bf16_gemm && h->split_ws && h->bm == 256) ? kUpSplitMax : 1;
     g.ncu = h->bf16_gemm ? gemm_slots(h) : h->ncu; g.split_ws = h->split_ws; g.split_cap = h->split_cap;
-    g.m_tiles_grid = mt_grid; g.act = h->cfg.activation;
+    g.m_tiles_grid = er.m_tiles; g.rows = er.rows; g.experts = er.experts; g.act = h->cfg.activation;
     // bf16 kernel: 128 h columns (gated, W1 and W3 rows) or 256 rows per tile
     g.n_tiles = up_ntiles(h);
     return g;
@@ -783,7 +788,7 @@ static GemmArgs up_args(moe_handle *h, int mt_grid, bool training) {
 static int down_ksplit(const moe_handle *h) { return h->bf16_gemm ? kDownSplitMax : 1; }
 
 
-static GemmArgs down_args(moe_handle *h, int mt_grid, int ksplit, bool y_f32) {
+static GemmArgs down_args(moe_handle *h, const ExpertRows &er, int ksplit, bool y_f32) {
     GemmArgs g{};
     g.A = h->hbuf; g.lda = h->H_pad;
     g.B0 = h->bf16_gemm ? h->w2t : h->w2; g.B1 = nullptr;
@@ -795,37 +800,37 @@ static GemmArgs down_args(moe_handle *h, int mt_grid, int ksplit, bool y_f32) {
     g.split_ws = h->split_ws; g.split_cap = h->split_cap;
     g.tiles = h->tiles; g.num_tiles = h->num_tiles; g.counts = h->counts; g.offsets = h->offsets;
     g.tile_start = h->tile_start; g.E = h->E;
-    g.m_tiles_grid = mt_grid; g.act = h->cfg.activation;
+    g.m_tiles_grid = er.m_tiles; g.rows = er.rows; g.experts = er.experts; g.act = h->cfg.activation;
     g.n_tiles = h->bf16_gemm ? h->Dout_npad / 256 : h->Dout_npad / kGemmBN;
     return g;
 }
 
 // The expert up GEMM (W1/W3 or W1 + activation) and the down GEMM (W2) over
-// mt_grid M tiles: the LDS-DMA kernel for bf16 and fp8 weights (bf16
+// a call's rows: the LDS-DMA kernel for bf16 and fp8 weights (bf16
 // activations), the register-staged fp32 kernel for fp32 weights.
-static hipError_t launch_up(moe_handle *h, int mt_grid, hipStream_t s, bool training = false) {
+static hipError_t launch_up(moe_handle *h, const ExpertRows &er, hipStream_t s, bool training = false) {
     const int mode = h->gated ? MODE_GATED_UP : MODE_STD_UP;
-    const GemmArgs g = up_args(h, mt_grid, training);
+    const GemmArgs g = up_args(h, er, training);
     if (h->bf16_gemm) return launch_grouped_gemm_bf16(mode, h->bm, h->wt == WT_FP8, g, s);
     return launch_grouped_gemm_f32(mode, g, s);
 }
 
 // y_f32: write y in fp32 also on the bf16-kernel path (moe_expert_forward
 // hands y back as fp32); the layer paths keep it in bf16 there.
-static hipError_t launch_down(moe_handle *h, int mt_grid, hipStream_t s, int ksplit, bool y_f32 = false) {
+static hipError_t launch_down(moe_handle *h, const ExpertRows &er, hipStream_t s, int ksplit, bool y_f32 = false) {
     if (h->bf16_gemm) {
-        const GemmArgs g = down_args(h, mt_grid, ksplit, y_f32);
+        const GemmArgs g = down_args(h, er, ksplit, y_f32);
         hipError_t e = launch_grouped_gemm_bf16(MODE_DOWN, h->bm, h->wt == WT_FP8, g, s);
         if (e == hipSuccess && ksplit > 1) e = launch_fold_split(h->bm, g, s);
         return e;
     }
-    return launch_grouped_gemm_f32(MODE_DOWN, down_args(h, mt_grid, 1, true), s);
+    return launch_grouped_gemm_f32(MODE_DOWN, down_args(h, er, 1, true), s);
 }
 
 static int run_experts(moe_handle *h, int T, int training, hipStream_t s) {
-    const int mt = m_tiles_for(h, T);
-    HIP_TRY(h, launch_up(h, mt, s, training != 0));
-    HIP_TRY(h, launch_down(h, mt, s, down_ksplit(h)));
+    const ExpertRows er = expert_rows(h, T);
+    HIP_TRY(h, launch_up(h, er, s, training != 0));
+    HIP_TRY(h, launch_down(h, er, s, down_ksplit(h)));
     return MOE_OK;
 }
 
@@ -1075,7 +1080,7 @@ int moe_create(const moe_config *cfg, moe_handle **out) {
     // workgroups per CU of 128 x 128 floats, of 128 x 256 where the handle's
     // batches reach the f32x3 kernel
     h->split_cap = h->bf16_gemm ? (long long)h->ncu * 256 * 256
-                                : 2LL * h->ncu * kGemmBM * kGemmBN * (f32x3_rows(h->max_tiles - 1, h->E) ? 2 : 1);
+                                : 2LL * h->ncu * kGemmBM * kGemmBN * (f32x3_rows(h->rows_max, h->E) ? 2 : 1);
     A((void **)&h->split_ws, sizeof(float) * (size_t)h->split_cap);
     if (r != MOE_OK) return cleanup(r);
     // Pads of the packed weights and of the activation rows must read as 0.
@@ -1669,8 +1674,9 @@ int moe_expert_forward(moe_handle *h, int32_t expert, const float *x, int32_t n,
                            h->xp, h->D_pad, h->bf16_gemm ? h->bm : 0);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = launch_up(h, nt, s);
-    if (e == hipSuccess) e = launch_down(h, nt, s, 1, true);
+    const ExpertRows er{n, 1, nt};
+    if (e == hipSuccess) e = launch_up(h, er, s);
+    if (e == hipSuccess) e = launch_down(h, er, s, 1, true);
     if (e == hipSuccess)
         e = hipMemcpy2DAsync(y, sizeof(float) * h->Dout, h->y, sizeof(float) * (size_t)h->ld_y,
                              sizeof(float) * h->Dout, n, hipMemcpyDeviceToHost, s);
@@ -1879,7 +1885,7 @@ int moe_stage_expert_up_async(moe_handle *h, int32_t T, void *stream) {
     hipStream_t s = stream ? (hipStream_t)stream : h->stream;
     r = join_stream(h, s);
     if (r != MOE_OK) return r;
-    HIP_TRY(h, launch_up(h, m_tiles_for(h, T), s, h->last_training != 0));
+    HIP_TRY(h, launch_up(h, expert_rows(h, T), s, h->last_training != 0));
     return mark_stream(h, s);
 }
 
@@ -1891,7 +1897,7 @@ int moe_stage_expert_down_async(moe_handle *h, int32_t T, void *stream) {
     hipStream_t s = stream ? (hipStream_t)stream : h->stream;
     r = join_stream(h, s);
     if (r != MOE_OK) return r;
-    HIP_TRY(h, launch_down(h, m_tiles_for(h, T), s, down_ksplit(h)));
+    HIP_TRY(h, launch_down(h, expert_rows(h, T), s, down_ksplit(h)));
     return mark_stream(h, s);
 }
 

@@ -2,7 +2,7 @@
 #pragma once
 
 namespace moe {
-// Whether an fp32 call over m_tiles_grid M tiles (its rows / 128 + E) runs on
-// the bf16 matrix unit (moe_gemm_f32x3.h).
-bool f32x3_rows(int m_tiles_grid, int E);
+// Whether an fp32 call's expert segments are long enough for the bf16 matrix
+// unit (moe_gemm_f32x3.h): at most `rows` rows that `experts` experts hold.
+bool f32x3_rows(long long rows, int experts);
 }  // namespace moe

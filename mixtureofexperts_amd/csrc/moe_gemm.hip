@@ -330,7 +330,7 @@ static int f32_ksplit(const GemmArgs &g, int nb) {
 // grouped_gemm_kernel / f32x3, us: 1024 / 4096 gated, 16 rows 127 / 125, 32 rows 206 /
 // 128; 768 / 3072 standard, 16 rows 64 / 68, 32 rows 94 / 63; 64 experts of 512 /
 // 1024, 16 rows 132 / 137, 32 rows 219 / 142.
-bool f32x3_rows(int m_tiles_grid, int E) { return 4LL * (m_tiles_grid - E) >= E; }
+bool f32x3_rows(long long rows, int experts) { return rows >= 32LL * experts; }
 
 // ... and layers of 96 tiles of 128 x 128 or more in the larger of their two
 // GEMMs (K here is the other one's columns): fewer leave CUs idle in 128 x 256
@@ -365,7 +365,7 @@ static int f32x3_ksplit(const GemmArgs &g) {
 hipError_t launch_grouped_gemm_f32(int mode, const GemmArgs &g0, hipStream_t s) {
     if (g0.m_tiles_grid <= 0 || g0.n_tiles <= 0) return hipSuccess;
     GemmArgs g = g0;
-    if (f32x3_rows(g.m_tiles_grid, g.E) && f32x3_tiles(g)) {
+    if (f32x3_rows(g.rows, g.experts) && f32x3_tiles(g)) {
         // n_tiles counts 128 output columns; standard and down tiles take 256
         if (mode != MODE_GATED_UP) g.n_tiles = (g.n_tiles + 1) / 2;
         g.ksplit = f32x3_ksplit(g);

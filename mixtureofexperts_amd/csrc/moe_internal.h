@@ -284,7 +284,8 @@ struct GemmArgs {
     const int *tile_start;               // [E+1] (bf16 kernel work list)
     const int *item_start;               // [E+1] or null: the up GEMM's paired items (256-row tiles, n_tiles even)
     int E;
-    int m_tiles_grid; int n_tiles;
+    int m_tiles_grid; int n_tiles;       // at most this many M tiles
+    long long rows; int experts;         // expert rows of the call, at most, and the experts that hold them
     int ksplit;                          // bf16 kernel: the most K ranges a tail tile may be split into (tail_split)
     int ncu;                             // workgroup slots of one round (CUs x workgroups per CU)
     float *split_ws;                     // partials of split tiles (ksplit > 1)

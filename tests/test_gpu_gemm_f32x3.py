@@ -53,6 +53,40 @@ def test_f32x3_layer(moe, oracle, T, D, H, Dout, E, k, etype, act):
         c.dev.close()
 
 
+def test_fp32_kernel_follows_the_calls_rows(moe, oracle):
+    # ExpertChoice: the slots a token may hold grow with the handle's
+    # max_tokens, the rows of a call do not.  64 tokens choose 4 rows per expert,
+    # far below the 32 from which on the bf16 matrix unit takes an fp32 layer;
+    # on a handle for 2048 tokens the call has the bits it has on one for 64
+    outs = []
+    for cap in (64, 2048):
+        c = Case(moe, oracle, T=64, D=256, H=512, E=32, k=2, gate="expert_choice", gate_param=2.0, wdtype="f32", seed=71,
+                 max_tokens=cap)
+        try:
+            out, _, res = c.run(training=True)
+            assert res["counts"].max() <= 4
+            outs.append(out)
+        finally:
+            c.dev.close()
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
+def test_expert_forward_takes_the_layers_kernel(moe, oracle):
+    # one expert's rows are as long a segment for moe_expert_forward as in a
+    # layer call that gives them all to that expert: the same bits (at sizes
+    # where the layer grid's further M tiles change no K split)
+    T, D = 1000, 260
+    c = Case(moe, oracle, T=T, D=D, H=4096, Dout=40, E=12, k=1, gate="switch", wdtype="f32", seed=72)
+    try:
+        print("expert_forward against the layer", flush=True)
+        x = np.ascontiguousarray(c.x)
+        out = c.dev.forward_routed(x, 0, False, np.full((T, 1), 2, np.int32), np.ones((T, 1), np.float32))[0]
+        y = c.dev.expert_forward(1, x)
+        assert np.array_equal(y.view(np.uint32), out.view(np.uint32))
+    finally:
+        c.dev.close()
+
+
 @pytest.mark.parametrize("T,D,H,E,k,etype,act", [
     (4608, 64, 64, 96, 1, "gated", "silu"),     # two stages per sum
     (2048, 128, 256, 64, 2, "standard", "gelu"),
