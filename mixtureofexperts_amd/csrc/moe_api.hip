@@ -1718,17 +1718,35 @@ static int decode_wide_route(const moe_handle *h) { return (long long)h->D * h->
 
 // Whether a decode call of n tokens runs grouped by expert (four launches)
 // instead of token by token (two launches, the routing repeated by every
-// block).  Measured by the multiply-adds of the call's expert products, n kt
-// 3 D H, both ways in us (token by token / grouped).
-// fp32, several tokens: from 28 M on where a row is 320 long or more (26 M 38 /
-// 55, 27 M 53 / 62, 34 M 22 / 17, 72 M 52 / 37); shorter rows are bound by the
-// per-entry reductions, which the groups run in series, up to about 170 M (D
-// 136 to 224: 33 M 33 / 43, 47 M 42 / 60, 119 M 101 / 129, 161 M 143 / 167, 189 M
-// 162 / 139, 223 M 200 / 163).
-// bf16, two to four tokens: few weights are shared (25 M 23 / 28, 39 M 28 / 34,
-// 59 M 33 / 36); more: 25 M 25 / 18, 37 M 33 / 30.
-// One token: fp32 25 M 23 / 23, 50 M 52 / 41; bf16 25 M 16 / 19, 50 M 36 / 28.
-// fp8: 8 M 13 / 16, 13 M 19 / 16, 17 M 20 / 16.
+// block).  us below: token by token / grouped, five rounds of each in turn over
+// three handles; a side's rounds differ by 1 to 3 %.  M: the multiply-adds of
+// the call's expert products, n kt 3 D H; router: D x its experts, which every
+// block reads token by token.
+//
+// fp32 (same bits either way), several tokens: by the weights that grouping
+// does not read again, i.e. the M of the entries past the n tokens' expected
+// number of experts.  Rows of 1024 values or more: 4 M (1024 / 2816 of 8: 2 tokens
+// 34 / 36, 3 tokens = 12 M 46 / 45; 2048 / 700, 4 of 16, 2 tokens = 4 M 51 / 48).
+// From 448 on: 18 M (512 / 1376 of 8: 6 tokens 25 / 26, 8 tokens = 19 M 28 / 28 and, on
+// one handle whose weights the Infinity Cache keeps, 19 / 16 to 19; 16 tokens =
+// 53 M 45 / 34; 500 / 665 of 73: 16 tokens = 6 M 54 / 65, 32 tokens = 21 M
+// 77 / 77).  Shorter rows are bound by the per-entry reductions, which a group
+// runs in series, up to a call's 170 M (320 / 600 of 8, 64 tokens = 74 M 44 / 46;
+// 384 / 1536, 6 of 64: 85 M 74 / 75, 170 M 119 / 104; 136 / 1000, 4 of 32, 104 M 95 /
+// 92; 200 / 2000 of 16, 154 M 100 / 92).
+// fp32, one token: 64 M (1024 / 8192 = 50 M 47 / 52, 2048 / 5504 = 68 M 69 / 67), 40 M
+// with a router of more than 48 K (2048 / 1408, 6 of 30 = 52 M 87 / 77).
+//
+// bf16, up to four tokens: 140 M (1024 / 8192: 1 token = 50 M 33 / 48, 2 tokens = 101 M
+// 51 / 63, 3 tokens = 151 M 68 / 70; 2048 / 5504: 1 token = 68 M 48 / 57, 2 tokens =
+// 135 M 69 / 76, 3 tokens = 203 M 93 / 90), 60 M with a router of 32 K (2048 / 768, 4
+// of 16, 4 tokens = 75 M 59 / 51; 4096 / 4096 of 8, 1 token = 101 M 74 / 74, 2 tokens
+// 105 / 105), 40 M above 48 K (2048 / 1408, 6 of 30, 1 token = 52 M 68 / 60).
+// More tokens: 40 M (512 / 1376: 8 tokens = 34 M 21 / 24, 16 tokens = 67 M 32 / 25;
+// 768 / 2048: 6 tokens = 57 M 28 / 27; 4096 / 300: 6 tokens = 44 M 55 / 48).
+// fp8: 7.2 M (512 / 768: 3 tokens = 7.1 M 16 / 18; 4096 / 300: 1 token = 7.4 M 50 / 34;
+// 512 / 1376: 1 token = 4 M 15 / 17, 2 tokens = 8 M 20 / 18; 256 / 704 of 16, 8 tokens =
+// 9 M 19 / 19).
 static bool decode_batched(const moe_handle *h, int n) {
     const int c = std::min(n, kDecodeChunk);
     // workspace: y of every entry; bf16 / fp8: x in the split workspace and h
@@ -1736,12 +1754,17 @@ static bool decode_batched(const moe_handle *h, int n) {
     if ((long long)c * h->kt * h->Dout > (long long)h->rows_max * h->ld_y) return false;
     if (h->wt != WT_F32 && (6LL * c * h->D_pad > 4 * h->split_cap || 3LL * c * h->kt > h->act_rows)) return false;
     if (decode_wide_route(h)) return true;
-    const long long mac = (long long)n * h->kt * 3 * h->D * h->H;
-    if (h->wt == WT_FP8) return mac >= 12000000LL;
-    if (h->wt == WT_F32 && h->D < 320) return mac >= 170000000LL;
-    if (n == 1) return mac >= 40000000LL;
-    if (h->wt == WT_F32) return mac >= 28000000LL;
-    return mac >= (n <= 4 ? 60000000LL : 24000000LL);
+    const long long mac1 = 3LL * h->D * h->H, mac = n * h->kt * mac1, router = (long long)h->D * h->Er_pad;
+    if (h->wt == WT_FP8) return mac >= 7200000LL;
+    if (h->wt == WT_BF16) {
+        if (n > 4) return mac >= 40000000LL;
+        return mac >= (router > 48 * 1024 ? 40000000LL : router >= 32 * 1024 ? 60000000LL : 140000000LL);
+    }
+    if (n == 1) return mac >= (router > 48 * 1024 ? 40000000LL : 64000000LL);
+    if (h->D < 448) return mac >= 170000000LL;
+    // the routed experts that n tokens of k pick, loads being even
+    const double experts = h->Er * (1.0 - std::pow(1.0 - (double)h->k / h->Er, n)) + h->lsh;
+    return (n * h->kt - experts) * mac1 >= (h->D >= 1024 ? 4e6 : 18e6);
 }
 
 static int decode_locked(moe_handle *h, const float *x_dev, int n, float *out_dev, hipStream_t s,

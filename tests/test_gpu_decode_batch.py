@@ -9,6 +9,7 @@ sqrt(K) 2^-24 = 3e-6 of each other."""
 import numpy as np
 import pytest
 
+from kernel_names import kernels_of
 from test_gpu_layer import Case, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -24,6 +25,10 @@ TOL = 1e-5
     (1000, 700, 40, 5, 2, 1, 65),    # a shared expert that takes whole chunks of 64, then one token
     (200, 330, 200, 3, 3, 0, 41),    # every expert takes all 41 tokens (three column tiles)
     (128, 96, 160, 40, 12, 3, 64),   # 15 slots per token: the index list at its largest but one
+    # the second to sixth again with rows long enough for bf16 and fp32 to run grouped too
+    (452, 331, 90, 2, 1, 0, 130),
+    (456, 700, 200, 3, 3, 0, 41),
+    (448, 300, 160, 40, 12, 3, 64),
     (2048, 64, 64, 40, 2, 0, 1),     # the 16-wave router, one token
     (2048, 128, 72, 300, 8, 0, 5),   # ... with eight experts per lane, most experts idle
 ])
@@ -47,6 +52,31 @@ def test_decode_grouped(moe, oracle, wdtype, D, H, Dout, E, k, lsh, n):
             c.dev.decode(x)
             f2 = c.run(training=False)[0]
             assert np.array_equal(f1.view(np.uint32), f2.view(np.uint32))
+    finally:
+        c.dev.close()
+
+
+@pytest.mark.parametrize("wdtype,D,H,E,k,n,grouped", [
+    # measured us of both ways beside each line of the rule; here one call on either side of it
+    ("f32", 512, 1376, 8, 2, 6, False), ("f32", 512, 1376, 8, 2, 8, True),   # rows of 448 values or more: 18 M saved
+    ("f32", 500, 665, 73, 2, 16, False),                                      # few tokens share an expert of 73
+    ("f32", 1024, 704, 16, 4, 2, False), ("f32", 1024, 704, 16, 4, 6, True),  # rows of 1024: 4 M saved
+    ("f32", 320, 600, 8, 2, 64, False), ("f32", 320, 1408, 8, 2, 64, True),   # short rows: a call's 170 M
+    ("f32", 2048, 4160, 2, 2, 1, False), ("f32", 2048, 5504, 2, 2, 1, True),  # one token: 64 M
+    ("bf16", 1024, 8192, 2, 2, 1, False), ("bf16", 1024, 8192, 2, 2, 3, True),
+    ("bf16", 512, 1376, 8, 2, 8, False), ("bf16", 512, 1376, 8, 2, 16, True),
+    ("fp8", 512, 1376, 8, 2, 1, False), ("fp8", 512, 1376, 8, 2, 2, True),
+])
+def test_decode_path(moe, oracle, wdtype, D, H, E, k, n, grouped):
+    # the way a call takes, token by token or grouped, against the sizes from
+    # which on the latter is the faster one
+    c = Case(moe, oracle, T=n, D=D, H=H, E=E, k=k, wdtype=wdtype, seed=95, max_tokens=2 * n)
+    try:
+        x = np.ascontiguousarray(c.x)
+        names = kernels_of(lambda: c.dev.decode(x))
+        print(sorted(names), flush=True)
+        up = {"f32": "decode_up_f32_kernel", "bf16": "decode_up_mfma_kernel<0>", "fp8": "decode_up_mfma_kernel<1>"}[wdtype]
+        assert (up in names) == grouped and any(m.startswith("decode_up_kernel") for m in names) != grouped, names
     finally:
         c.dev.close()
 
@@ -76,7 +106,8 @@ def test_decode_grouped_independent_of_the_batch(moe, oracle, wdtype, n):
         c.dev.close()
 
 
-@pytest.mark.parametrize("wdtype,T,D,H", [("bf16", 40, 512, 700), ("bf16", 70, 260, 300), ("f32", 40, 512, 700)])
+@pytest.mark.parametrize("wdtype,T,D,H", [("bf16", 40, 512, 700), ("bf16", 70, 260, 300), ("bf16", 100, 260, 300),
+                                           ("f32", 40, 512, 700)])
 def test_decode_grouped_infinite_weights(moe, oracle, wdtype, T, D, H):
     # an infinite weight gives the infinities of its products, as in a single
     # call, and not the NaN of infinity times a part of x that is 0
