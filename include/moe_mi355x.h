@@ -303,7 +303,13 @@ int moe_expert_forward(moe_handle *h, int32_t expert, const float *x, int32_t n,
  * xb [n][D] fp32, out [n][D_out] fp32 (host); logits [n][E_router], indices
  * [n][slots] (1-based), gates [n][slots] may be NULL.  Gated experts with TopKGating or
  * SwitchGating only (else MOE_EUNSUPPORTED); 1 <= n <= max_tokens (handles
- * with bf16 or fp8 weights: max_tokens / 2). */
+ * with bf16 or fp8 weights: max_tokens / 2).
+ * A token's logits, indices and gates are the same bits in a call of any n,
+ * and with fp32 weights its output too.  With bf16 or fp8 weights calls of few
+ * tokens on a small layer sum on the vector unit and others on the matrix
+ * unit, both in fp32 from the fp32 activations: the output of a token may
+ * differ between calls of different n by the rounding of those sums (a few
+ * 1e-7 of its norm), not between calls of the same n. */
 int moe_decode(moe_handle *h, const float *xb, int32_t n, float *out, float *logits, int32_t *indices,
                float *gates);
 

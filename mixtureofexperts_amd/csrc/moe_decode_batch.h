@@ -19,8 +19,8 @@
 // What bounds it: HBM, once the layer's matrices are a few tens of MB; below
 // that the four launches.  Measured against the single-token kernels (one MoE
 // call, host launches included, weights cold): 4096 / 14336, 2 of 8 experts,
-// bf16: n = 1 150 -> 129 us, n = 16 1668 -> 400 us (7.0 TB/s), n = 64 5756 ->
-// 765 us; fp8 n = 1 301 -> 78 us, n = 16 3842 -> 238 us; fp32 2048 / 1408, 6 of
+// bf16: n = 1 148 -> 127 us, n = 16 1712 -> 452 to 505 us (5.6 to 6.2 TB/s), n = 64
+// 5756 -> 765 us; fp8 n = 1 301 -> 78 us, n = 16 3842 -> 238 us; fp32 2048 / 1408, 6 of
 // 64 experts: n = 1 100 -> 49 us, n = 64 1612 -> 433 us.
 //
 // bf16 / fp8 weights (MFMA): the weights are the MFMA's A operand (16 rows),
@@ -34,7 +34,13 @@
 // whole lines); the waves of a block split K and add their partial sums
 // through LDS in wave order.  K ranges and row tiles depend on the layer's
 // sizes only, and an MFMA column on its own token only, so a token's result
-// does not depend on the batch it is in.
+// does not depend on the batch it is in, as long as that runs here: calls of few
+// tokens on small layers (decode_batched in moe_api.hip) sum in the order of
+// the single-token kernels and differ in the last bits (2.5e-7 of the output's
+// norm at 512 / 700).  Either order for every call of a layer costs more than it
+// gives: grouped VALU kernels with a single call's sums took 75 us instead of 33
+// for 64 tokens of 512 / 1376 in bf16 and 293 instead of 86 at 1024 / 4096, and
+// one token grouped 19 instead of 10 and 30 instead of 21.
 //
 // fp32 weights (VALU): the arithmetic of decode_up_kernel / decode_down_kernel
 // (one wave per row, chunks of 4 per lane in order, a fixed butterfly), each

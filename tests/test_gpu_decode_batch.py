@@ -133,6 +133,37 @@ def test_decode_grouped_infinite_weights(moe, oracle, wdtype, T, D, H):
         c.dev.close()
 
 
+@pytest.mark.parametrize("wdtype,D,H", [("bf16", 512, 700), ("fp8", 512, 700), ("bf16", 2048, 128), ("f32", 512, 700)])
+def test_decode_calls_of_any_size_agree(moe, oracle, wdtype, D, H):
+    # a token's routing is the same bits in a call of any size, its output too
+    # with fp32 weights.  bf16 and fp8 layers below the sizes of the grouped
+    # kernels run small calls on the VALU and larger ones on the matrix unit
+    # (D = 2048, 48 experts: all of them grouped, a rule on the layer): both
+    # round fp32 sums of K products, a lane's K / 64 and then 6 more additions or
+    # fewer, so each is about sqrt(K / 64 + 6) 2^-25 off the exact one, twice in
+    # turn: they differ by at most 4 sqrt(K / 64 + 6) 2^-25 = 4.9e-7 at K = 700
+    # (2.5e-7 measured); between calls that take the same way by no bit
+    E = 48 if D == 2048 else 6
+    c = Case(moe, oracle, T=64, D=D, H=H, E=E, k=2, wdtype=wdtype, seed=96, max_tokens=128)
+    try:
+        x = np.ascontiguousarray(c.x)
+        out, logits, idx, gates = c.dev.decode(x)
+        same, worst = 0, 0.0
+        for t, n in ((0, 1), (9, 1), (20, 2), (31, 4), (40, 5), (3, 8), (11, 16), (24, 40)):
+            o, lg, i, g = c.dev.decode(np.ascontiguousarray(x[t:t + n]))
+            assert np.array_equal(lg.view(np.uint32), logits[t:t + n].view(np.uint32)), (t, n)
+            assert np.array_equal(i, idx[t:t + n]) and np.array_equal(g.view(np.uint32), gates[t:t + n].view(np.uint32))
+            equal = np.array_equal(o.view(np.uint32), out[t:t + n].view(np.uint32))
+            grouped = any("mfma" in m for m in kernels_of(lambda: c.dev.decode(np.ascontiguousarray(x[t:t + n]))))
+            assert equal or (wdtype != "f32" and not grouped), (t, n)
+            same += equal
+            worst = max(worst, rel_err(o, out[t:t + n]))
+        print(f"{same} of 8 calls with equal bits, others within {worst:.1e}", flush=True)
+        assert worst <= 4 * np.sqrt(max(D, H) / 64 + 6) * 2.0 ** -25 and (same == 8 if wdtype == "f32" or D == 2048 else same < 8)
+    finally:
+        c.dev.close()
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf, 3.4e38])
 def test_decode_grouped_is_not_held_up_by_one_token(moe, oracle, value):
     # one token whose every product is not finite: the other tokens' results
