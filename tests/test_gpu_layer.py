@@ -6,8 +6,12 @@ Tolerances (north star): layer output relative error (Frobenius) <= 1e-4 at
 fp32, 2e-2 at bf16, 5e-2 at fp8 weights; balance loss within 1e-5; routing
 bit-exact given identical router logits (the oracle is run on the GPU's
 logits; the logits themselves are checked against the oracle's fp32 GEMM)."""
+import re
+
 import numpy as np
 import pytest
+
+from kernel_names import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -16,6 +20,12 @@ TOL = {"f32": 1e-4, "bf16": 2e-2, "fp8": 5e-2}
 
 def rel_err(a, b):
     return float(np.linalg.norm((a - b).astype(np.float64)) / max(np.linalg.norm(b.astype(np.float64)), 1e-30))
+
+
+def tile_heights(call):
+    """Tile rows of the bf16 / fp8 GEMMs that call() launches."""
+    ms = [re.match(r"grouped_gemm_bf16_kernel<\d+, (\d+),", n) for n in kernels_of(call)]
+    return {int(m.group(1)) for m in ms if m}
 
 
 class Case:
@@ -462,23 +472,29 @@ def test_mixtral_shape_scaled(moe, oracle):
     check_case(c, TOL["bf16"])
 
 
-@pytest.mark.parametrize("E,k,etype,act,wdtype", [
-    (4, 1, "gated", "silu", "bf16"),
-    (4, 1, "gated", "silu", "fp8"),
-    (4, 1, "standard", "gelu", "bf16"),
-    (4, 1, "standard", "gelu", "fp8"),
-    (8, 2, "gated", "silu", "bf16"),
+@pytest.mark.parametrize("E,k,etype,act,wdtype,H,bm", [
+    (4, 1, "gated", "silu", "bf16", 13100, 256),
+    (4, 1, "gated", "silu", "fp8", 384, 128),
+    (4, 1, "standard", "gelu", "bf16", 26200, 256),
+    (4, 1, "standard", "gelu", "fp8", 384, 128),
+    (8, 2, "gated", "silu", "bf16", 6600, 256),
+    (8, 2, "gated", "silu", "bf16", 384, 128),
 ])
-def test_256_row_tiles(moe, oracle, E, k, etype, act, wdtype):
-    # at most 16 experts averaging >= 384 rows: the 256-row tile kernels (one
-    # workgroup per CU; standard experts with fp8 weights stay on 128-row
-    # tiles); a skewed router bias gives partial last tiles, and D = 320
-    # leaves y rows past the last 256-column block (cut at N)
+def test_256_row_tiles(moe, oracle, E, k, etype, act, wdtype, H, bm):
+    # few experts of 400 rows, with n-tiles for four rounds of work items (6
+    # M tiles and one per expert): the 256-row tile kernels (one workgroup per
+    # CU); fewer items or fp8 weights: 128-row tiles.  A skewed router bias
+    # gives partial last tiles, and D = 320 leaves y rows past the last
+    # 256-column block (cut at N)
     rng = np.random.default_rng(70 + E)
     bias = (rng.standard_normal(E) * 0.7).astype(np.float32)
-    c = Case(moe, oracle, T=1600, D=320, H=384, E=E, k=k, gate="switch" if k == 1 else "topk", expert_type=etype,
+    c = Case(moe, oracle, T=1600, D=320, H=H, E=E, k=k, gate="switch" if k == 1 else "topk", expert_type=etype,
              act=act, wdtype=wdtype, xdtype="bf16", seed=70 + E, router_bias=bias)
-    check_case(c, TOL[wdtype])
+    try:
+        check_case(c, TOL[wdtype])
+        assert tile_heights(lambda: c.run(training=True)) == {bm}
+    finally:
+        c.dev.close()
 
 
 def test_standard_experts_gelu(moe, oracle):
@@ -758,7 +774,8 @@ def test_random_layer_shapes(moe, oracle):
     # seeded shapes across the paths the bf16 kernel takes: D / Dout not
     # multiples of 8 (element-wise permute, direct y stores) or of 256 (cut
     # columns), 2..40 experts, top-1..4, gated / standard, bf16 / fp8, batches
-    # that give 128- and 256-row tiles, partial tiles and tail-split down tiles
+    # and widths that give 128- and 256-row tiles, partial tiles and tail-split
+    # down tiles
     rng = np.random.default_rng(2026)
     for case in range(14):
         E = int(rng.integers(2, 41))
@@ -768,16 +785,22 @@ def test_random_layer_shapes(moe, oracle):
         H = int(rng.choice([96, 200, 384, 688]))
         T = int(rng.integers(16, 700)) if case % 2 == 0 else int(rng.integers(1200, 2400))
         if case % 4 == 1:
-            E = int(rng.integers(2, 9))  # few large experts: 256-row tiles
+            E = int(rng.integers(2, 9))
             k = int(rng.integers(1, min(2, E) + 1))
         etype = "gated" if rng.random() < 0.7 else "standard"
         act = "silu" if etype == "gated" else str(rng.choice(["gelu", "relu"]))
         wdtype = str(rng.choice(["bf16", "fp8"]))
         bias = (rng.standard_normal(E) * float(rng.choice([0.0, 1.0]))).astype(np.float32)
+        if case % 4 == 1:  # few large experts, n-tiles for four rounds of work items: 256-row tiles
+            E, D, wdtype = min(E, T * k // 192), min(D, 200), "bf16"
+            bias = bias[:E]
+            H = -(-1024 // (T * k // 256 + E)) * (128 if etype == "gated" else 256) - 40
         c = Case(moe, oracle, T=T, D=D, H=H, Dout=Dout, E=E, k=k, gate="switch" if k == 1 else "topk",
                  expert_type=etype, act=act, wdtype=wdtype, xdtype="bf16", seed=900 + case, router_bias=bias)
         try:
             check_case(c, TOL[wdtype])
+            if case % 4 == 1:
+                assert tile_heights(lambda: c.run(training=True)) == {256}
         finally:
             c.dev.close()
 
