@@ -9,6 +9,7 @@ combines both: 8 sqrt(K) 2^-25 <= 1.3e-5 at K = 2816, 4.6e-6 at K = 330."""
 import numpy as np
 import pytest
 
+from kernel_names import kernels_of
 from test_gpu_layer import Case, check_case
 
 pytestmark = pytest.mark.gpu
@@ -106,6 +107,44 @@ def test_f32x3_small_k(moe, oracle, T, D, H, E, k, etype, act):
         ref = exact_forward(c, res["indices"], res["gates"])
         err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
         assert err <= 10 * 2.0 ** -25, err
+    finally:
+        c.dev.close()
+
+
+@pytest.mark.parametrize("T,D,H,E,k,etype,act,ran,fp32_unit", [
+    (1037, 520, 2731, 6, 2, "gated", "silu", "<0, false>", 8.2e-7),
+    (1037, 520, 2731, 6, 2, "standard", "gelu", "<1, false>", 7.0e-7),
+])
+def test_f32x3_running_sums(moe, oracle, T, D, H, E, k, etype, act, ran, fp32_unit):
+    # the up GEMMs of large layers: K of 512 or more, tiles for every CU and none
+    # cut into K ranges (22 M tiles of 22 or 11 n-tiles), ragged in every
+    # dimension.  Running sums are used where they are no less accurate than the
+    # fp32 matrix unit, whose error on the same layers is the bound (5.3e-7 and
+    # 3.9e-7 measured)
+    c = Case(moe, oracle, T=T, D=D, H=H, E=E, k=k, expert_type=etype, act=act, wdtype="f32", seed=800)
+    try:
+        out, _ = check_case(c, 1e-5)
+        res = c.run(training=True)[2]
+        assert "grouped_gemm_f32x3_kernel" + ran in kernels_of(lambda: c.run(training=True))
+        ref = exact_forward(c, res["indices"], res["gates"])
+        err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+        print(f"error against 64 bits {err:.2e}", flush=True)
+        assert err <= fp32_unit, err
+        # an infinity, a NaN and a value above bf16's largest in x: their tokens'
+        # outputs as fp32 sums give them, the others' bits as they were
+        bad = np.ascontiguousarray(c.x)
+        o0 = c.dev.forward_routed(bad, 0, False, res["indices"], res["gates"])[0]
+        bad = bad.copy()
+        bad[5, 519], bad[700, 0], bad[1036, 77] = np.inf, np.nan, 3.4e38
+        o = c.dev.forward_routed(bad, 0, False, res["indices"], res["gates"])[0]
+        keep = np.ones(T, bool)
+        keep[[5, 700, 1036]] = False
+        assert np.array_equal(o[keep].view(np.uint32), o0[keep].view(np.uint32))
+        assert np.isnan(o[700]).all() and not np.isfinite(o[5]).any()
+        if etype == "standard":  # 3.4e38 times the weights is finite, the value's first part is not
+            c.x[1036] = bad[1036]
+            big = exact_forward(c, res["indices"], res["gates"])[1036]
+            assert np.max(np.abs(o[1036] - big)) <= 1e-5 * np.max(np.abs(big))
     finally:
         c.dev.close()
 

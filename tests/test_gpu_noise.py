@@ -12,6 +12,7 @@ and the z-loss the logits without noise (moe_layer.jl:117-121)."""
 import numpy as np
 import pytest
 
+from kernel_names import kernels_of
 from test_gpu_layer import TOL, Case, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -107,8 +108,9 @@ def test_layer_router_noise_python_api(moe):
     layer.close()
 
 
-@pytest.mark.parametrize("wdtype,p", [("f32", 0.25), ("bf16", 0.25), ("f32", 0.15)])
-def test_standard_expert_dropout(moe, oracle, wdtype, p):
+@pytest.mark.parametrize("wdtype,p,T", [("f32", 0.25, 512), ("bf16", 0.25, 512), ("f32", 0.15, 512),
+                                        ("f32", 0.15, 6144)])  # 104 tiles: the fp32 GEMM on the bf16 matrix unit
+def test_standard_expert_dropout(moe, oracle, wdtype, p, T):
     """StandardExpert's Dropout(p) in training (src/experts/standard.jl:49-51):
     with W1 = W2 = I, zero biases, the identity activation and k = 1 (gate
     exactly 1) the layer output is dropout(x): every element is 0 or x times
@@ -119,7 +121,7 @@ def test_standard_expert_dropout(moe, oracle, wdtype, p):
     from mixtureofexperts_amd import _lib
     from mixtureofexperts_amd._device import DeviceLayer, GateSpec
 
-    T, D, E = 512, 64, 4
+    D, E = 64, 4
     rng = np.random.default_rng(31)
     x = rng.standard_normal((T, D)).astype(np.float32)
     if wdtype == "bf16":
@@ -135,6 +137,8 @@ def test_standard_expert_dropout(moe, oracle, wdtype, p):
     for e in range(E):
         dev.set_expert(e, eye, eye, None, np.zeros(D, np.float32), np.zeros(D, np.float32), src_dtype=_lib.MOE_F32)
     dev.set_expert_dropout(p, seed=77)
+    f32x3 = kernels_of(lambda: dev.forward(x, _lib.MOE_F32, False)) & {"grouped_gemm_f32x3_kernel<1, true>"}
+    assert bool(f32x3) == (wdtype == "f32" and T > 512)
     y_inf, _, _ = dev.forward(x, _lib.MOE_F32, False)
     assert np.array_equal(y_inf, x)
     y, _, _ = dev.forward(x, _lib.MOE_F32, True)
