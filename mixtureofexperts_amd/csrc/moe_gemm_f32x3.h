@@ -1,13 +1,15 @@
 // moe_gemm_f32x3.h -- the fp32 grouped GEMM on the bf16 matrix unit, for expert
 // segments of many rows.  Part of moe_gemm.hip.
 //
-// An fp32 value is the sum of three bf16 ones (8 significant bits each, rounded
-// to nearest: |x1| <= 2^-9 |x|, |x2| <= 2^-17 |x|), and an fp32 product to
-// fp32 accuracy the sum of the six products of parts i + j <= 2: the three
-// left out are below 2^-25 of it, random in sign, under the rounding of the
-// fp32 sum.  Per 32 x 32 outputs and 16 K, six bf16 products take 192 cycles
-// of the matrix unit, eight v_mfma_f32_32x32x2_f32 512; the running sums stay
-// fp32 and take 6 roundings per 32 K instead of 16.
+// An fp32 value of 2^-110 or more is the sum of three bf16 ones (8 significant
+// bits each, rounded to nearest: |x1| <= 2^-9 |x|, |x2| <= 2^-17 |x|), and an
+// fp32 product to fp32 accuracy the sum of the six products of parts i + j <=
+// 2: the three left out are below 2^-25 of it, random in sign, under the
+// rounding of the fp32 sum.  Smaller values keep their bits down to 2^-133,
+// bf16's smallest: the error of one is 2^-22 of it at 2^-112, 2^-14 at 2^-120,
+// 2^-8 at 2^-126, where grouped_gemm_kernel takes it whole.  Per 32 x 32 outputs and
+// 16 K, six bf16 products take 192 cycles of the matrix unit, eight
+// v_mfma_f32_32x32x2_f32 512; the running sums stay fp32.
 //
 // What bounds it: the matrix unit's power at large sizes, per-tile latencies
 // (24 stages between prologue and epilogue) at small K.  Against
@@ -39,13 +41,17 @@
 // MFMAs over the fp32 operands (redo).
 //
 // STAGE_SUMS: the six products of a stage start from zero, the smallest first,
-// and are added to the running sum with one rounded addition.  The matrix unit
-// cuts every sum off (towards zero: a bias), so six sums of the running size
-// per 32 K cost more accuracy at small K than grouped_gemm_kernel's 16 of
-// random sign: error against 64 bits at 300 / 300 gated 2.5e-7 there, 5.0e-7 with
-// running sums, 1.6e-7 with stage sums; 64 / 64 2.0e-7, 2.9e-7, 1.0e-7; 128 / 256
-// standard 1.8e-7, 3.4e-7, 1.2e-7; 768 / 3072 standard 11.3e-7, 9.9e-7,
-// 2.6e-7.
+// and are added to the running sum with one rounded addition.  An MFMA adds its
+// products to its accumulator in several steps, each rounded at the
+// accumulator's size, without a bias: a chain of 4096 random bf16 products has
+// an error of 3.9e-7 in a running accumulator, 2.1e-7 in sums of 32 from zero
+// and one addition each, 6.0e-7 with v_mfma_f32_16x16x4_f32 (the mean along the
+// sum's sign below 1e-8 in all).  Six instructions of the running size per 32 K
+// cost more accuracy at small K than grouped_gemm_kernel's 16 smaller ones:
+// error against 64 bits at 300 / 300 gated 2.5e-7 there, 5.0e-7 with running
+// sums, 1.6e-7 with stage sums; 64 / 64 2.0e-7, 2.9e-7, 1.0e-7; 128 / 256 standard
+// 1.8e-7, 3.4e-7, 1.2e-7; and no more from 512 on: 520 / 2731 gated 8.2e-7, 5.3e-7
+// with running sums in the up GEMM; 768 / 3072 standard 11.3e-7, 9.9e-7, 2.6e-7.
 // The additions wait for the matrix unit and cost 6 % where it is the bound
 // (768 / 3072 standard, 4096 tokens: 427 -> 453 us), 0 to 2 % elsewhere, so the running sums
 // stay for large calls of large K (launch_f32x3).

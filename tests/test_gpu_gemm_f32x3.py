@@ -97,8 +97,9 @@ def test_expert_forward_takes_the_layers_kernel(moe, oracle):
 def test_f32x3_small_k(moe, oracle, T, D, H, E, k, etype, act):
     # Small K: as accurate as the fp32 matrix unit (2.0e-7, 1.8e-7 and 2.5e-7 on the
     # first three).  Per GEMM sqrt(K / 32) 2^-25 for the rounded additions of the
-    # stages (1.2e-7 at 480) and, since stage sums are cut off, at most 2^-23 of a stage, random
-    # over them: about 0.6 x 2^-23; h rounds once more.  Two GEMMs in
+    # stages (1.2e-7 at 480) and for each stage's own sum, rounded in several
+    # steps, at most 2^-23 of it, random over the stages: about 0.6 x 2^-23; h
+    # rounds once more.  Two GEMMs in
     # turn and the gates: below 10 x 2^-25.
     c = Case(moe, oracle, T=T, D=D, H=H, E=E, k=k, gate="switch" if k == 1 else "topk", expert_type=etype, act=act,
              wdtype="f32", seed=700 + D)
