@@ -6,9 +6,8 @@
 // fp32 product to fp32 accuracy the sum of the six products of parts i + j <=
 // 2: the three left out are below 2^-25 of it, random in sign, under the
 // rounding of the fp32 sum.  Smaller values keep their bits down to 2^-133,
-// bf16's smallest: the error of one is 2^-22 of it at 2^-112, 2^-14 at 2^-120,
-// 2^-8 at 2^-126, where grouped_gemm_kernel takes it whole.  Per 32 x 32 outputs and
-// 16 K, six bf16 products take 192 cycles of the matrix unit, eight
+// bf16's smallest (an error of 2^-22 at 2^-112, 2^-14 at 2^-120), so sums below
+// 2^-90 are redone too.  Per 32 x 32 outputs and 16 K, six bf16 products take 192 cycles of the matrix unit, eight
 // v_mfma_f32_32x32x2_f32 512; the running sums stay fp32.
 //
 // What bounds it: the matrix unit's power at large sizes, per-tile latencies
@@ -37,8 +36,8 @@
 // ((r >> 2) & 3), as in the bf16 kernel.
 //
 // Infinities, NaN and values that round up to an infinity: their parts give
-// NaN or infinite sums, and a wave that holds such a sum takes it from fp32
-// MFMAs over the fp32 operands (redo).
+// NaN or infinite sums, and a wave that holds such a sum, or one that is not
+// 0 and below 2^-90, takes it from fp32 MFMAs over the fp32 operands (redo).
 //
 // STAGE_SUMS: the six products of a stage start from zero, the smallest first,
 // and are added to the running sum with one rounded addition.  An MFMA adds its
@@ -255,19 +254,36 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int NJ = 4 / NB;
 
     // redo: the wave's 64 x 64 sums on v_mfma_f32_16x16x4_f32, operands straight
-    // from memory; those that were not finite are replaced.  It takes about
+    // from memory; those that the parts do not give are replaced.  It takes about
     // four times the tile's own MFMAs and runs for whole waves, whatever the
     // number of such sums: 768 / 3072 standard, 4096 tokens, us a call: 545; with
     // an infinity in one row 945, in every row 1300 (1720 and 46070 by one lane
     // per output and one K value after the other).
-    bool fin = true;
+    auto good = [](float v) { return __builtin_isfinite(v) && (fabsf(v) >= 0x1p-90f || v == 0.0f); };
+    // first in two instructions per sum: 0 v is not 0 for infinities and NaN, and
+    // the smallest size, which zeros (rows of zeros, row blocks past the tile)
+    // bring below the line too
+    float nil[4] = {0.0f, 0.0f, 0.0f, 0.0f}, least = INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) fin = fin && (__builtin_isfinite(acc[i][j][c]) || row_of(i) >= rows);
-    if (__any(!fin)) {
+            for (int c = 0; c < 4; ++c) {
+                nil[c] = fmaf(acc[i][j][c], 0.0f, nil[c]);
+                least = fminf(least, fabsf(acc[i][j][c]));
+            }
+    bool all_good = (nil[0] + nil[1]) + (nil[2] + nil[3]) == 0.0f && least >= 0x1p-90f;
+    if (!all_good) {
+        all_good = true;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) all_good = all_good && (good(acc[i][j][c]) || row_of(i) >= rows);
+    }
+    if (__any(!all_good)) {
         const float *ap[4], *bp[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) ap[i] = A + (arow0 + min(row_of(i), rows - 1)) * g.lda + 4 * q4;
@@ -300,7 +316,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) acc[i][j][c] = __builtin_isfinite(acc[i][j][c]) ? acc[i][j][c] : sum[i][j][c];
+                for (int c = 0; c < 4; ++c) acc[i][j][c] = good(acc[i][j][c]) ? acc[i][j][c] : sum[i][j][c];
     }
 
     float *ws = S > 1 ? g.split_ws + ((long long)(mt * g.n_tiles + nt) * S + ks) * (BM * BR) : nullptr;

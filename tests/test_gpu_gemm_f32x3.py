@@ -233,3 +233,31 @@ def test_f32x3_calls_with_infinities_take_their_time(moe, oracle, etype, H):
             assert held <= 5 * clean, (clean, held)
     finally:
         c.dev.close()
+
+
+@pytest.mark.parametrize("exp", [-126, -120, -112, -100])
+@pytest.mark.parametrize("T,H", [(12800, 96), (200, 6400)])
+def test_f32x3_tiny_values(moe, oracle, T, H, exp):
+    # values whose low parts are below bf16's smallest: identity experts give
+    # them back bit for bit, as fp32 products and sums with zeros do (H = 6400:
+    # K ranges)
+    D = 64
+    c = Case(moe, oracle, T=T, D=D, H=H, E=2, k=1, gate="switch", expert_type="standard", act="identity", wdtype="f32",
+             seed=64, max_tokens=T)
+    try:
+        print(f"f32x3 values of 2^{exp} H={H}", flush=True)
+        w1, w2 = np.zeros((H, D), np.float32), np.zeros((D, H), np.float32)
+        w1[np.arange(D), np.arange(D)] = 1.0
+        w2[np.arange(D), np.arange(D)] = 1.0
+        for e in range(2):
+            c.dev.set_expert(e, w1, w2, None, np.zeros(H, np.float32), np.zeros(D, np.float32))
+        x = np.ascontiguousarray((1 + np.random.default_rng(65).random((T, D))) * 2.0 ** exp).astype(np.float32)
+        x[3] = 0.0
+
+        def forward():
+            return c.dev.forward_routed(x, 0, False, np.ones((T, 1), np.int32), np.ones((T, 1), np.float32))[0]
+
+        assert any(n.startswith("grouped_gemm_f32x3_kernel") for n in kernels_of(forward))
+        assert np.array_equal(forward().view(np.uint32), x.view(np.uint32))
+    finally:
+        c.dev.close()
