@@ -3,7 +3,6 @@
 // orchestration of the MoE-layer forward pass on one HIP stream.
 #include <algorithm>
 #include <climits>
-#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -1718,35 +1717,31 @@ static int decode_wide_route(const moe_handle *h) { return (long long)h->D * h->
 
 // Whether a decode call of n tokens runs grouped by expert (four launches)
 // instead of token by token (two launches, the routing repeated by every
-// block).  us below: token by token / grouped, five rounds of each in turn over
-// three handles; a side's rounds differ by 1 to 3 %.  M: the multiply-adds of
-// the call's expert products, n kt 3 D H; router: D x its experts, which every
-// block reads token by token.
+// block).  The lines are multiply-adds of the call's expert products, n kt 3 D H,
+// and were chosen on 1560 random calls (128 - 4096 / 96 - 14336, 4 - 128 experts, 1 - 64
+// tokens, half of them with 1 to 4), both ways in turn for three rounds over
+// two handles, by events on one stream and by the clock around the loop; a
+// side's rounds differ by 1 to 3 %.  Geometric mean of a call's time over that of
+// its faster way: fp32 1.01 to 1.03, bf16 1.00 to 1.04, fp8 1.01 to 1.02 (all calls
+// token by token 1.16, 1.43 and 3.4, all grouped 1.11, 1.13 and 1.02).  us below:
+// token by token / grouped.
 //
-// fp32 (same bits either way), several tokens: by the weights that grouping
-// does not read again, i.e. the M of the entries past the n tokens' expected
-// number of experts.  Rows of 1024 values or more: 4 M (1024 / 2816 of 8: 2 tokens
-// 34 / 36, 3 tokens = 12 M 46 / 45; 2048 / 700, 4 of 16, 2 tokens = 4 M 51 / 48).
-// From 448 on: 18 M (512 / 1376 of 8: 6 tokens 25 / 26, 8 tokens = 19 M 28 / 28 and, on
-// one handle whose weights the Infinity Cache keeps, 19 / 16 to 19; 16 tokens =
-// 53 M 45 / 34; 500 / 665 of 73: 16 tokens = 6 M 54 / 65, 32 tokens = 21 M
-// 77 / 77).  Shorter rows are bound by the per-entry reductions, which a group
-// runs in series, up to a call's 170 M (320 / 600 of 8, 64 tokens = 74 M 44 / 46;
-// 384 / 1536, 6 of 64: 85 M 74 / 75, 170 M 119 / 104; 136 / 1000, 4 of 32, 104 M 95 /
-// 92; 200 / 2000 of 16, 154 M 100 / 92).
-// fp32, one token: 64 M (1024 / 8192 = 50 M 47 / 52, 2048 / 5504 = 68 M 69 / 67), 40 M
-// with a router of more than 48 K (2048 / 1408, 6 of 30 = 52 M 87 / 77).
+// fp32 (the same bits either way): 28 M (512 / 1376, 2 of 8: 6 tokens = 25 M 25 / 26,
+// 8 = 34 M 28 / 28, 16 = 68 M 45 / 33); rows under 320 are bound by the per-entry
+// reductions, which a group runs in series, up to 170 M (200 / 2000, 2 of 16, 64
+// tokens = 154 M 100 / 92; 136 / 1000, 4 of 32: 32 tokens = 52 M 55 / 59); one token
+// 40 M (2048 / 1408, 6 of 30 = 52 M 87 / 77; 1024 / 8192, 2 of 8 = 50 M 47 / 52).
 //
-// bf16, up to four tokens: 140 M (1024 / 8192: 1 token = 50 M 33 / 48, 2 tokens = 101 M
-// 51 / 63, 3 tokens = 151 M 68 / 70; 2048 / 5504: 1 token = 68 M 48 / 57, 2 tokens =
-// 135 M 69 / 76, 3 tokens = 203 M 93 / 90), 60 M with a router of 32 K (2048 / 768, 4
-// of 16, 4 tokens = 75 M 59 / 51; 4096 / 4096 of 8, 1 token = 101 M 74 / 74, 2 tokens
-// 105 / 105), 40 M above 48 K (2048 / 1408, 6 of 30, 1 token = 52 M 68 / 60).
-// More tokens: 40 M (512 / 1376: 8 tokens = 34 M 21 / 24, 16 tokens = 67 M 32 / 25;
-// 768 / 2048: 6 tokens = 57 M 28 / 27; 4096 / 300: 6 tokens = 44 M 55 / 48).
-// fp8: 7.2 M (512 / 768: 3 tokens = 7.1 M 16 / 18; 4096 / 300: 1 token = 7.4 M 50 / 34;
-// 512 / 1376: 1 token = 4 M 15 / 17, 2 tokens = 8 M 20 / 18; 256 / 704 of 16, 8 tokens =
-// 9 M 19 / 19).
+// bf16, one token: 40 M, and H < 2 D (long down rows run well token by token: 1024 /
+// 8192, 2 of 8 = 50 M 33 / 48; 2048 / 5504 = 68 M 48 / 57) or a router of 28 K values,
+// which every block reads (4096 / 14336 of 8: 148 / 127).  To four tokens: 20 M with
+// more than two slots (2048 / 768, 4 of 16: 3 tokens = 57 M 52 / 48; 520 / 1000, 4 of 32: 4
+// tokens = 25 M 29 / 28), else 60 M (1024 / 2816, 2 of 8: 4 tokens = 69 M 36 / 37).  More:
+// 12 M with more than two slots, H < D or such a router (768 / 141, 2 of 50: 37 tokens =
+// 24 M 62 / 42), else 40 M (512 / 1376, 2 of 8: 8 tokens = 34 M 21 / 24, 16 = 68 M 32 / 25).
+//
+// fp8: 7 M (512 / 1376, 2 of 8: 1 token = 4 M 15 / 17, 2 = 8 M 20 / 18; 148 / 271, 3 of 17: 22
+// tokens = 8 M 33 / 23; 512 / 768, 2 of 8: 3 tokens = 7 M 16 / 18).
 static bool decode_batched(const moe_handle *h, int n) {
     const int c = std::min(n, kDecodeChunk);
     // workspace: y of every entry; bf16 / fp8: x in the split workspace and h
@@ -1754,17 +1749,17 @@ static bool decode_batched(const moe_handle *h, int n) {
     if ((long long)c * h->kt * h->Dout > (long long)h->rows_max * h->ld_y) return false;
     if (h->wt != WT_F32 && (6LL * c * h->D_pad > 4 * h->split_cap || 3LL * c * h->kt > h->act_rows)) return false;
     if (decode_wide_route(h)) return true;
-    const long long mac1 = 3LL * h->D * h->H, mac = n * h->kt * mac1, router = (long long)h->D * h->Er_pad;
-    if (h->wt == WT_FP8) return mac >= 7200000LL;
-    if (h->wt == WT_BF16) {
-        if (n > 4) return mac >= 40000000LL;
-        return mac >= (router > 48 * 1024 ? 40000000LL : router >= 32 * 1024 ? 60000000LL : 140000000LL);
+    const long long M = 1000000, K = 1024;
+    const long long mac = (long long)n * h->kt * 3 * h->D * h->H, router = (long long)h->D * h->Er_pad;
+    if (h->wt == WT_FP8) return mac >= 7 * M;
+    if (h->wt == WT_F32) {
+        if (h->D < 320) return mac >= 170 * M;
+        return mac >= (n == 1 ? 40 * M : 28 * M);
     }
-    if (n == 1) return mac >= (router > 48 * 1024 ? 40000000LL : 64000000LL);
-    if (h->D < 448) return mac >= 170000000LL;
-    // the routed experts that n tokens of k pick, loads being even
-    const double experts = h->Er * (1.0 - std::pow(1.0 - (double)h->k / h->Er, n)) + h->lsh;
-    return (n * h->kt - experts) * mac1 >= (h->D >= 1024 ? 4e6 : 18e6);
+    const bool wide = router >= 28 * K;
+    if (n == 1) return mac >= 40 * M && (h->H < 2 * h->D || wide);
+    if (n <= 4) return mac >= (h->kt > 2 ? 20 * M : 60 * M);
+    return mac >= (h->kt > 2 || h->H < h->D || wide ? 12 * M : 40 * M);
 }
 
 static int decode_locked(moe_handle *h, const float *x_dev, int n, float *out_dev, hipStream_t s,

@@ -57,15 +57,17 @@ def test_decode_grouped(moe, oracle, wdtype, D, H, Dout, E, k, lsh, n):
 
 
 @pytest.mark.parametrize("wdtype,D,H,E,k,n,grouped", [
-    # measured us of both ways beside each line of the rule; here one call on either side of it
-    ("f32", 512, 1376, 8, 2, 6, False), ("f32", 512, 1376, 8, 2, 8, True),   # rows of 448 values or more: 18 M saved
-    ("f32", 500, 665, 73, 2, 16, False),                                      # few tokens share an expert of 73
-    ("f32", 1024, 704, 16, 4, 2, False), ("f32", 1024, 704, 16, 4, 6, True),  # rows of 1024: 4 M saved
-    ("f32", 320, 600, 8, 2, 64, False), ("f32", 320, 1408, 8, 2, 64, True),   # short rows: a call's 170 M
-    ("f32", 2048, 4160, 2, 2, 1, False), ("f32", 2048, 5504, 2, 2, 1, True),  # one token: 64 M
-    ("bf16", 1024, 8192, 2, 2, 1, False), ("bf16", 1024, 8192, 2, 2, 3, True),
-    ("bf16", 512, 1376, 8, 2, 8, False), ("bf16", 512, 1376, 8, 2, 16, True),
-    ("fp8", 512, 1376, 8, 2, 1, False), ("fp8", 512, 1376, 8, 2, 2, True),
+    # measured us of both ways beside each line of the rule; here a call on either side of it
+    ("f32", 512, 1376, 8, 2, 6, False), ("f32", 512, 1376, 8, 2, 8, True),      # 28 M
+    ("f32", 316, 600, 8, 2, 64, False), ("f32", 316, 1408, 8, 2, 64, True),     # short rows: 170 M
+    ("f32", 2048, 3000, 2, 2, 1, False), ("f32", 2048, 3600, 2, 2, 1, True),    # one token: 40 M
+    ("bf16", 1024, 8192, 2, 2, 1, False), ("bf16", 2048, 3600, 2, 2, 1, True),  # one token: 40 M, H < 2 D
+    ("bf16", 1792, 3648, 16, 3, 1, True),                                       # ... or a router of 28 K
+    ("bf16", 512, 1376, 8, 3, 2, False), ("bf16", 512, 1376, 8, 3, 4, True),    # to four tokens: 20 M with 3 slots
+    ("bf16", 512, 4096, 8, 2, 4, False), ("bf16", 512, 5120, 8, 2, 4, True),    # ... 60 M with 2
+    ("bf16", 512, 1376, 8, 2, 8, False), ("bf16", 512, 1376, 8, 2, 16, True),   # more: 40 M
+    ("bf16", 512, 384, 16, 4, 5, False), ("bf16", 512, 384, 16, 4, 6, True),    # ... 12 M with 4 slots
+    ("fp8", 512, 1376, 8, 2, 1, False), ("fp8", 512, 1376, 8, 2, 2, True),      # 7 M
 ])
 def test_decode_path(moe, oracle, wdtype, D, H, E, k, n, grouped):
     # the way a call takes, token by token or grouped, against the sizes from
