@@ -39,7 +39,9 @@
 //
 // LDS: per stage an A tile (BM rows) and a B tile (256 rows) of 32 bf16 =
 // 64 B per row; the 16-byte chunks of row r are stored at chunk ^ ((r >> 2) & 3)
-// so the fragment reads (16 rows, four chunks) spread over all 64 banks.  Each
+// so that 16 rows' chunks of one K group lie in all 64 banks once.  (The counters
+// show 3 to 5.5 conflict cycles per LDS instruction all the same; the 32 rows x
+// one chunk that a 32x32x16 fragment reads had none.)  Each
 // global_load_lds_dwordx4 writes 1 KB = 16 rows linearly (lane l -> offset
 // 16 l), so the swizzle is part of the tile images.
 #include <algorithm>
@@ -616,11 +618,12 @@ struct RowOffsetPut {
 // The kernel, BM = 128 or 256.
 // ============================================================================
 // v_mfma_f32_16x16x32_bf16: at the card's power limit a loop of it alone runs
-// 2040 TFLOP/s, one of v_mfma_f32_32x32x16_bf16 1770 (random operands, 128 x
-// 128 per wave), and the GEMMs here are at that limit.  Up / down GEMM, us, with
+// 1940 to 2040 TFLOP/s, one of v_mfma_f32_32x32x16_bf16 1740 to 1770 (random
+// operands), and the GEMMs here are at that limit.  Up / down GEMM, us, with
 // the 32x32x16 instruction (128 x 128 waves on 256-row tiles) and now: 66 fp8
 // experts of 2048 / 1408, 8192 tokens: 654 / 350 and 604 / 323; 8 bf16 experts
-// of 4096 / 14336, 4096 tokens: 1577 / 841 and 1506 / 790 (1.28 PFLOP/s, up).
+// of 4096 / 14336, 4096 tokens: 1577 / 841 and 1506 / 790 (1.21 to 1.28 PFLOP/s, up,
+// over runs and boxes).
 // A wave's 64 x 128 outputs are 128 accumulator registers; a 128 x 128 wave
 // (256 of them in 64 blocks) spilled hundreds.
 // Two waves per SIMD: one workgroup of eight on 256-row tiles; on 128-row

@@ -10,17 +10,15 @@
 // 2^-90 are redone too.  Per 32 x 32 outputs and 16 K, six bf16 products take 192 cycles of the matrix unit, eight
 // v_mfma_f32_32x32x2_f32 512; the running sums stay fp32.
 //
-// What bounds it: the matrix unit's power at large sizes, per-tile latencies
-// (24 stages between prologue and epilogue) at small K.  Against
+// What bounds it: the work besides the MFMAs (splits, LDS), which keep the
+// matrix unit busy 64 to 67 % of cycles at 1.8 GHz at 4096 / 14336, 43 to 54 % at
+// 2.2 to 2.3 GHz at 768 / 3072 with its 24 and 96 stages per tile.  Against
 // grouped_gemm_kernel (whole layer forward, 8 experts, top-2, 4096 tokens):
-// 4096 / 14336 gated 25.4 -> 14.2 ms, 768 / 3072 standard 746 -> 440 us, 1024 / 4096
+// 4096 / 14336 gated 25.4 -> 14.2 ms, 768 / 3072 standard 722 -> 428 us, 1024 / 4096
 // gated 1861 -> 1040 us; error against 64 bits 2.8e-6 -> 2.4e-6, 1.13e-6 ->
 // 0.99e-6, 1.44e-6 -> 1.24e-6.  Two 128 x 128 workgroups per CU instead of one
-// kept the MFMAs busier (77 instead of 68 % of cycles) at a lower clock (1.51
-// instead of 1.66 GHz) and took 4 % longer: what counts is the work besides the
-// MFMAs, and the MFMA's own (16x16x32 5 % faster than 32x32x16).  Splitting the
-// last round's tiles into K ranges gained nothing for the same reason (467 and
-// 463 us).
+// took 4 % longer, 32x32x16 instead of 16x16x32 MFMAs 5 %, and splitting the last
+// round's tiles into K ranges gained nothing (467 and 463 us).
 //
 // Tile 128 rows x 256 weight rows (gated: 128 of W1 and the same 128 of W3), 8
 // waves as 2 (rows) x 4 (columns), two per SIMD, each 64 x 64.  A stage is 32
