@@ -1762,6 +1762,13 @@ static bool decode_batched(const moe_handle *h, int n) {
     return mac >= (h->kt > 2 || h->H < h->D || wide ? 12 * M : 40 * M);
 }
 
+// Whether a chunk's out would overwrite x of a later chunk: out may share memory
+// with x (token by token, all of x is read before any of out is written).
+static bool decode_out_in_later_x(const moe_handle *h, const float *x, int n, const float *out) {
+    if (n <= kDecodeChunk || out + (long long)n * h->Dout <= x || x + (long long)n * h->D <= out) return false;
+    return !(out == x && h->Dout <= h->D);
+}
+
 static int decode_locked(moe_handle *h, const float *x_dev, int n, float *out_dev, hipStream_t s,
                          hipEvent_t done = nullptr) {
     DecodeArgs a{};
@@ -1773,7 +1780,7 @@ static int decode_locked(moe_handle *h, const float *x_dev, int n, float *out_de
     a.Dpad = h->D_pad; a.H = h->H; a.Hpad = h->H_pad; a.Dout = h->Dout;
     a.s1 = h->s1; a.s3 = h->s3; a.s2 = h->s2; a.Dout_npad = h->Dout_npad;
     a.h = (float *)h->hbuf; a.out = out_dev;
-    if (decode_batched(h, n)) {
+    if (decode_batched(h, n) && !decode_out_in_later_x(h, x_dev, n, out_dev)) {
         for (int t0 = 0; t0 < n; t0 += kDecodeChunk) {
             DecodeArgs c = a;
             c.n = std::min(kDecodeChunk, n - t0);

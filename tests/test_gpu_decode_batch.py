@@ -166,6 +166,35 @@ def test_decode_calls_of_any_size_agree(moe, oracle, wdtype, D, H):
         c.dev.close()
 
 
+@pytest.mark.parametrize("wdtype", ["f32", "bf16"])
+@pytest.mark.parametrize("Dout,shift", [(1024, 0), (512, 0), (256, 0), (512, 40 * 512)])
+def test_decode_out_over_x(moe, oracle, wdtype, Dout, shift):
+    # out in the memory of x, at its start or some rows on, wider and narrower:
+    # every token's x is read before it is overwritten, also where a call runs in
+    # chunks of 64 tokens
+    import torch
+
+    from mixtureofexperts_amd import _lib
+
+    n, D = 150, 512
+    c = Case(moe, oracle, T=n, D=D, H=700, Dout=Dout, E=6, k=2, wdtype=wdtype, seed=97, max_tokens=2 * n)
+    try:
+        print(f"decode over x, w={wdtype} Dout={Dout} shift={shift}", flush=True)
+        ref = c.dev.decode(np.ascontiguousarray(c.x))[0]
+        buf = torch.zeros(n * max(D, Dout) + shift, device="cuda")
+        buf[:n * D] = torch.from_numpy(np.ascontiguousarray(c.x)).cuda().ravel()
+        out = buf[shift:shift + n * Dout]
+        torch.cuda.synchronize()
+        _lib.check(_lib.lib().moe_decode_async(c.dev.h, buf.data_ptr(), n, out.data_ptr(), None), c.dev.h)
+        torch.cuda.synchronize()
+        o = out.cpu().numpy().reshape(n, Dout)
+        if wdtype == "f32":
+            assert np.array_equal(o.view(np.uint32), ref.view(np.uint32))
+        assert rel_err(o, ref) <= 4.9e-7  # the bound of calls that sum in another order, above
+    finally:
+        c.dev.close()
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf, 3.4e38])
 def test_decode_grouped_is_not_held_up_by_one_token(moe, oracle, value):
     # one token whose every product is not finite: the other tokens' results
