@@ -55,7 +55,6 @@
 
 namespace moe {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -109,16 +108,6 @@ __device__ __forceinline__ int decode_group(const DecodeArgs &a, int ai, DecodeG
 }
 
 // ---- bf16 / fp8 weights -------------------------------------------------------------
-// Eight fp8 e4m3 bytes -> eight bf16 (exact).
-__device__ __forceinline__ bf16x8_t widen_fp8(uint32_t lo, uint32_t hi) {
-    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-    const bf16x2_t a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
-    const bf16x2_t b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
-    const bf16x2_t c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
-    const bf16x2_t d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
-    return bf16x8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
-}
-
 // One wave's share of C[rows][tokens] += W[rows][K range] X[tokens][K range]^T:
 // NM matrices x 2 row tiles of 16 rows, NT column tiles of 16 tokens, K steps
 // [s0, s1) of KS K values (32 bf16, 64 fp8).  wsrc[m]: lane address of row tile
@@ -185,7 +174,7 @@ __device__ __forceinline__ void stream_rows(const uint8_t *const (&wsrc)[NM], lo
 #pragma unroll
                     for (int u = 0; u < XL; ++u) {
                         bf16x8_t wf;
-                        if constexpr (WF8) wf = widen_fp8(wc[p][m][i][2 * u], wc[p][m][i][2 * u + 1]);
+                        if constexpr (WF8) wf = widen_fp8x8(wc[p][m][i][2 * u], wc[p][m][i][2 * u + 1]);
                         else __builtin_memcpy(&wf, &wc[p][m][i], 16);
 #pragma unroll
                         for (int j = 0; j < NT; ++j) {

@@ -51,7 +51,6 @@
 
 namespace moe {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 #define MOE_LDS_AS __attribute__((address_space(3)))
 
@@ -83,17 +82,8 @@ __device__ __forceinline__ uint2 pack_bf16x4(float a, float b, float c, float d)
     return r;
 }
 
-// Eight fp8 e4m3 bytes (lo: bytes 0-3, hi: bytes 4-7) -> eight bf16 (exact).
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ bf16x8_t widen_fp8x8(uint32_t lo, uint32_t hi) {
-    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-    const bf16x2_t a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
-    const bf16x2_t b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
-    const bf16x2_t c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
-    const bf16x2_t d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
-    return bf16x8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
-}
 
 // Wait until at most N vector-memory operations of this wave are outstanding.
 // The LDS writes of global_load_lds are counted by vmcnt.

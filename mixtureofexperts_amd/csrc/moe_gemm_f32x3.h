@@ -56,7 +56,6 @@
 // K split (g.ksplit = S > 1): as in grouped_gemm_kernel, blocks of BM x 256
 // floats.
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 // Eight fp32 -> three chunks of eight bf16.

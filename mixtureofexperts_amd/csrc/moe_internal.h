@@ -268,6 +268,18 @@ struct CombineArgs {
     int u, nchunk;               // set by launch_combine: 4-column groups per lane, column chunks per token
 };
 
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+// Eight fp8 e4m3 bytes (lo: bytes 0-3, hi: bytes 4-7) -> eight bf16 (exact).
+__device__ __forceinline__ bf16x8_t widen_fp8x8(uint32_t lo, uint32_t hi) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    const bf16x2_t a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
+    const bf16x2_t b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+    const bf16x2_t c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
+    const bf16x2_t d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
+    return bf16x8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
 struct GemmArgs {
     const void *A; long long lda;        // activations [rows][lda] (elements); bf16 kernel: A tile image
     const void *B0; const void *B1;      // packed weights [E][Npad][ldb]; bf16 kernel: B tile images
