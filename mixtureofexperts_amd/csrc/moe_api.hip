@@ -1718,11 +1718,12 @@ static int decode_wide_route(const moe_handle *h) { return (long long)h->D * h->
 // Whether a decode call of n tokens runs grouped by expert (four launches)
 // instead of token by token (two launches, the routing repeated by every
 // block).  The lines are multiply-adds of the call's expert products, n kt 3 D H,
-// and were chosen on 1560 random calls (128 - 4096 / 96 - 14336, 4 - 128 experts, 1 - 64
-// tokens, half of them with 1 to 4), both ways in turn for three rounds over
+// and were chosen on 2010 random calls (128 - 4096 / 96 - 14336, 4 - 128 experts, 1 - 64
+// tokens, most of them with few), both ways in turn for three rounds over
 // two handles, by events on one stream and by the clock around the loop; a
-// side's rounds differ by 1 to 3 %.  Geometric mean of a call's time over that of
-// its faster way: fp32 1.01 to 1.03, bf16 1.00 to 1.04, fp8 1.01 to 1.02 (all calls
+// side's rounds differ by 1 to 3 %, but a call below 25 us may take a third more
+// in one process than in the next.  Geometric mean of a call's time over that of
+// its faster way: fp32 1.01 to 1.03, bf16 1.02, fp8 1.01 to 1.02 (all calls
 // token by token 1.16, 1.43 and 3.4, all grouped 1.11, 1.13 and 1.02).  us below:
 // token by token / grouped.
 //
@@ -1734,11 +1735,13 @@ static int decode_wide_route(const moe_handle *h) { return (long long)h->D * h->
 //
 // bf16, one token: 40 M, and H < 2 D (long down rows run well token by token: 1024 /
 // 8192, 2 of 8 = 50 M 33 / 48; 2048 / 5504 = 68 M 48 / 57) or a router of 28 K values,
-// which every block reads (4096 / 14336 of 8: 148 / 127).  To four tokens: 20 M with
-// more than two slots (2048 / 768, 4 of 16: 3 tokens = 57 M 52 / 48; 520 / 1000, 4 of 32: 4
-// tokens = 25 M 29 / 28), else 60 M (1024 / 2816, 2 of 8: 4 tokens = 69 M 36 / 37).  More:
-// 12 M with more than two slots, H < D or such a router (768 / 141, 2 of 50: 37 tokens =
-// 24 M 62 / 42), else 40 M (512 / 1376, 2 of 8: 8 tokens = 34 M 21 / 24, 16 = 68 M 32 / 25).
+// which every block reads (4096 / 14336 of 8: 148 / 127).  From two tokens on the
+// router counts too, as 1000 multiply-adds a value to four tokens and 600 from
+// there: 800 / 1228, 4 of 56, 3 tokens = 35 M and 45 M 34 / 22, but 396 / 1831, 4 of 6, 4 = 35 M
+// and 3 M 15 / 15; 204 / 1383, 2 of 111, 14 = 24 M and 14 M 37 / 21, but 308 / 571, 3 of 7, 11 = 17 M
+// and 1 M 14 / 21.  To four tokens 70 M, with more than two slots 50 M (636 / 7561, 2 of 14,
+// 2 = 58 M and 9 M 25 / 31; 648 / 3391, 2 of 64, 3 = 40 M and 41 M 38 / 27); more: 24 M and 20 M
+// (864 / 338, 2 of 13, 7 = 12 M and 8 M 15 / 20; 588 / 163, 4 of 42, 16 = 18 M and 15 M 35 / 18).
 //
 // fp8: 7 M (512 / 1376, 2 of 8: 1 token = 4 M 15 / 17, 2 = 8 M 20 / 18; 148 / 271, 3 of 17: 22
 // tokens = 8 M 33 / 23; 512 / 768, 2 of 8: 3 tokens = 7 M 16 / 18).
@@ -1756,10 +1759,9 @@ static bool decode_batched(const moe_handle *h, int n) {
         if (h->D < 320) return mac >= 170 * M;
         return mac >= (n == 1 ? 40 * M : 28 * M);
     }
-    const bool wide = router >= 28 * K;
-    if (n == 1) return mac >= 40 * M && (h->H < 2 * h->D || wide);
-    if (n <= 4) return mac >= (h->kt > 2 ? 20 * M : 60 * M);
-    return mac >= (h->kt > 2 || h->H < h->D || wide ? 12 * M : 40 * M);
+    if (n == 1) return mac >= 40 * M && (h->H < 2 * h->D || router >= 28 * K);
+    if (n <= 4) return mac + 1000 * router >= (h->kt > 2 ? 50 : 70) * M;
+    return mac + 600 * router >= (h->kt > 2 ? 20 : 24) * M;
 }
 
 // Whether a chunk's out would overwrite x of a later chunk: out may share memory

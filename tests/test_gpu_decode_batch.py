@@ -63,10 +63,12 @@ def test_decode_grouped(moe, oracle, wdtype, D, H, Dout, E, k, lsh, n):
     ("f32", 2048, 3000, 2, 2, 1, False), ("f32", 2048, 3600, 2, 2, 1, True),    # one token: 40 M
     ("bf16", 1024, 8192, 2, 2, 1, False), ("bf16", 2048, 3600, 2, 2, 1, True),  # one token: 40 M, H < 2 D
     ("bf16", 1792, 3648, 16, 3, 1, True),                                       # ... or a router of 28 K
-    ("bf16", 512, 1376, 8, 3, 2, False), ("bf16", 512, 1376, 8, 3, 4, True),    # to four tokens: 20 M with 3 slots
-    ("bf16", 512, 4096, 8, 2, 4, False), ("bf16", 512, 5120, 8, 2, 4, True),    # ... 60 M with 2
-    ("bf16", 512, 1376, 8, 2, 8, False), ("bf16", 512, 1376, 8, 2, 16, True),   # more: 40 M
-    ("bf16", 512, 384, 16, 4, 5, False), ("bf16", 512, 384, 16, 4, 6, True),    # ... 12 M with 4 slots
+    # two tokens and more: with the router, 1000 a value to four tokens, then 600
+    ("bf16", 512, 2560, 8, 3, 3, False), ("bf16", 512, 2720, 8, 3, 4, True),    # to four tokens: 50 M with 3 slots
+    ("bf16", 512, 4096, 8, 2, 4, False), ("bf16", 512, 5504, 8, 2, 4, True),    # ... 70 M with 2
+    ("bf16", 512, 1376, 8, 2, 5, False), ("bf16", 512, 1376, 8, 2, 6, True),    # more: 24 M
+    ("bf16", 256, 600, 8, 2, 16, False), ("bf16", 256, 600, 64, 2, 16, True),   # ... the router's part
+    ("bf16", 512, 384, 16, 4, 6, False), ("bf16", 512, 384, 16, 4, 7, True),    # ... 20 M with 4 slots
     ("fp8", 512, 1376, 8, 2, 1, False), ("fp8", 512, 1376, 8, 2, 2, True),      # 7 M
 ])
 def test_decode_path(moe, oracle, wdtype, D, H, E, k, n, grouped):
